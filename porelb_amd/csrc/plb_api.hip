@@ -157,8 +157,9 @@ int plb::ctx_alloc_state(plb_ctx* c)
         PLB_HIP(hipMalloc(&c->f[1], nf));
     PLB_HIP(hipMalloc(&c->macros, sizeof(double) * 4 * c->Npad));
     PLB_HIP(hipMemsetAsync(c->macros, 0, sizeof(double) * 4 * c->Npad, c->stream));
-    PLB_HIP(hipMalloc(&c->fault, sizeof(unsigned long long)));
-    PLB_HIP(hipMemsetAsync(c->fault, 0xff, sizeof(unsigned long long), c->stream));
+    PLB_HIP(hipMalloc(&c->fault, 2 * sizeof(unsigned long long)));
+    PLB_HIP(hipMemsetAsync(c->fault, 0xff, 2 * sizeof(unsigned long long), c->stream));
+    PLB_HIP(hipHostMalloc((void**)&c->host_words, 2 * sizeof(unsigned long long), hipHostMallocDefault));
     int dev_cus = 256;
     (void)hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, c->device);
     c->red_blocks = std::max(1, std::min<int>(dev_cus * 4, (int)((c->N + 255) / 256)));
@@ -184,6 +185,8 @@ extern "C" void plb_destroy(plb_ctx* c)
                     c->inv_perm, c->key_perm, c->kseg, c->node_xyz, c->macros, c->fault, c->red, c->reserve};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    if (c->host_words) (void)hipHostFree(c->host_words);
+    onchip_destroy(c);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     for (hipGraphExec_t& g : c->gexec)
@@ -265,6 +268,17 @@ __global__ void k_fill_macros(double* m, int64_t Npad, double rho0)
     m[3 * Npad + i] = 0.0;
 }
 
+// A state written in from outside starts with a clear density guard: the
+// fault words are reset and nothing is pending.
+static int clear_fault(plb_ctx* c)
+{
+    PLB_HIP(hipMemsetAsync(c->fault, 0xff, 2 * sizeof(unsigned long long), c->stream));
+    PLB_HIP(hipStreamSynchronize(c->stream));
+    c->segs.clear();
+    c->fault_seen = false;
+    return PLB_OK;
+}
+
 extern "C" int plb_init_equilibrium(plb_ctx* c)
 {
     if (!c) return PLB_ERR_INVALID;
@@ -277,31 +291,63 @@ extern "C" int plb_init_equilibrium(plb_ctx* c)
     hipLaunchKernelGGL(k_fill_macros, dim3((unsigned)((c->Npad + 255) / 256)), dim3(256), 0,
                        c->stream, c->macros, c->Npad, c->cfg.rho0);
     PLB_HIP(hipGetLastError());
-    PLB_HIP(hipMemsetAsync(c->fault, 0xff, sizeof(unsigned long long), c->stream));
+    return clear_fault(c);
+}
+
+// The fault words, once everything queued has run.
+static int read_fault_words(plb_ctx* c, unsigned long long* key, unsigned long long* gave_up)
+{
+    PLB_HIP(hipMemcpyAsync(c->host_words, c->fault, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream));
     PLB_HIP(hipStreamSynchronize(c->stream));
-    c->pending_n = 0;
+    *key = c->host_words[0];
+    *gave_up = c->host_words[1];
     return PLB_OK;
 }
 
-static unsigned long long read_fault_key(plb_ctx* c, int* rc)
+// Waits for the calls since the last plb_sync.  An on-chip run in which the
+// density guard tripped, or which gave up waiting for a block, has left the
+// state before it (and the macros) untouched, and everything queued behind it
+// has left the state alone: it and the calls after it are repeated with one
+// launch per step, which freeze at the end of the faulting step.
+static int settle(plb_ctx* c, unsigned long long* key)
 {
-    unsigned long long key = NO_FAULT;
-    hipError_t e = hipMemcpyAsync(&key, c->fault, sizeof key, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) {
-        plb_set_hip_error(e, "read fault", __FILE__, __LINE__);
-        *rc = PLB_ERR_HIP;
+    unsigned long long gave_up = NO_FAULT;
+    int rc = read_fault_words(c, key, &gave_up);
+    if (rc || *key == NO_FAULT) return rc;
+    size_t k = 0;
+    const int64_t fs = (int64_t)(*key >> 32);
+    for (; k < c->segs.size(); k++) {
+        const Segment& s = c->segs[k];
+        if (s.serial && (s.serial == gave_up || (*key != HOLD_FAULT && fs >= s.it0 && fs < s.it0 + s.n))) break;
     }
-    return key;
+    if (k == c->segs.size()) return PLB_OK;
+    if (gave_up != NO_FAULT) {
+        fprintf(stderr, "libplb: an on-chip run's blocks were not all resident; this lattice goes on with one launch per step\n");
+        c->chip_state = -1;
+    }
+    PLB_HIP(hipMemsetAsync(c->fault, 0xff, 2 * sizeof(unsigned long long), c->stream));
+    c->cur = c->segs[k].cur;
+    onchip_restore_macros(c, c->segs[k].macros);
+    for (; k < c->segs.size(); k++) {
+        Segment& s = c->segs[k];
+        s.serial = 0;
+        s.cur = c->cur;
+        for (int64_t t = 0; t < s.n; t++) {
+            rc = launch_step(c, s.it0 + t, t == s.n - 1);
+            if (rc) return rc;
+        }
+    }
+    return read_fault_words(c, key, &gave_up);
 }
 
-// A state written in from outside starts with a clear density guard: the
-// fault word is reset and nothing is pending.
-static int clear_fault(plb_ctx* c)
+// Before the state or the macros are read without a plb_sync.
+int plb::settle_for_read(plb_ctx* c)
 {
-    PLB_HIP(hipMemsetAsync(c->fault, 0xff, sizeof(unsigned long long), c->stream));
-    PLB_HIP(hipStreamSynchronize(c->stream));
-    c->pending_n = 0;
+    for (const Segment& s : c->segs)
+        if (s.serial) {
+            unsigned long long key;
+            return settle(c, &key);
+        }
     return PLB_OK;
 }
 
@@ -310,9 +356,20 @@ extern "C" int plb_step_async(plb_ctx* c, int64_t it0, int64_t nsteps)
     if (!c || nsteps < 0 || it0 < 0 || it0 + nsteps >= ((int64_t)1 << 31)) return PLB_ERR_INVALID;
     Range range("plb_step");
     PLB_HIP(hipSetDevice(c->device));
-    if (c->pending_n == 0) {
-        c->pending_it0 = it0;
-        c->cur_before = c->cur;
+    // A call that goes back in time behind an unsettled on-chip run would
+    // not be held off by a fault of that run.
+    if (!c->segs.empty() && it0 < c->segs.back().it0 + c->segs.back().n) {
+        int rc = settle_for_read(c);
+        if (rc) return rc;
+    }
+    Segment seg{it0, nsteps, c->cur, 0, c->macros};
+    if (onchip_ready(c, nsteps)) {
+        int rc = launch_onchip(c, it0, nsteps, &seg.serial);
+        if (rc) return rc;
+        if (seg.serial) {
+            c->segs.push_back(seg);
+            return PLB_OK;
+        }
     }
     int64_t s = 0;
     // Runs of graph_steps steps replay a captured graph; the last step of the
@@ -325,7 +382,7 @@ extern "C" int plb_step_async(plb_ctx* c, int64_t it0, int64_t nsteps)
         int rc = launch_step(c, it0 + s, s == nsteps - 1);
         if (rc) return rc;
     }
-    c->pending_n += nsteps;
+    if (nsteps > 0) c->segs.push_back(seg);
     return PLB_OK;
 }
 
@@ -333,22 +390,23 @@ extern "C" int plb_sync(plb_ctx* c)
 {
     if (!c) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
-    int rc = PLB_OK;
-    const unsigned long long key = read_fault_key(c, &rc);
+    unsigned long long key = NO_FAULT;
+    int rc = settle(c, &key);
     if (rc) return rc;
-    const int64_t it0 = c->pending_it0, n = c->pending_n;
-    c->pending_n = 0;
+    std::vector<Segment> segs;
+    segs.swap(c->segs);
     if (key == NO_FAULT) return PLB_OK;
+    c->fault_seen = true;
     const int64_t fs = (int64_t)(key >> 32);
-    if (n > 0) {
-        // Steps after the faulting one did not run: the faulting step's
-        // output buffer holds the current state.  A fault from an earlier
-        // call made every launch of this one a no-op.
-        if (fs >= it0 && fs < it0 + n)
-            c->cur = c->cur_before ^ (int)((fs - it0 + 1) & 1);
-        else if (fs < it0)
-            c->cur = c->cur_before;
-    }
+    // Steps after the faulting one did not run: the faulting step's output
+    // buffer holds the current state.  A fault from an earlier call made
+    // every launch of this one a no-op.
+    if (!segs.empty() && fs < segs[0].it0) c->cur = segs[0].cur;
+    for (const Segment& s : segs)
+        if (fs >= s.it0 && fs < s.it0 + s.n) {
+            c->cur = s.cur ^ (int)((fs - s.it0 + 1) & 1);
+            break;
+        }
     return PLB_ERR_DENSITY;
 }
 
@@ -408,6 +466,7 @@ extern "C" int plb_read_macros(plb_ctx* c, double* rho, double* ux, double* uy, 
     if (!c) return PLB_ERR_INVALID;
     Range range("plb_read_macros");
     PLB_HIP(hipSetDevice(c->device));
+    if (const int rcs = settle_for_read(c)) return rcs;
     double* outs[4] = {rho, ux, uy, uz};
     const int64_t chunk = std::min<int64_t>(std::max<int64_t>(c->N, 1), 8 * CHUNK_NODES);
     double* d = nullptr;
@@ -432,6 +491,7 @@ extern "C" int plb_read_populations(plb_ctx* c, double* f_aos)
 {
     if (!c || (!f_aos && c->N)) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
+    if (const int rcs = settle_for_read(c)) return rcs;
     const int64_t chunk = std::min<int64_t>(std::max<int64_t>(c->N, 1), CHUNK_NODES);
     double* d = nullptr;
     PLB_HIP(hipMalloc(&d, sizeof(double) * Q * chunk));
@@ -452,6 +512,7 @@ extern "C" int plb_write_populations(plb_ctx* c, const double* f_aos)
 {
     if (!c || (!f_aos && c->N)) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
+    if (const int rcs = settle_for_read(c)) return rcs;
     const int64_t chunk = std::min<int64_t>(std::max<int64_t>(c->N, 1), CHUNK_NODES);
     double* d = nullptr;
     PLB_HIP(hipMalloc(&d, sizeof(double) * Q * chunk));
@@ -487,6 +548,7 @@ static int copy_state(plb_ctx* c, void* host, bool to_device)
 {
     if (!c || (!host && c->N)) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
+    if (const int rcs = settle_for_read(c)) return rcs;
     const int64_t chunk = std::min<int64_t>(std::max<int64_t>(c->N, 1), CHUNK_NODES);
     const size_t rec = Q * c->elem;
     void* d = nullptr;
@@ -545,6 +607,7 @@ extern "C" int plb_reduce(plb_ctx* c, plb_reduction* out)
     if (!c || !out) return PLB_ERR_INVALID;
     Range range("plb_reduce");
     PLB_HIP(hipSetDevice(c->device));
+    if (const int rcs = settle_for_read(c)) return rcs;
     double r[2] = {0.0, 0.0};
     if (c->N > 0) {
         int rc = launch_reduce(c, r);
@@ -596,9 +659,10 @@ extern "C" int plb_last_fault(plb_ctx* c, plb_fault* out)
 {
     if (!c || !out) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
+    if (const int rcs = settle_for_read(c)) return rcs;
     memset(out, 0, sizeof *out);
-    int rc = PLB_OK;
-    const unsigned long long key = read_fault_key(c, &rc);
+    unsigned long long key = NO_FAULT, gave_up = NO_FAULT;
+    const int rc = read_fault_words(c, &key, &gave_up);
     if (rc) return rc;
     if (key == NO_FAULT) return PLB_OK;
     out->tripped = 1;

@@ -9,6 +9,9 @@
 
 namespace plb {
 
+struct StepArgs;
+StepArgs make_args(plb_ctx* c, int64_t it, bool write_macros);
+
 struct StepArgs {
     const void* fin;
     void* fout;
@@ -69,12 +72,13 @@ __device__ __forceinline__ void record_fault(const StepArgs& a, int64_t i, doubl
 }
 
 // A step after the first faulting step stores nothing, so the state stays
-// that of the faulting step (the reference exits there).  The fault word is
+// that of the faulting step (the reference exits there); nor does any step
+// queued behind an on-chip run that gave up (HOLD_FAULT).  The fault word is
 // loaded at kernel entry but only consulted before the stores, so it adds no
 // latency in front of the table and population loads.
 __device__ __forceinline__ bool frozen(unsigned long long fk, int64_t it)
 {
-    return fk != NO_FAULT && (int64_t)(fk >> 32) < it;
+    return fk != NO_FAULT && ((int64_t)(fk >> 32) < it || fk == HOLD_FAULT);
 }
 
 // ---------------------------------------------------------------- phases of one node

@@ -42,6 +42,9 @@ constexpr double TP[Q] = {1.0 / 3,  1.0 / 18, 1.0 / 18, 1.0 / 18, 1.0 / 18, 1.0 
 constexpr int32_t TAB_BOUNCE = -1;
 constexpr int32_t TAB_CONST = -2;
 constexpr unsigned long long NO_FAULT = ~0ull;
+// Fault word while a given-up on-chip run waits to be replayed: every later
+// launch leaves the state alone.  Above every real key (step < 2^31).
+constexpr unsigned long long HOLD_FAULT = ~0ull - 1;
 constexpr int TILE8_WORDS = 5;  // words of packed u8 offsets per node: 4 u32 + one u16
 constexpr int TILE8_FULL = 4;   // the u32 words; directions 17 and 18 live in the u16
 
@@ -101,6 +104,17 @@ __host__ __device__ __forceinline__ uint64_t pack_xyz(uint64_t x, uint64_t y, ui
 
 }  // namespace plb
 
+namespace plb {
+struct OnchipPlan;
+// One plb_step_async call that plb_sync has not settled yet.
+struct Segment {
+    int64_t it0, n;
+    int cur;             // buffer of the state before it
+    uint32_t serial;     // on-chip run: its serial number; 0: one launch per step
+    double* macros;      // macros array before it
+};
+}  // namespace plb
+
 struct plb_ctx {
     plb_config cfg;
     int device = 0;
@@ -137,15 +151,19 @@ struct plb_ctx {
     uint64_t* node_xyz = nullptr;  // internal order
     double* macros = nullptr;   // [4][Npad]
     void* reserve = nullptr;    // placement reserve (cfg.placement_reserve_gib)
-    unsigned long long* fault = nullptr;
+    unsigned long long* fault = nullptr;  // [0] density-guard key, [1] serial of an on-chip run that gave up
+    unsigned long long* host_words = nullptr;  // page-locked copy of the two words
     double* red = nullptr;      // reduction partials
     int red_blocks = 0;
     double omega = 0.0;
     float scale = 1.f, inv_scale = 1.f;  // FP16 storage scale 2^scale_log2
     int scale_log2 = 0;
-    int64_t last_it = -1;       // last step issued
-    int64_t pending_it0 = 0, pending_n = 0;
-    int cur_before = 0;
+    std::vector<plb::Segment> segs;  // calls since the last plb_sync
+    bool fault_seen = false;    // the density guard tripped and the state was not replaced
+    // On-chip runs of small lattices (plb_onchip.hip)
+    plb::OnchipPlan* chip = nullptr;
+    int chip_state = 0;         // 0: no plan yet, 1: plan ready, -1: not used for this lattice
+    int64_t chip_steps = 0;     // steps asked for in calls long enough for the on-chip run
 };
 
 // Error helpers (host).
@@ -259,5 +277,11 @@ int permute_ref_table(const int32_t* tabref, int64_t n, const uint32_t* inv_perm
                       hipStream_t s);
 int ctx_begin(plb_ctx* c, const plb_config* cfg, int nx, int ny, int nz, int num_p);
 int noalloc_setup(int device);
+// On-chip runs: `n` steps it0.. of a lattice that fits the CUs' LDS, as one launch.
+bool onchip_ready(plb_ctx* c, int64_t nsteps);
+int launch_onchip(plb_ctx* c, int64_t it0, int64_t n, uint32_t* serial);
+void onchip_destroy(plb_ctx* c);
+void onchip_restore_macros(plb_ctx* c, double* macros);
+int settle_for_read(plb_ctx* c);
 int ctx_alloc_state(plb_ctx* c);
 }  // namespace plb

@@ -73,6 +73,7 @@ extern "C" int plb_read_macros_noalloc(plb_ctx* c, int64_t first, int64_t n, dou
     if (n == 0) return PLB_OK;
     if (c->device < 0 || c->device >= MAX_DEVICES || !scratch_ptr[c->device]) return PLB_ERR_HIP;
     PLB_HIP(hipSetDevice(c->device));
+    if (const int rcs = settle_for_read(c)) return rcs;
     double* d = scratch_ptr[c->device];
     hipLaunchKernelGGL(k_gather_macros4, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, c->macros,
                        c->Npad, c->inv_perm, first, n, d);

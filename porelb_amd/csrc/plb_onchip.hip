@@ -1,0 +1,901 @@
+// plb_onchip.hip -- many time steps of a small lattice in one launch, with the
+// populations held in the CUs' LDS.
+//
+// One launch per step costs a small lattice the launch gap (2.6 us) and one
+// load -> gather -> store latency chain per step, whatever its size, and its
+// populations cross the L2s every step.  Here every CU keeps one block of
+// nodes for the whole run: a step reads and writes LDS, and only the links
+// between blocks go through memory.
+//
+// Blocks.  The pore nodes are ranked along a Morton curve (compact blocks) and
+// cut into G <= CUs blocks of equal size, at most NS node slots each.  Inside
+// a block, nodes with a link to another block come first, then the others, each
+// in V order (short runs along x, which keep the LDS gathers nearly free of
+// bank conflicts).  LDS holds the post-collision populations as F[slot][j]: the
+// row length 19 is odd, so neighbouring slots' populations of one direction lie
+// in different banks, and a node's 19 stores share one address register.
+//
+// Links.  idx holds, per node and direction, the LDS position the population
+// is pulled from: the upstream node's row; the node's own cell re[j] for a
+// bounce; a constant cell (reference bounce order); and again the node's own
+// cell re[j] for a link from another block -- that slot's value has left for the
+// other block, and no node of this block reads it, so the incoming value takes
+// its place.  An exchange entry therefore is one LDS cell, the place of its
+// value in the partner's receive buffer, and its own place in this block's.
+// Links between blocks are always exchanged both ways (in the reference bounce
+// order one way may be unused and is dropped on arrival), so no block can be
+// more than one step ahead of a neighbour and two receive buffers, used by
+// turns, are enough.
+//
+// Exchange.  A value travels with the step's number in one word that is stored
+// and loaded as one atomic (FP32: 8 bytes, FP64: two halves of 8 bytes, FP16: 4
+// bytes), and the receiver polls that word: no flag, no fence, one trip through
+// memory (0.9 us per round between 256 blocks, against 5.1 us for a grid barrier
+// with agent fences).  Blocks with more than 64 x T/64 slots send their
+// boundary nodes' values before they update the interior ones, so the trip
+// overlaps the update.
+//
+// Ends.  Blocks wait for each other, so the launch is cooperative, and every
+// wait is bounded: a block that waits too long (50 ms for the first exchange,
+// 2 s later) names the run in fault[1], holds all queued work off (HOLD_FAULT) and
+// every block leaves.  The state before the run is in the other buffer, and
+// plb_sync repeats the run with one launch per step; it does the same after a
+// density-guard trip, since blocks far from the tripping node go on.
+#include <stdio.h>
+
+#include <algorithm>
+
+#include "plb_device.hpp"
+
+namespace plb {
+
+// One lattice, or one sample of a batch: its nodes and its share of the blocks.
+struct OnchipSample {
+    int64_t off, n;        // internal ids off .. off + n
+    int64_t rank0, word0;  // first rank and first word of its Morton bitmask
+    int32_t bits[3];       // coordinate bits of x, y, z
+    int32_t block0, nblocks;
+};
+
+struct OnchipPlan {
+    int G = 0, NS = 0, T = 0, K = 0;
+    bool twice = false;
+    int64_t E = 0;
+    void* fixed = nullptr;     // arrays whose size is known before the links are counted
+    void* exchange = nullptr;  // per-entry arrays and the receive buffers
+    uint32_t *node = nullptr, *idx = nullptr, *seg = nullptr, *ent_lds = nullptr, *ent_dst = nullptr;
+    void* recv = nullptr;
+    double* macros_alt = nullptr;
+    uint32_t tag = 16;     // step number the next run starts with
+    uint32_t serial = 0;   // of the last run
+};
+
+constexpr uint32_t EMPTY = 0xffffffffu;
+// Cells behind the NS rows of F: the constants of directions 1..6 and 7..18,
+// and one that takes what is dropped on arrival.
+constexpr int EXTRA = 3, DROP = 2;
+
+// ---------------------------------------------------------------- plan
+__device__ __forceinline__ int64_t morton(uint64_t p, const OnchipSample& s)
+{
+    const uint32_t c[3] = {(uint32_t)(p & 0xffff), (uint32_t)((p >> 16) & 0xffff), (uint32_t)((p >> 32) & 0xffff)};
+    uint64_t m = 0;
+    int o = 0;
+    for (int l = 0; l < 16; l++)
+        for (int d = 0; d < 3; d++)
+            if (l < s.bits[d]) m |= (uint64_t)((c[d] >> l) & 1u) << o++;
+    return (int64_t)m;
+}
+
+struct OnchipBuild {
+    const OnchipSample* samples;
+    int nsamples;
+    int64_t Ntot;               // internal ids, pads between samples included
+    const uint64_t* xyz;
+    const uint32_t* xyz_of;     // xyz is in V order: V id of an internal id (batches); null: by internal id
+    const uint32_t* vid;        // V id of an internal id; null: identity
+    const uint32_t* node_of_v;  // its inverse
+    unsigned long long* bits;
+    uint32_t* wpre;
+    uint32_t* order;            // rank -> internal id
+    uint16_t* blk;              // internal id -> block
+    uint32_t* slot_of;          // internal id -> block * NS + slot
+    int32_t* T;                 // [18][Ntot] pull sources
+    uint32_t* M;                // [18][Ntot] node that pulls population re[j]; later the shared link's entry
+    int* err;                   // the table is not that of a lattice (records that contradict each other)
+    uint32_t* cnt;              // entries per group of 64 slots
+    uint32_t *node, *idx, *seg, *ent_lds, *ent_dst;
+    int G, NS;
+};
+
+__device__ __forceinline__ int sample_of(const OnchipBuild& b, int64_t k)
+{
+    int lo = 0, hi = b.nsamples - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (b.samples[mid].off <= k) lo = mid;
+        else hi = mid - 1;
+    }
+    return k >= b.samples[lo].off && k < b.samples[lo].off + b.samples[lo].n && b.samples[lo].nblocks > 0 ? lo : -1;
+}
+
+__device__ __forceinline__ int64_t curve_pos(const OnchipBuild& b, int s, int64_t k)
+{
+    return b.samples[s].word0 * 64 + morton(b.xyz[b.xyz_of ? (int64_t)b.xyz_of[k] : k], b.samples[s]);
+}
+
+__global__ void k_onchip_bits(const OnchipBuild b)
+{
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= b.Ntot) return;
+    const int s = sample_of(b, k);
+    if (s < 0) return;
+    const int64_t m = curve_pos(b, s, k);
+    const unsigned long long bit = 1ull << (m & 63);
+    if (atomicOr(b.bits + (m >> 6), bit) & bit) *b.err = 1;  // two records with the same coordinates
+}
+
+// Exclusive scan by one block (out[n] = total): a few thousand to a few
+// hundred thousand values, not worth several launches and their allocations.
+// POPC: the values are the bit counts of 64-bit words.
+template <bool POPC>
+__global__ void __launch_bounds__(1024) k_onchip_scan(const void* in, uint32_t* out, int64_t n)
+{
+    constexpr int PER = 8;
+    __shared__ uint32_t wsum[16];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    uint32_t carry = 0;
+    for (int64_t b = 0; b < n; b += 1024 * PER) {
+        uint32_t v[PER], sum = 0;
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int64_t i = b + (int64_t)tid * PER + k;
+            v[k] = i < n ? (POPC ? (uint32_t)__popcll(((const unsigned long long*)in)[i]) : ((const uint32_t*)in)[i]) : 0u;
+            sum += v[k];
+        }
+        uint32_t inc = sum;
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) {
+            const uint32_t t = __shfl_up(inc, m, 64);
+            if (lane >= m) inc += t;
+        }
+        if (lane == 63) wsum[w] = inc;
+        __syncthreads();
+        uint32_t before = 0, total = 0;
+        for (int q = 0; q < 16; q++) {
+            if (q < w) before += wsum[q];
+            total += wsum[q];
+        }
+        uint32_t e = carry + before + inc - sum;
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int64_t i = b + (int64_t)tid * PER + k;
+            if (i < n) out[i] = e;
+            e += v[k];
+        }
+        carry += total;
+        __syncthreads();
+    }
+    if (tid == 0) out[n] = carry;
+}
+
+__global__ void k_onchip_rank(const OnchipBuild b)
+{
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= b.Ntot) return;
+    const int si = sample_of(b, k);
+    if (si < 0) return;
+    const OnchipSample s = b.samples[si];
+    const int64_t m = curve_pos(b, si, k);
+    const int64_t r = (int64_t)b.wpre[m >> 6] + __popcll(b.bits[m >> 6] & ((1ull << (m & 63)) - 1ull));
+    b.order[r] = (uint32_t)k;
+    b.blk[k] = (uint16_t)(s.block0 + (r - s.rank0) * s.nblocks / s.n);
+}
+
+template <int LAYOUT, int IDX>
+__global__ void k_onchip_links(const StepArgs a, const OnchipBuild b)
+{
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= b.Ntot || sample_of(b, k) < 0) return;
+    int32_t t[Q];
+    lane_sources<LAYOUT, IDX>(a, k, t);
+#pragma unroll
+    for (int j = 1; j < Q; j++) {
+        b.T[(int64_t)(j - 1) * b.Ntot + k] = t[j];
+        if (t[j] >= 0 && atomicExch(b.M + (int64_t)(RE[j] - 1) * b.Ntot + t[j], (uint32_t)k) != EMPTY) *b.err = 1;
+    }
+}
+
+// Link j of node k: the node of another block it is shared with, or EMPTY.
+// The node it pulls from must be the one that pulls re[j] from it, if any:
+// the exchange and the reuse of its LDS cell rest on that.  A mask always
+// gives such links; V records are taken as they are, so it is checked.
+__device__ __forceinline__ uint32_t partner(const OnchipBuild& b, int64_t k, int j, uint16_t mine, int32_t& t)
+{
+    t = b.T[(int64_t)(j - 1) * b.Ntot + k];
+    const uint32_t m = b.M[(int64_t)(j - 1) * b.Ntot + k];
+    if (t >= 0 && m != EMPTY && (uint32_t)t != m) *b.err = 1;
+    const uint32_t with = t >= 0 ? (uint32_t)t : m;
+    return with != EMPTY && b.blk[with] != mine ? with : EMPTY;
+}
+
+// Slot order of one block's nodes: key (no shared link, V id), sorted in LDS.
+constexpr int SORT_MAX = 4096;
+__global__ void __launch_bounds__(1024) k_onchip_slots(const OnchipBuild b, const int32_t* block_sample)
+{
+    __shared__ uint32_t key[SORT_MAX];
+    const int blk = blockIdx.x;
+    const OnchipSample s = b.samples[block_sample[blk]];
+    const int64_t lb = blk - s.block0;
+    const int64_t r0 = (lb * s.n + s.nblocks - 1) / s.nblocks, r1 = ((lb + 1) * s.n + s.nblocks - 1) / s.nblocks;
+    const int n = (int)(r1 - r0);
+    int P = 64;
+    while (P < n) P <<= 1;
+    for (int q = threadIdx.x; q < P; q += blockDim.x) {
+        uint32_t v = EMPTY;
+        if (q < n) {
+            const uint32_t k = b.order[s.rank0 + r0 + q];
+            if (k != EMPTY) {  // a rank stays empty where two records share a voxel
+                bool shared = false;
+                int32_t t;
+                for (int j = 1; j < Q; j++) shared |= partner(b, k, j, (uint16_t)blk, t) != EMPTY;
+                v = (b.vid ? b.vid[k] : k) | (shared ? 0u : 0x80000000u);
+            }
+        }
+        key[q] = v;
+    }
+    __syncthreads();
+    for (int size = 2; size <= P; size <<= 1)
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+            for (int q = threadIdx.x; q < P / 2; q += blockDim.x) {
+                const int lo = 2 * q - (q & (stride - 1)), hi = lo + stride;
+                const bool up = (lo & size) == 0;
+                const uint32_t x = key[lo], y = key[hi];
+                if ((x > y) == up) {
+                    key[lo] = y;
+                    key[hi] = x;
+                }
+            }
+            __syncthreads();
+        }
+    for (int q = threadIdx.x; q < b.NS; q += blockDim.x) {
+        uint32_t k = EMPTY;
+        if (q < n && key[q] != EMPTY) {
+            const uint32_t v = key[q] & 0x7fffffffu;
+            k = b.node_of_v ? b.node_of_v[v] : v;
+            b.slot_of[k] = (uint32_t)blk * (uint32_t)b.NS + (uint32_t)q;
+        }
+        b.node[(int64_t)blk * b.NS + q] = k;
+    }
+}
+
+// Entries of each group of 64 slots, in the order (direction, slot).
+// FILL 0: counts them; 1: writes the entries and the index words.
+template <int FILL>
+__global__ void __launch_bounds__(256) k_onchip_groups(const OnchipBuild b)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int ng = b.NS / 64;
+    if (g >= (int64_t)b.G * ng) return;
+    const int blk = (int)(g / ng);
+    const uint32_t slot = (uint32_t)(g % ng) * 64 + lane;
+    const uint32_t k = b.node[g * 64 + lane];
+    uint32_t e = FILL ? b.seg[g] : 0u, lo = 0;
+#pragma unroll
+    for (int j = 1; j < Q; j++) {
+        int32_t t = TAB_CONST;
+        uint32_t with = EMPTY;
+        if (k != EMPTY) with = partner(b, k, j, (uint16_t)blk, t);
+        const uint64_t m = __builtin_amdgcn_ballot_w64(with != EMPTY);
+        if constexpr (FILL) {
+            const uint32_t own = slot * Q + RE[j];
+            const bool in_block = t >= 0 && b.blk[t] == (uint16_t)blk;
+            uint32_t pos = own;
+            if (in_block) pos = b.slot_of[t] % (uint32_t)b.NS * Q + j;
+            else if (t == TAB_CONST) pos = (uint32_t)b.NS * Q + (j > 6 ? 1u : 0u);
+            if (k == EMPTY) pos = 0;
+            // words 0..8 hold directions 1, 2 | 3, 4 | ... | 17, 18
+            if (j & 1) lo = pos;
+            else b.idx[((int64_t)blk * 9 + (j / 2 - 1)) * b.NS + slot] = lo | (pos << 16);
+            if (with != EMPTY) {
+                const uint32_t at = e + __popcll(m & ((1ull << lane) - 1ull));
+                const uint32_t to = t >= 0 && !in_block ? own : (uint32_t)b.NS * Q + DROP;
+                b.ent_lds[at] = own | (to << 16);
+                b.ent_dst[at] = with;                      // the partner node until k_onchip_dst
+                b.M[(int64_t)(j - 1) * b.Ntot + k] = at;   // read by this lane only, above
+            }
+        }
+        e += (uint32_t)__popcll(m);
+    }
+    // Whole rows of 64, so that the exchange needs no lane masks: the rest are
+    // entries a block sends to itself and drops.
+    if constexpr (FILL) {
+        if (e + lane < b.seg[g + 1]) {
+            const uint32_t drop = (uint32_t)b.NS * Q + DROP;
+            b.ent_lds[e + lane] = drop | (drop << 16);
+            b.ent_dst[e + lane] = e + lane;
+        }
+    } else {
+        if (lane == 0) b.cnt[g] = (e + 63u) & ~63u;
+    }
+}
+
+// The partner's entry is the other end of the same link: direction re[j] at
+// the partner node, and re[j] is the direction of the entry's LDS cell.
+__global__ void k_onchip_dst(const OnchipBuild b, int64_t E)
+{
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= E) return;
+    const uint32_t cell = b.ent_lds[e] & 0xffffu;
+    if (cell < (uint32_t)b.NS * Q) b.ent_dst[e] = b.M[(int64_t)(cell % Q - 1) * b.Ntot + b.ent_dst[e]];
+}
+
+// ---------------------------------------------------------------- exchange words
+// A population and the step's number in one word; FP64 takes two words, one
+// per half, in two planes of the buffer.
+template <typename S>
+struct Wire;
+template <>
+struct Wire<float> {
+    using Word = uint64_t;
+    static constexpr int WORDS = 1;
+    static __device__ __forceinline__ void pack(float v, uint32_t tag, Word w[1])
+    {
+        w[0] = ((uint64_t)tag << 32) | __float_as_uint(v);
+    }
+    static __device__ __forceinline__ bool is(Word w, uint32_t tag) { return (uint32_t)(w >> 32) == tag; }
+    static __device__ __forceinline__ Word none(uint32_t tag) { return (uint64_t)tag << 32; }
+    static __device__ __forceinline__ float unpack(const Word w[1]) { return __uint_as_float((uint32_t)w[0]); }
+};
+template <>
+struct Wire<double> {
+    using Word = uint64_t;
+    static constexpr int WORDS = 2;
+    static __device__ __forceinline__ void pack(double v, uint32_t tag, Word w[2])
+    {
+        const uint64_t b = (uint64_t)__double_as_longlong(v);
+        w[0] = ((uint64_t)tag << 32) | (b & 0xffffffffull);
+        w[1] = ((uint64_t)tag << 32) | (b >> 32);
+    }
+    static __device__ __forceinline__ bool is(Word w, uint32_t tag) { return (uint32_t)(w >> 32) == tag; }
+    static __device__ __forceinline__ Word none(uint32_t tag) { return (uint64_t)tag << 32; }
+    static __device__ __forceinline__ double unpack(const Word w[2])
+    {
+        return __longlong_as_double((long long)((w[0] & 0xffffffffull) | (w[1] << 32)));
+    }
+};
+template <>
+struct Wire<__half> {
+    using Word = uint32_t;
+    static constexpr int WORDS = 1;
+    static __device__ __forceinline__ void pack(__half v, uint32_t tag, Word w[1])
+    {
+        w[0] = (tag << 16) | __half_as_ushort(v);
+    }
+    static __device__ __forceinline__ bool is(Word w, uint32_t tag) { return (w >> 16) == (tag & 0xffffu); }
+    static __device__ __forceinline__ Word none(uint32_t tag) { return tag << 16; }
+    static __device__ __forceinline__ __half unpack(const Word w[1])
+    {
+        return __ushort_as_half((unsigned short)(w[0] & 0xffffu));
+    }
+};
+
+struct OnchipArgs {
+    const uint32_t *node, *idx, *seg, *ent_lds, *ent_dst;
+    void* recv;
+    int64_t E;
+    int NS;
+    int64_t nstride, dstride;  // element (j, node): AoSoA (node >> 6) * nstride + (node & 63) + j * dstride
+    int soa;
+    int64_t nsteps;
+    uint32_t tag, serial;
+    uint64_t first_ticks, wait_ticks;
+};
+
+// ---------------------------------------------------------------- the run
+// K nodes per thread, slots tid, tid + T, ...: the shared nodes, which come
+// first, are spread over all waves.
+// TWICE: two copies of F, read and written by turns, where they fit the LDS:
+// one block barrier per step instead of two, and no values held across it.
+template <typename S, int K, bool TWICE, int MAXT>
+__global__ void __launch_bounds__(MAXT) k_onchip(StepArgs a, const OnchipArgs p)
+{
+    using W = Wire<S>;
+    using Word = typename W::Word;
+    constexpr int RL = MAXT > 512 ? 6 : 10;   // rows of the entry list kept in registers
+    extern __shared__ __align__(16) char lds[];
+    S* F = (S*)lds;                            // the copy that is read
+    __shared__ int bad[2];                     // by step parity: a wave may be one poll ahead of another
+    // Queued behind a step that did not complete: nothing to do.  (A key of
+    // this run's own steps, set by a block that started earlier, does not count.)
+    const unsigned long long fk = *a.fault;
+    if (frozen(fk, a.it)) return;
+
+    const int T = blockDim.x, tid = threadIdx.x, lane = tid & 63, NS = p.NS;
+    const int copy = NS * Q + EXTRA;
+    S* G = TWICE ? F + copy : F;               // the copy that is written
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t blk = blockIdx.x;
+    const S* __restrict__ fin = (const S*)a.fin;
+    uint32_t node[K], w[K][9], key[K], s0[K], s1[K];
+    const bool sr = sizeof(S) == 2 && a.stochastic;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int slot = k * T + tid;
+        node[k] = p.node[blk * NS + slot];
+#pragma unroll
+        for (int q = 0; q < 9; q++) w[k][q] = p.idx[(blk * 9 + q) * NS + slot];
+        const int64_t g = blk * (NS / 64) + k * (T / 64) + wave;
+        s0[k] = p.seg[g];
+        s1[k] = p.seg[g + 1];
+        key[k] = node[k];
+        if (node[k] != EMPTY) {
+            if (sr && a.key_perm) key[k] = a.key_perm[node[k]];
+            const int64_t at = p.soa ? (int64_t)node[k] : (int64_t)(node[k] >> 6) * p.nstride + (node[k] & 63u);
+#pragma unroll
+            for (int j = 0; j < Q; j++) F[slot * Q + j] = fin[at + j * p.dstride];
+        }
+    }
+    if (tid < EXTRA) {
+        S v = S(0);
+        if constexpr (sizeof(S) == 8) v = tid == DROP ? 0.0 : (tid ? TP[7] : TP[1]) * a.rho0 * 1.0;
+        F[NS * Q + tid] = v;
+        G[NS * Q + tid] = v;
+    }
+    if (tid < 2) bad[tid] = 0;
+    // The first RL rows of the wave's first group's entries stay in registers
+    // (read from memory every step, the lists cost more than the exchange);
+    // the other groups, which mostly have none, look theirs up.
+    uint32_t cell[RL], dst[RL];
+#pragma unroll
+    for (int r = 0; r < RL; r++) {
+        const uint32_t e = s0[0] + r * 64;
+        cell[r] = dst[r] = 0;
+        if (e < s1[0]) {
+            cell[r] = p.ent_lds[e + lane];
+            dst[r] = p.ent_dst[e + lane];
+        }
+    }
+    __syncthreads();
+
+    // Cells of a group are written and read by lanes of one wave: LDS
+    // operations of a wave stay in order, the fence keeps the compiler to it.
+    auto put_word = [&](Word* buf, uint32_t to, S value, uint32_t tag) {
+        Word v[W::WORDS];
+        W::pack(value, tag, v);
+#pragma unroll
+        for (int q = 0; q < W::WORDS; q++)
+            __hip_atomic_store(buf + to + q * p.E, v[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto send = [&](int k, const S* from, uint32_t tag) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        Word* const buf = (Word*)p.recv + (int64_t)(tag & 1u) * W::WORDS * p.E;
+        if (k == 0) {
+            // All values first, then all stores: with an LDS read between two
+            // stores the compiler may put a wait for the first one, a trip
+            // through memory, in front of it (2.5 -> 5 us a step).
+            S v[RL];
+#pragma unroll
+            for (int r = 0; r < RL; r++) {
+                if (s0[0] + r * 64 >= s1[0]) break;
+                v[r] = from[cell[r] & 0xffffu];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < RL; r++) {
+                if (s0[0] + r * 64 >= s1[0]) break;
+                put_word(buf, dst[r], v[r], tag);
+            }
+        }
+        for (uint32_t e = s0[k] + (k == 0 ? RL * 64 : 0); e < s1[k]; e += 64)
+            put_word(buf, p.ent_dst[e + lane], from[p.ent_lds[e + lane] & 0xffffu], tag);
+    };
+    // Up to N rows of entries from e0: all are waited for, then stored to `to`.
+    auto receive_rows = [&](auto count, uint32_t e0, uint32_t e1, S* to, uint32_t tag, uint64_t limit, auto cell_of) {
+        constexpr int N = decltype(count)::value;
+        const int parity = (int)(tag & 1u);
+        const Word* const buf = (const Word*)p.recv + (int64_t)(tag & 1u) * W::WORDS * p.E + lane;
+        Word v[N][W::WORDS];
+        auto load = [&](int r) {
+#pragma unroll
+            for (int q = 0; q < W::WORDS; q++)
+                v[r][q] = __hip_atomic_load(buf + (e0 + r * 64) + q * p.E, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        auto missing = [&](int r) {
+            bool ok = true;
+#pragma unroll
+            for (int q = 0; q < W::WORDS; q++) ok &= W::is(v[r][q], tag);
+            return !ok;
+        };
+#pragma unroll
+        for (int r = 0; r < N; r++) {
+            if (e0 + r * 64 >= e1) break;
+            load(r);
+        }
+        uint64_t since = 0;
+        for (uint32_t spins = 1;; spins++) {
+            bool wait = false;
+#pragma unroll
+            for (int r = 0; r < N; r++) {
+                if (e0 + r * 64 >= e1) break;
+                wait |= missing(r);
+            }
+            if (__builtin_amdgcn_ballot_w64(wait) == 0) break;
+#pragma unroll
+            for (int r = 0; r < N; r++) {
+                if (e0 + r * 64 >= e1) break;
+                if (missing(r)) load(r);
+            }
+            if (spins % 256 == 0) {
+                const uint64_t now = wall_clock64();
+                if (since == 0) since = now;
+                const bool late = now - since > limit;
+                if (late) {
+                    __hip_atomic_store(a.fault + 1, (unsigned long long)p.serial, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_fetch_min(a.fault, HOLD_FAULT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                if (late || __hip_atomic_load(a.fault + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                                (unsigned long long)p.serial) {
+                    bad[parity] = 1;
+                    return;
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < N; r++) {
+            if (e0 + r * 64 >= e1) break;
+            to[cell_of(r) >> 16] = W::unpack(v[r]);
+        }
+    };
+    auto receive = [&](int k, S* to, uint32_t tag, uint64_t limit) {
+        if (k == 0 && s0[0] < s1[0])
+            receive_rows(std::integral_constant<int, RL>{}, s0[0], s1[0], to, tag, limit, [&](int r) { return cell[r]; });
+        for (uint32_t b = s0[k] + (k == 0 ? RL * 64 : 0); b < s1[k]; b += 64 * 4)
+            receive_rows(std::integral_constant<int, 4>{}, b, s1[k], to, tag, limit,
+                         [&](int r) { return p.ent_lds[b + r * 64 + lane]; });
+    };
+    auto cell_at = [&](int k, int j) -> S {
+        return j == 0 ? F[(k * T + tid) * Q] : F[(w[k][(j - 1) >> 1] >> (((j - 1) & 1) * 16)) & 0xffffu];
+    };
+    auto update = [&](int k, auto value) {
+        if (node[k] == EMPTY) return;
+        S* const own = G + (k * T + tid) * Q;
+        auto put = [&](int j, S v) { own[j] = v; };
+        if constexpr (sizeof(S) == 8) {
+            double f[Q];
+#pragma unroll
+            for (int j = 0; j < Q; j++) f[j] = value(j);
+            relax_f64(a, node[k], f, NO_FAULT, put);
+        } else {
+            float ds[Q];
+#pragma unroll
+            for (int j = 0; j < Q; j++) ds[j] = to_float(value(j));
+            relax_shift<S>(a, node[k], ds, NO_FAULT, key[k], put);
+        }
+    };
+
+#pragma unroll
+    for (int k = 0; k < K; k++) send(k, F, p.tag);
+    const int64_t it0 = a.it;
+    for (int64_t t = 0; t < p.nsteps; t++) {
+        const uint32_t tag = p.tag + (uint32_t)t;
+        const bool last = t + 1 == p.nsteps;
+        a.it = it0 + t;
+        a.write_macros = last ? 1 : 0;
+        if constexpr (MAXT > 512) {
+            // Unpacked every step: hoisted out of the loop, the addresses
+            // would spill.
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                asm volatile("" : "+v"(node[k]));
+#pragma unroll
+                for (int q = 0; q < 9; q++) asm volatile("" : "+v"(w[k][q]));
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++) receive(k, F, tag, t == 0 ? p.first_ticks : p.wait_ticks);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if constexpr (TWICE) {
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                update(k, [&](int j) { return cell_at(k, j); });
+                if (!last) send(k, G, tag + 1);
+                if constexpr (K > 1) __builtin_amdgcn_sched_barrier(0);  // one node's values at a time
+            }
+            S* const r = F;
+            F = G;
+            G = r;
+        } else {
+            S raw[K][Q];
+#pragma unroll
+            for (int k = 0; k < K; k++)
+#pragma unroll
+                for (int j = 0; j < Q; j++) raw[k][j] = cell_at(k, j);
+            __syncthreads();  // every gather is done
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                update(k, [&](int j) { return raw[k][j]; });
+                if (!last) send(k, G, tag + 1);
+                if constexpr (K > 1) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __syncthreads();  // every population is in place
+        if (bad[tag & 1u]) return;  // set before the barrier, the same for all threads
+        if constexpr (TWICE) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    S* __restrict__ fout = (S*)a.fout;
+#pragma unroll
+    for (int k = 0; k < K; k++)
+        if (node[k] != EMPTY) {
+            const int64_t at = p.soa ? (int64_t)node[k] : (int64_t)(node[k] >> 6) * p.nstride + (node[k] & 63u);
+#pragma unroll
+            for (int j = 0; j < Q; j++) fout[at + j * p.dstride] = F[(k * T + tid) * Q + j];
+        }
+}
+
+// ---------------------------------------------------------------- host
+static unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
+static int log2_ceil(int n)
+{
+    int b = 0;
+    while ((1 << b) < n) b++;
+    return b;
+}
+
+void onchip_destroy(plb_ctx* c)
+{
+    OnchipPlan* p = c->chip;
+    if (!p) return;
+    for (void* q : {p->fixed, p->exchange, (void*)p->macros_alt})
+        if (q) (void)hipFree(q);
+    delete p;
+    c->chip = nullptr;
+}
+
+void onchip_restore_macros(plb_ctx* c, double* macros)
+{
+    if (c->chip && c->chip->macros_alt == macros) std::swap(c->macros, c->chip->macros_alt);
+}
+
+// Node slots of a block, and whether two copies of its populations fit the
+// LDS.  One copy holds what the registers can carry over the barrier: 1 FP64
+// or 2 FP32 nodes per thread.
+static size_t lds_bytes(const plb_ctx* c, int NS, bool twice)
+{
+    return ((size_t)Q * NS + EXTRA) * c->elem * (twice ? 2 : 1);
+}
+static bool fits_twice(const plb_ctx* c, int NS) { return lds_bytes(c, NS, true) + 64 <= (size_t)c->lds_per_cu; }
+static bool fits(const plb_ctx* c, int NS)
+{
+    // FP16 blocks of more than 2048 slots (3 nodes per thread, one copy) spill:
+    // 22 us a step for 629 146 nodes, against 16.8 us with one launch per step.
+    const int most = c->cfg.precision == PLB_FP64 ? 1024 : 2048;
+    if (c->cfg.precision == PLB_FP16 && !fits_twice(c, NS)) return false;
+    return NS <= most && lds_bytes(c, NS, false) + 64 <= (size_t)c->lds_per_cu;
+}
+
+template <typename F>
+static void with_kernel(const plb_ctx* c, const OnchipPlan* p, F f)
+{
+    const bool small = p->T <= 512, twice = p->twice;
+    if (c->cfg.precision == PLB_FP64) twice ? f(k_onchip<double, 1, true, 512>) : f(k_onchip<double, 1, false, 1024>);
+    else if (c->cfg.precision == PLB_FP32)
+        !twice ? f(k_onchip<float, 2, false, 1024>)
+               : small ? f(k_onchip<float, 1, true, 512>) : f(k_onchip<float, 1, true, 1024>);
+    else if (p->K == 2) f(k_onchip<__half, 2, true, 1024>);
+    else small ? f(k_onchip<__half, 1, true, 512>) : f(k_onchip<__half, 1, true, 1024>);
+}
+
+static int build_onchip(plb_ctx* c, std::vector<OnchipSample>& samples, int G, int NS)
+{
+    OnchipPlan* p = new OnchipPlan();
+    c->chip = p;
+    hipStream_t s = c->stream;
+    p->G = G;
+    p->K = (NS + 1023) / 1024;
+    p->NS = (NS + 64 * p->K - 1) / (64 * p->K) * (64 * p->K);
+    p->T = p->NS / p->K;
+    NS = p->NS;
+    p->twice = fits_twice(c, NS);
+    const int ng = NS / 64;
+    const int64_t Ntot = c->N;
+    int64_t words = 0;
+    std::vector<int32_t> block_sample(G);
+    for (size_t k = 0; k < samples.size(); k++) {
+        samples[k].word0 = words;
+        const int b = samples[k].bits[0] + samples[k].bits[1] + samples[k].bits[2];
+        words += std::max<int64_t>(1, ((int64_t)1 << b) / 64);
+        for (int q = 0; q < samples[k].nblocks; q++) block_sample[samples[k].block0 + q] = (int32_t)k;
+    }
+    // arrays of the plan
+    const int64_t slots = (int64_t)G * NS, groups = (int64_t)G * ng;
+    PLB_HIP(hipMalloc(&p->fixed, sizeof(uint32_t) * (slots * 10 + groups + 1)));
+    p->node = (uint32_t*)p->fixed;
+    p->idx = p->node + slots;
+    p->seg = p->idx + 9 * slots;
+    // scratch of the build
+    DevBuf<char> scratch;
+    size_t need = 0;
+    auto part = [&](size_t bytes) {
+        const size_t at = need;
+        need += (bytes + 255) / 256 * 256;
+        return at;
+    };
+    const size_t o_smp = part(sizeof(OnchipSample) * samples.size()), o_bs = part(sizeof(int32_t) * G),
+                 o_bits = part(8 * (size_t)words), o_wpre = part(4 * (size_t)(words + 1)), o_order = part(4 * Ntot),
+                 o_blk = part(2 * Ntot), o_slot = part(4 * Ntot), o_T = part(4 * 18 * Ntot), o_M = part(4 * 18 * Ntot),
+                 o_cnt = part(4 * groups), o_err = part(4);
+    PLB_HIP(scratch.alloc((int64_t)need));
+    char* const base = scratch.p;
+    OnchipBuild b = {};
+    b.samples = (const OnchipSample*)(base + o_smp);
+    b.nsamples = (int)samples.size();
+    b.Ntot = Ntot;
+    b.xyz = c->node_xyz;
+    b.xyz_of = c->key_perm ? c->perm : nullptr;  // batches keep coordinates in V order
+    b.vid = c->perm;
+    b.node_of_v = c->inv_perm;
+    b.bits = (unsigned long long*)(base + o_bits);
+    b.wpre = (uint32_t*)(base + o_wpre);
+    b.order = (uint32_t*)(base + o_order);
+    b.blk = (uint16_t*)(base + o_blk);
+    b.slot_of = (uint32_t*)(base + o_slot);
+    b.T = (int32_t*)(base + o_T);
+    b.M = (uint32_t*)(base + o_M);
+    b.cnt = (uint32_t*)(base + o_cnt);
+    b.err = (int*)(base + o_err);
+    b.node = p->node;
+    b.idx = p->idx;
+    b.seg = p->seg;
+    b.G = G;
+    b.NS = NS;
+    PLB_HIP(hipMemcpyAsync(base + o_smp, samples.data(), sizeof(OnchipSample) * samples.size(), hipMemcpyHostToDevice, s));
+    PLB_HIP(hipMemcpyAsync(base + o_bs, block_sample.data(), sizeof(int32_t) * G, hipMemcpyHostToDevice, s));
+    PLB_HIP(hipMemsetAsync(b.bits, 0, 8 * (size_t)words, s));
+    PLB_HIP(hipMemsetAsync(b.M, 0xff, 4 * 18 * (size_t)Ntot, s));
+    PLB_HIP(hipMemsetAsync(b.order, 0xff, 4 * (size_t)Ntot, s));
+    PLB_HIP(hipMemsetAsync(b.err, 0, sizeof(int), s));
+    const dim3 per_node(nblk(Ntot, 256)), t256(256);
+    hipLaunchKernelGGL(k_onchip_bits, per_node, t256, 0, s, b);
+    hipLaunchKernelGGL(k_onchip_scan<true>, dim3(1), dim3(1024), 0, s, b.bits, b.wpre, words);
+    hipLaunchKernelGGL(k_onchip_rank, per_node, t256, 0, s, b);
+    const StepArgs a = make_args(c, 0, false);
+    const int idx = c->cfg.index_kind;
+#define PLB_LINKS(L, I) hipLaunchKernelGGL((k_onchip_links<L, I>), per_node, t256, 0, s, a, b)
+    if (c->cfg.layout == PLB_LAYOUT_SOA) {
+        if (idx == PLB_INDEX_TILE8) PLB_LINKS(PLB_LAYOUT_SOA, PLB_INDEX_TILE8);
+        else if (idx == PLB_INDEX_BITMAP) PLB_LINKS(PLB_LAYOUT_SOA, PLB_INDEX_BITMAP);
+        else PLB_LINKS(PLB_LAYOUT_SOA, PLB_INDEX_I32);
+    } else {
+        if (idx == PLB_INDEX_TILE8) PLB_LINKS(PLB_LAYOUT_AOSOA, PLB_INDEX_TILE8);
+        else if (idx == PLB_INDEX_BITMAP) PLB_LINKS(PLB_LAYOUT_AOSOA, PLB_INDEX_BITMAP);
+        else PLB_LINKS(PLB_LAYOUT_AOSOA, PLB_INDEX_I32);
+    }
+#undef PLB_LINKS
+    hipLaunchKernelGGL(k_onchip_slots, dim3(G), dim3(std::min(1024, NS)), 0, s, b, (const int32_t*)(base + o_bs));
+    hipLaunchKernelGGL(k_onchip_groups<0>, dim3(nblk(groups, 4)), t256, 0, s, b);
+    hipLaunchKernelGGL(k_onchip_scan<false>, dim3(1), dim3(1024), 0, s, b.cnt, b.seg, groups);
+    PLB_HIP(hipGetLastError());
+    uint32_t E = 0;
+    int err = 0;
+    PLB_HIP(hipMemcpyAsync(&E, b.seg + groups, sizeof E, hipMemcpyDeviceToHost, s));
+    PLB_HIP(hipMemcpyAsync(&err, b.err, sizeof err, hipMemcpyDeviceToHost, s));
+    PLB_HIP(hipStreamSynchronize(s));
+    if (err) return PLB_ERR_INVALID;
+    p->E = E;
+    if (E) {
+        const size_t word = c->cfg.precision == PLB_FP16 ? 4 : c->cfg.precision == PLB_FP32 ? 8 : 16;
+        const size_t lists = (8 * (size_t)E + 255) / 256 * 256;
+        PLB_HIP(hipMalloc(&p->exchange, lists + 2 * word * E));
+        b.ent_lds = p->ent_lds = (uint32_t*)p->exchange;
+        b.ent_dst = p->ent_dst = p->ent_lds + E;
+        p->recv = (char*)p->exchange + lists;
+        // no number a run will wait for
+        PLB_HIP(hipMemsetAsync(p->recv, 0, 2 * word * E, s));
+    }
+    hipLaunchKernelGGL(k_onchip_groups<1>, dim3(nblk(groups, 4)), t256, 0, s, b);
+    if (E) hipLaunchKernelGGL(k_onchip_dst, dim3(nblk(E, 256)), t256, 0, s, b, (int64_t)E);
+    PLB_HIP(hipGetLastError());
+    PLB_HIP(hipMalloc(&p->macros_alt, sizeof(double) * 4 * c->Npad));
+    PLB_HIP(hipMemsetAsync(p->macros_alt, 0, sizeof(double) * 4 * c->Npad, s));
+    PLB_HIP(hipStreamSynchronize(s));  // the scratch goes back
+    int rc = PLB_OK;
+    with_kernel(c, p, [&](auto* kern) {
+        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(c, NS, p->twice)) !=
+            hipSuccess)
+            rc = PLB_ERR_HIP;
+    });
+    return rc;
+}
+
+static int plan_single(plb_ctx* c)
+{
+    int cus = 0;
+    PLB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
+    const int64_t per = std::max<int64_t>(256, (c->N + cus - 1) / cus);
+    const int NS = (int)std::min<int64_t>(65536, (per + 63) / 64 * 64);
+    if (!fits(c, NS)) return PLB_ERR_RANGE;
+    OnchipSample smp = {};
+    smp.n = c->N;
+    const int d[3] = {c->nx, c->ny, c->nz};
+    for (int k = 0; k < 3; k++) smp.bits[k] = log2_ceil(d[k]);
+    if (smp.bits[0] + smp.bits[1] + smp.bits[2] > 26) return PLB_ERR_RANGE;  // a sparse mask in a huge box
+    smp.nblocks = (int)((c->N + NS - 1) / NS);
+    std::vector<OnchipSample> samples{smp};
+    return build_onchip(c, samples, smp.nblocks, NS);
+}
+
+// Whether this call of nsteps steps runs on chip; builds the plan when it pays.
+bool onchip_ready(plb_ctx* c, int64_t nsteps)
+{
+    if (c->chip_state < 0 || nsteps < 16 || c->N == 0 || c->fault_seen) return false;
+    if (c->cfg.stream_mode != PLB_STREAM_PULL || c->cfg.graph_steps != 0) return false;
+    if (c->chip_state == 0) {
+        c->chip_steps += nsteps;
+        if (c->chip_steps < 128) return false;
+        // a capture of the caller's elsewhere in this thread is none of the plan's business
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        const int rc = plan_single(c);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (rc) {  // too large, or no memory for the plan: one launch per step
+            (void)hipGetLastError();
+            onchip_destroy(c);
+        }
+        c->chip_state = rc ? -1 : 1;
+    }
+    return c->chip_state == 1;
+}
+
+int launch_onchip(plb_ctx* c, int64_t it0, int64_t n, uint32_t* serial)
+{
+    OnchipPlan* p = c->chip;
+    *serial = 0;
+    std::swap(c->macros, p->macros_alt);
+    StepArgs a = make_args(c, it0, false);
+    OnchipArgs o = {};
+    o.node = p->node;
+    o.idx = p->idx;
+    o.seg = p->seg;
+    o.ent_lds = p->ent_lds;
+    o.ent_dst = p->ent_dst;
+    o.recv = p->recv;
+    o.E = p->E;
+    o.NS = p->NS;
+    o.soa = c->cfg.layout == PLB_LAYOUT_SOA;
+    o.nstride = Q * 64;
+    o.dstride = o.soa ? c->Npad : 64;
+    o.nsteps = n;
+    o.tag = p->tag;
+    o.serial = ++p->serial ? p->serial : ++p->serial;
+    int khz = 0;
+    (void)hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device);
+    if (khz < 1000) khz = 100000;
+    o.first_ticks = (uint64_t)khz * 50;
+    o.wait_ticks = (uint64_t)khz * 2000;
+    hipError_t e = hipErrorUnknown;
+    with_kernel(c, p, [&](auto* kern) {
+        void* args[] = {(void*)&a, (void*)&o};
+        const size_t lds = lds_bytes(c, p->NS, p->twice);
+        if (p->G > 1) {
+            e = hipLaunchCooperativeKernel((const void*)kern, dim3(p->G), dim3(p->T), args, (unsigned)lds, c->stream);
+        } else {
+            hipLaunchKernelGGL(kern, dim3(1), dim3(p->T), lds, c->stream, a, o);
+            e = hipGetLastError();
+        }
+    });
+    if (e != hipSuccess) {  // refused before anything ran: one launch per step
+        (void)hipGetLastError();
+        std::swap(c->macros, p->macros_alt);
+        c->chip_state = -1;
+        return PLB_OK;
+    }
+    p->tag += (uint32_t)n + 2;  // the runs' numbers do not meet
+    *serial = o.serial;
+    c->cur ^= 1;
+    return PLB_OK;
+}
+
+}  // namespace plb

@@ -728,7 +728,7 @@ static unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); 
         else PLB_DISPATCH_ONE_IDX(PREC, LAYOUT, PLB_INDEX_TILE8, KERNEL, __VA_ARGS__);         \
     } while (0)
 
-static StepArgs make_args(plb_ctx* c, int64_t it, bool write_macros)
+StepArgs make_args(plb_ctx* c, int64_t it, bool write_macros)
 {
     StepArgs a;
     a.fin = c->f[c->cur];

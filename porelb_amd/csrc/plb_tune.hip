@@ -133,6 +133,7 @@ extern "C" int plb_autotune(const plb_config* base, const uint8_t* flag, int nx,
     auto time_cfg = [&](const plb_config& cfg, double* mlups) -> int {
         plb_ctx* c = nullptr;
         int r = plb_create_from_flag(&c, &cfg, flag, nx, ny, nz, num_p);
+        if (!r) c->chip_state = -1;  // the shapes are those of the launches per step
         if (r) return r;
         double ms = 0.0;
         r = plb_step(c, 0, std::max(2, steps / 4));
@@ -183,6 +184,7 @@ extern "C" int plb_autotune(const plb_config* base, const uint8_t* flag, int nx,
     const plb_config stage1 = *best;
     plb_ctx* c = nullptr;
     rc = plb_create_from_flag(&c, &stage1, flag, nx, ny, nz, num_p);
+    if (!rc) c->chip_state = -1;
     if (rc) return rc;
     const double n_nodes = (double)plb_num_nodes(c);
     int64_t it = 0;

@@ -1,0 +1,117 @@
+"""On-chip runs (calls of 16 steps or more of a lattice whose populations fit
+the LDS) against calls of 15 steps, which take one launch per step: stored
+state and macros bit for bit, at the edges of the block sizes, in both bounce
+modes, over odd extents, through a density-guard trip, and for V records that
+no mask gives, which must stay off the on-chip path."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CUS = 256
+SHAPE = dict(index_kind=1, layout=1, ordering=2)
+
+
+def mask_of(n, shape, seed):
+    """A random mask with exactly n pores."""
+    m = np.zeros(int(np.prod(shape)), dtype=np.uint8)
+    m[np.random.default_rng(seed).permutation(m.size)[:n]] = 1
+    return m.reshape(shape)
+
+
+def same(a, b, calls):
+    """Advances a by whole calls and b by calls of at most 15 steps."""
+    it = 0
+    for n in calls:
+        a.step(it, n)
+        for s in range(0, n, 15):
+            b.step(it + s, min(15, n - s))
+        it += n
+        assert np.array_equal(a.read_state(), b.read_state())
+        assert np.array_equal(a.read_macros(), b.read_macros())
+
+
+# (precision, nodes): one block; a full and an overfull slot count of each
+# kernel variant (2 or 1 copies in LDS, 1 or 2 nodes per thread); the largest
+# lattice that fits and the first that does not.
+EDGES = [(p, n) for p in (0, 1, 2) for n in (1, 255, 257, 256 * CUS, 256 * CUS + 1)] + [
+    (0, 512 * CUS), (0, 512 * CUS + 1), (0, 1024 * CUS), (0, 1024 * CUS + 1),
+    (1, 1024 * CUS), (1, 1024 * CUS + 1), (1, 2048 * CUS), (1, 2048 * CUS + 1),
+    (2, 1024 * CUS), (2, 1024 * CUS + 1), (2, 2048 * CUS), (2, 2048 * CUS + 1)]
+
+
+@pytest.mark.parametrize("precision,nodes", EDGES)
+def test_block_sizes(plb, precision, nodes):
+    edge = max(4, int(np.ceil((nodes / 0.6) ** (1 / 3))))
+    flag = mask_of(nodes, (edge, edge + 1, edge + 2), nodes)
+    kw = dict(tau=0.8, gx=1e-5, precision=precision, bb_mode=nodes % 2, fp16_rounding=1, brick=(edge + 2, 16, 1), **SHAPE)
+    with plb.Lattice.from_flag(flag, **kw) as a, plb.Lattice.from_flag(flag, **kw) as b:
+        same(a, b, [130, 17])
+
+
+@pytest.mark.parametrize("index,layout,order", [(0, 0, 0), (0, 1, 1), (1, 0, 2), (2, 1, 2), (2, 0, 0)])
+@pytest.mark.parametrize("dims", [(1, 1, 70), (2, 3, 64), (37, 5, 41), (31, 33, 30)])
+def test_shapes_and_extents(plb, dims, index, layout, order):
+    flag = mask_of(max(1, int(0.7 * np.prod(dims))), dims, 3)
+    brick = (dims[2], 4, 1) if order == 2 else (8, 4, 2)
+    kw = dict(tau=0.7, gx=2e-5, precision=1, bb_mode=1, index_kind=index, layout=layout, ordering=order, brick=brick)
+    with plb.Lattice.from_flag(flag, **kw) as a, plb.Lattice.from_flag(flag, **kw) as b:
+        same(a, b, [128, 16, 33])
+
+
+@pytest.mark.parametrize("ranks", [1, 3])
+def test_reference_order_against_oracle(plb, oracle_mod, ranks):
+    O = oracle_mod
+    flag = mask_of(9000, (24, 26, 28), 9)
+    V, start = O.build_V(flag, ranks)
+    f0, _ = O.init_equilibrium(len(V))
+    mac = O.pull_run(O.pull_table(V, start, O.BB_REFCOMPAT), f0, 150, 0.8, 1e-4)
+    with plb.Lattice.from_flag(flag, ranks, tau=0.8, gx=1e-4, brick=(28, 8, 1), **SHAPE) as lat:
+        lat.step(0, 150)
+        assert np.array_equal(lat.read_populations(), f0)
+        assert np.array_equal(lat.read_macros(), mac)
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2])
+def test_density_guard_trip(plb, precision):
+    """The trip falls inside an on-chip run, with another call queued behind it."""
+    flag = mask_of(15000, (30, 32, 34), 4)
+    kw = dict(tau=0.51, gx=0.03, precision=precision, bb_mode=1, brick=(34, 8, 1), **SHAPE)
+    L = plb.lib()
+    with plb.Lattice.from_flag(flag, **kw) as a, plb.Lattice.from_flag(flag, **kw) as b:
+        assert b.step_rc(0, 15) == plb.ERR_DENSITY
+        fault = b.last_fault()
+        assert 5 <= fault["step"] < 15
+        assert L.plb_step_async(a._h, 0, 400) == 0
+        assert L.plb_step_async(a._h, 400, 100) == 0
+        assert L.plb_sync(a._h) == plb.ERR_DENSITY
+        assert a.last_fault() == fault
+        assert np.array_equal(a.read_state(), b.read_state())
+        assert np.array_equal(a.read_macros(), b.read_macros())
+        assert a.step_rc(500, 200) == plb.ERR_DENSITY      # still frozen
+        assert np.array_equal(a.read_state(), b.read_state())
+        # queued, read without a plb_sync
+        a.init_equilibrium()
+        assert L.plb_step_async(a._h, 0, 200) == 0
+        assert a.last_fault() == fault
+        assert np.array_equal(a.read_macros(), b.read_macros())
+        assert L.plb_sync(a._h) == plb.ERR_DENSITY
+        assert np.array_equal(a.read_state(), b.read_state())
+
+
+@pytest.mark.parametrize("what", ["link", "coordinates"])
+def test_records_that_contradict_each_other(plb, what):
+    """plb_create takes V records as they are; a link whose other end points
+    elsewhere, or two nodes on one voxel, still step as one launch per step does."""
+    flag = mask_of(3000, (16, 18, 20), 6)
+    V, start = plb.preprocess(flag, 1)
+    V = V.copy()
+    if what == "link":
+        k = int(np.flatnonzero(V["nb"]["node_type"][:, 0] == plb.TYPE_FLUID)[5])
+        V["nb"]["node_id"][k, 0] = (int(V["nb"]["node_id"][k, 0]) + 1500) % len(V)
+    else:
+        for c in "xyz":
+            V[c][10] = V[c][2000]
+    kw = dict(tau=0.8, gx=1e-5, bb_mode=1)
+    with plb.Lattice.from_V(V, start, flag.shape, **kw) as a, plb.Lattice.from_V(V, start, flag.shape, **kw) as b:
+        same(a, b, [130, 20])
