@@ -16,6 +16,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <utility>
 #include <vector>
 
 #include "plb_internal.hpp"
@@ -33,7 +34,11 @@ struct plb_batch {
     std::vector<int> sample_cur;
     std::vector<char> active;
     int32_t* d_block_sample = nullptr;
-    int32_t* d_active = nullptr;
+    int32_t* d_active = nullptr;   // blocks of the active samples
+    int32_t* d_stepped = nullptr;  // those of them that take one launch per step
+    int32_t* d_chip = nullptr;     // on-chip blocks of the other active samples, launch by launch
+    std::vector<int> chip_launch;  // blocks of each of these launches
+    int n_active = 0, n_stepped = 0;
     int64_t* d_end = nullptr;
     int64_t* d_off = nullptr;
     int64_t* d_n = nullptr;
@@ -50,7 +55,7 @@ extern "C" void plb_batch_destroy(plb_batch* b)
         (void)hipSetDevice(b->c->device);
         (void)hipStreamSynchronize(b->c->stream);
     }
-    void* ptrs[] = {b->d_block_sample, b->d_active, b->d_end, b->d_off, b->d_n,
+    void* ptrs[] = {b->d_block_sample, b->d_active, b->d_stepped, b->d_chip, b->d_end, b->d_off, b->d_n,
                     b->d_omega, b->d_gx, b->d_sums, b->d_partial};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -209,6 +214,8 @@ extern "C" int plb_batch_create(plb_batch** out, const plb_config* cfg, const pl
         }
         hipError_t e = hipMalloc(&b->d_block_sample, sizeof(int32_t) * nblocks);
         if (e == hipSuccess) e = hipMalloc(&b->d_active, sizeof(int32_t) * nblocks);
+        if (e == hipSuccess) e = hipMalloc(&b->d_stepped, sizeof(int32_t) * nblocks);
+        if (e == hipSuccess) e = hipMalloc(&b->d_chip, sizeof(int32_t) * (b->c->Npad / ONCHIP_MIN_SLOTS + n_samples));
         if (e == hipSuccess) e = hipMalloc(&b->d_end, sizeof(int64_t) * n_samples);
         if (e == hipSuccess) e = hipMalloc(&b->d_off, sizeof(int64_t) * n_samples);
         if (e == hipSuccess) e = hipMalloc(&b->d_n, sizeof(int64_t) * n_samples);
@@ -252,50 +259,104 @@ extern "C" int64_t plb_batch_num_nodes(const plb_batch* b, int s)
     return b->n[s];
 }
 
-static int upload_active(plb_batch* b, int* n_active)
+// Whether the run's samples that fit run on chip (and builds the plan).
+static bool batch_on_chip(plb_batch* b, int64_t max_steps, int64_t check_every)
 {
-    std::vector<int32_t> list;
-    const int bs = b->c->cfg.block_size;
+    return check_every >= 16 && onchip_batch_ready(b->c, b->off, b->n, b->nx, b->ny, b->nz, max_steps);
+}
+
+// The blocks of the active samples; with `chip`, the samples that have an
+// on-chip plan are packed into launches of at most one block per CU, and only
+// the others are stepped.
+static int upload_active(plb_batch* b, bool chip)
+{
+    std::vector<int32_t> all, stepped, on_chip;
+    plb_ctx* c = b->c;
+    const int bs = c->cfg.block_size;
+    int cus = 0;
+    PLB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
+    std::vector<int> block0(b->S, 0), blocks(b->S, 0);
     for (int s = 0; s < b->S; s++) {
         if (!b->active[s]) continue;
+        if (chip) blocks[s] = onchip_blocks(c, s, &block0[s]);
         const int64_t b0 = b->off[s] / bs;
         const int64_t b1 = (b->off[s] + b->n[s] + bs - 1) / bs;
-        for (int64_t k = b0; k < b1; k++) list.push_back((int32_t)k);
+        for (int64_t k = b0; k < b1; k++) {
+            all.push_back((int32_t)k);
+            if (!blocks[s]) stepped.push_back((int32_t)k);
+        }
     }
-    *n_active = (int)list.size();
-    if (!list.empty())
-        PLB_HIP(hipMemcpyAsync(b->d_active, list.data(), sizeof(int32_t) * list.size(),
-                               hipMemcpyHostToDevice, b->c->stream));
-    PLB_HIP(hipStreamSynchronize(b->c->stream));
+    std::vector<std::vector<int>> launches;
+    onchip_pack(blocks, cus, &launches);
+    b->chip_launch.clear();
+    for (const std::vector<int>& l : launches) {
+        const size_t before = on_chip.size();
+        for (int s : l)
+            for (int k = 0; k < blocks[s]; k++) on_chip.push_back(block0[s] + k);
+        b->chip_launch.push_back((int)(on_chip.size() - before));
+    }
+    b->n_active = (int)all.size();
+    b->n_stepped = (int)stepped.size();
+    const std::pair<int32_t*, const std::vector<int32_t>*> lists[] = {
+        {b->d_active, &all}, {b->d_stepped, &stepped}, {b->d_chip, &on_chip}};
+    for (const auto& l : lists)
+        if (!l.second->empty())
+            PLB_HIP(hipMemcpyAsync(l.first, l.second->data(), sizeof(int32_t) * l.second->size(), hipMemcpyHostToDevice,
+                                   c->stream));
+    PLB_HIP(hipStreamSynchronize(c->stream));
     return PLB_OK;
 }
 
-extern "C" int plb_batch_run(plb_batch* b, int64_t max_steps, int64_t check_every, double tol,
-                             int64_t* steps_done, int64_t* updates, double* ms)
+// Steps it .. it + m - 1 of the active samples; the last one stores macros.
+static int batch_steps(plb_batch* b, int64_t it, int64_t m, bool chip)
 {
-    if (!b || max_steps < 0 || check_every < 1 || !(tol >= 0.0)) return PLB_ERR_INVALID;
-    Range range("plb_batch_run");
     plb_ctx* c = b->c;
-    PLB_HIP(hipSetDevice(c->device));
+    const bool on = chip && m >= 16;  // shorter intervals: the launch and the LDS load and store cost more than they save
+    const int32_t* list = on ? b->d_stepped : b->d_active;
+    const int n = on ? b->n_stepped : b->n_active;
+    if (on) {
+        int at = 0;
+        for (int blocks : b->chip_launch) {
+            const int rc = launch_onchip_batch(c, it, m, b->d_chip + at, blocks, b->d_omega, b->d_gx);
+            if (rc) return rc;
+            at += blocks;
+        }
+        onchip_batch_next(c, m);
+    }
+    for (int64_t k = 0; k < m; k++) {
+        const int rc = launch_step_batch(c, it + k, k == m - 1, list, n, b->d_block_sample, b->d_end, b->d_omega, b->d_gx);
+        if (rc) return rc;
+    }
+    return PLB_OK;
+}
+
+// chip: samples with an on-chip plan run on chip.  *again: a density-guard trip
+// or a launch that gave up ended the run; the launches per step, which freeze
+// at the end of the faulting step, have to repeat it from its start.
+static int batch_run(plb_batch* b, int64_t max_steps, int64_t check_every, double tol, int64_t* steps_done,
+                     int64_t* updates, double* ms, bool chip, bool* again)
+{
+    plb_ctx* c = b->c;
+    *again = false;
     int rc = plb_init_equilibrium(c);
+    if (!rc && chip) rc = onchip_batch_begin(c);
     if (rc) return rc;
     b->active.assign(b->S, 1);
     for (int s = 0; s < b->S; s++)
         if (b->n[s] == 0) b->active[s] = 0;
     std::vector<int64_t> done(b->S, 0);
     std::vector<double> prev(b->S, NAN), sums(b->S, 0.0);
-    int n_active = 0;
-    rc = upload_active(b, &n_active);
+    rc = upload_active(b, chip);
     if (rc) return rc;
     int64_t upd = 0;
     int64_t it = 0;
     PLB_HIP(hipEventRecord(c->ev0, c->stream));
-    while (n_active > 0 && it < max_steps) {
+    while (b->n_active > 0 && it < max_steps) {
         const int64_t m = std::min(check_every, max_steps - it);
-        for (int64_t k = 0; k < m; k++) {
-            rc = launch_step_batch(c, it + k, k == m - 1, b->d_active, n_active, b->d_block_sample,
-                                   b->d_end, b->d_omega, b->d_gx);
-            if (rc) return rc;
+        rc = batch_steps(b, it, m, chip);
+        if (rc) {
+            *again = chip;
+            return rc;
         }
         it += m;
         for (int s = 0; s < b->S; s++)
@@ -303,7 +364,7 @@ extern "C" int plb_batch_run(plb_batch* b, int64_t max_steps, int64_t check_ever
                 done[s] += m;
                 upd += m * b->n[s];
             }
-        rc = launch_sample_sums(c, b->d_active, n_active, b->d_block_sample, b->d_end, b->d_off, b->d_n, b->S,
+        rc = launch_sample_sums(c, b->d_active, b->n_active, b->d_block_sample, b->d_end, b->d_off, b->d_n, b->S,
                                 b->d_partial, b->d_sums);
         if (rc) return rc;
         unsigned long long key = NO_FAULT;
@@ -311,7 +372,11 @@ extern "C" int plb_batch_run(plb_batch* b, int64_t max_steps, int64_t check_ever
                                c->stream));
         PLB_HIP(hipMemcpyAsync(&key, c->fault, sizeof key, hipMemcpyDeviceToHost, c->stream));
         PLB_HIP(hipStreamSynchronize(c->stream));
-        if (key != NO_FAULT) return PLB_ERR_DENSITY;
+        if (key != NO_FAULT) {
+            *again = chip;
+            if (key == HOLD_FAULT) c->chip_state = -1;  // blocks that were not all resident: not tried again
+            return PLB_ERR_DENSITY;
+        }
         bool changed = false;
         for (int s = 0; s < b->S; s++) {
             if (!b->active[s]) continue;
@@ -327,7 +392,7 @@ extern "C" int plb_batch_run(plb_batch* b, int64_t max_steps, int64_t check_ever
             prev[s] = mean;
         }
         if (changed) {
-            rc = upload_active(b, &n_active);
+            rc = upload_active(b, chip);
             if (rc) return rc;
         }
     }
@@ -344,6 +409,20 @@ extern "C" int plb_batch_run(plb_batch* b, int64_t max_steps, int64_t check_ever
     return PLB_OK;
 }
 
+extern "C" int plb_batch_run(plb_batch* b, int64_t max_steps, int64_t check_every, double tol,
+                             int64_t* steps_done, int64_t* updates, double* ms)
+{
+    if (!b || max_steps < 0 || check_every < 1 || !(tol >= 0.0)) return PLB_ERR_INVALID;
+    Range range("plb_batch_run");
+    plb_ctx* c = b->c;
+    PLB_HIP(hipSetDevice(c->device));
+    const bool chip = batch_on_chip(b, max_steps, check_every);
+    bool again = false;
+    int rc = batch_run(b, max_steps, check_every, tol, steps_done, updates, ms, chip, &again);
+    if (again) rc = batch_run(b, max_steps, check_every, tol, steps_done, updates, ms, false, &again);
+    return rc;
+}
+
 // The whole run as one persistent launch (k_batch_persistent): the same
 // steps, check schedule, convergence rule and per-sample sums as
 // plb_batch_run, with the checks made on the device.
@@ -355,6 +434,9 @@ extern "C" int plb_batch_run_persistent(plb_batch* b, int64_t max_steps, int64_t
     Range range("plb_batch_run_persistent");
     plb_ctx* c = b->c;
     PLB_HIP(hipSetDevice(c->device));
+    // Samples on chip: the same steps, checks and stops, without a grid barrier per step.
+    if (batch_on_chip(b, max_steps, check_every))
+        return plb_batch_run(b, max_steps, check_every, tol, steps_done, updates, ms);
     int rc = plb_init_equilibrium(c);
     if (rc) return rc;
     const int S = b->S;
@@ -590,6 +672,7 @@ extern "C" int plb_batch_autotune(const plb_config* base, const plb_sample* samp
         plb_batch* b = nullptr;
         int r = plb_batch_create(&b, &cfg, samples, n_samples);
         if (r) return r;
+        b->c->chip_state = -1;  // the shapes are those of the launches per step
         int64_t upd = 0;
         double ms = 0.0;
         r = run(b, std::max(2, steps / 4), steps, 0.0, nullptr, &upd, &ms);

@@ -281,6 +281,15 @@ int noalloc_setup(int device);
 bool onchip_ready(plb_ctx* c, int64_t nsteps);
 int launch_onchip(plb_ctx* c, int64_t it0, int64_t n, uint32_t* serial);
 void onchip_destroy(plb_ctx* c);
+constexpr int ONCHIP_MIN_SLOTS = 256;  // node slots of the smallest on-chip block
+bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::vector<int64_t>& n,
+                        const std::vector<int>& nx, const std::vector<int>& ny, const std::vector<int>& nz, int64_t steps);
+int onchip_blocks(const plb_ctx* c, int sample, int* block0);
+void onchip_pack(const std::vector<int>& blocks, int cus, std::vector<std::vector<int>>* launches);
+int onchip_batch_begin(plb_ctx* c);
+int launch_onchip_batch(plb_ctx* c, int64_t it0, int64_t n, const int32_t* list, int blocks, const double* omega,
+                        const double* gx);
+void onchip_batch_next(plb_ctx* c, int64_t n);
 void onchip_restore_macros(plb_ctx* c, double* macros);
 int settle_for_read(plb_ctx* c);
 int ctx_alloc_state(plb_ctx* c);

@@ -9,9 +9,10 @@
 //
 // Blocks.  The pore nodes are ranked along a Morton curve (compact blocks) and
 // cut into G <= CUs blocks of equal size, at most NS node slots each.  Inside
-// a block, nodes with a link to another block come first, then the others, each
-// in V order (short runs along x, which keep the LDS gathers nearly free of
-// bank conflicts).  LDS holds the post-collision populations as F[slot][j]: the
+// a block, the nodes with a link to another block are dealt out evenly to the
+// waves' first groups of 64 slots, and the others fill up; both in V order
+// (short runs along x, which keep the LDS gathers nearly free of bank
+// conflicts).  LDS holds the post-collision populations as F[slot][j]: the
 // row length 19 is odd, so neighbouring slots' populations of one direction lie
 // in different banks, and a node's 19 stores share one address register.
 //
@@ -52,7 +53,8 @@ namespace plb {
 // One lattice, or one sample of a batch: its nodes and its share of the blocks.
 struct OnchipSample {
     int64_t off, n;        // internal ids off .. off + n
-    int64_t rank0, word0;  // first rank and first word of its Morton bitmask
+    int64_t rank0;         // first rank
+    int64_t word0, words;  // its Morton bitmask
     int32_t bits[3];       // coordinate bits of x, y, z
     int32_t block0, nblocks;
 };
@@ -64,7 +66,10 @@ struct OnchipPlan {
     void* fixed = nullptr;     // arrays whose size is known before the links are counted
     void* exchange = nullptr;  // per-entry arrays and the receive buffers
     uint32_t *node = nullptr, *idx = nullptr, *seg = nullptr, *ent_lds = nullptr, *ent_dst = nullptr;
+    int32_t* blk_sample = nullptr;
     void* recv = nullptr;
+    size_t recv_bytes = 0;
+    std::vector<OnchipSample> samples;
     double* macros_alt = nullptr;
     uint32_t tag = 16;     // step number the next run starts with
     uint32_t serial = 0;   // of the last run
@@ -135,22 +140,21 @@ __global__ void k_onchip_bits(const OnchipBuild b)
     if (atomicOr(b.bits + (m >> 6), bit) & bit) *b.err = 1;  // two records with the same coordinates
 }
 
-// Exclusive scan by one block (out[n] = total): a few thousand to a few
-// hundred thousand values, not worth several launches and their allocations.
-// POPC: the values are the bit counts of 64-bit words.
-template <bool POPC>
-__global__ void __launch_bounds__(1024) k_onchip_scan(const void* in, uint32_t* out, int64_t n)
+// Exclusive scan of n values by one block, from `carry` on (out[n] = the total
+// when asked): a few thousand to a few hundred thousand values, not worth
+// several launches and their allocations.
+template <typename In>
+__device__ __forceinline__ void block_scan(In in, uint32_t* out, int64_t n, uint32_t carry, bool total_too)
 {
     constexpr int PER = 8;
     __shared__ uint32_t wsum[16];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    uint32_t carry = 0;
     for (int64_t b = 0; b < n; b += 1024 * PER) {
         uint32_t v[PER], sum = 0;
 #pragma unroll
         for (int k = 0; k < PER; k++) {
             const int64_t i = b + (int64_t)tid * PER + k;
-            v[k] = i < n ? (POPC ? (uint32_t)__popcll(((const unsigned long long*)in)[i]) : ((const uint32_t*)in)[i]) : 0u;
+            v[k] = i < n ? in(i) : 0u;
             sum += v[k];
         }
         uint32_t inc = sum;
@@ -176,7 +180,20 @@ __global__ void __launch_bounds__(1024) k_onchip_scan(const void* in, uint32_t* 
         carry += total;
         __syncthreads();
     }
-    if (tid == 0) out[n] = carry;
+    if (total_too && tid == 0) out[n] = carry;
+}
+
+// Pores before each word of a sample's Morton bitmask, one block per sample.
+__global__ void __launch_bounds__(1024) k_onchip_words(const OnchipBuild b)
+{
+    const OnchipSample s = b.samples[blockIdx.x];
+    const unsigned long long* const bits = b.bits + s.word0;
+    block_scan([&](int64_t i) { return (uint32_t)__popcll(bits[i]); }, b.wpre + s.word0, s.words, (uint32_t)s.rank0, false);
+}
+
+__global__ void __launch_bounds__(1024) k_onchip_segs(const OnchipBuild b, int64_t groups)
+{
+    block_scan([&](int64_t i) { return b.cnt[i]; }, b.seg, groups, 0u, true);
 }
 
 __global__ void k_onchip_rank(const OnchipBuild b)
@@ -221,7 +238,7 @@ __device__ __forceinline__ uint32_t partner(const OnchipBuild& b, int64_t k, int
 
 // Slot order of one block's nodes: key (no shared link, V id), sorted in LDS.
 constexpr int SORT_MAX = 4096;
-__global__ void __launch_bounds__(1024) k_onchip_slots(const OnchipBuild b, const int32_t* block_sample)
+__global__ void __launch_bounds__(1024) k_onchip_slots(const OnchipBuild b, const int32_t* block_sample, int T)
 {
     __shared__ uint32_t key[SORT_MAX];
     const int blk = blockIdx.x;
@@ -258,14 +275,38 @@ __global__ void __launch_bounds__(1024) k_onchip_slots(const OnchipBuild b, cons
             }
             __syncthreads();
         }
-    for (int q = threadIdx.x; q < b.NS; q += blockDim.x) {
-        uint32_t k = EMPTY;
-        if (q < n && key[q] != EMPTY) {
-            const uint32_t v = key[q] & 0x7fffffffu;
-            k = b.node_of_v ? b.node_of_v[v] : v;
-            b.slot_of[k] = (uint32_t)blk * (uint32_t)b.NS + (uint32_t)q;
+    // S shared nodes (of n), an equal share of them in each of the nw first groups
+    __shared__ int shared_nodes;
+    if (threadIdx.x == 0) {
+        int lo = 0, hi = n;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (key[mid] & 0x80000000u) hi = mid;
+            else lo = mid + 1;
         }
-        b.node[(int64_t)blk * b.NS + q] = k;
+        shared_nodes = lo;
+    }
+    __syncthreads();
+    const int S = shared_nodes, nw = T / 64;
+    for (int q = threadIdx.x; q < n; q += blockDim.x) {
+        if (key[q] == EMPTY) continue;
+        int slot = q;
+        if (S < T) {
+            if (q < S) {
+                const int g = ((q + 1) * nw - 1) / S;
+                slot = g * 64 + q - S * g / nw;
+            } else {
+                const int i = q - S;   // the groups hold 64 - (their shared nodes) others
+                int g = 0;
+                while (g < nw && i >= 64 * (g + 1) - S * (g + 1) / nw) g++;
+                if (g < nw) slot = 64 * g + (S * (g + 1) / nw - S * g / nw) + i - (64 * g - S * g / nw);
+                else slot = T + i - (T - S);
+            }
+        }
+        const uint32_t v = key[q] & 0x7fffffffu;
+        const uint32_t k = b.node_of_v ? b.node_of_v[v] : v;
+        b.slot_of[k] = (uint32_t)blk * (uint32_t)b.NS + (uint32_t)slot;
+        b.node[(int64_t)blk * b.NS + slot] = k;
     }
 }
 
@@ -391,6 +432,9 @@ struct OnchipArgs {
     int64_t nsteps;
     uint32_t tag, serial;
     uint64_t first_ticks, wait_ticks;
+    // batches: the blocks of this launch, and each block's sample
+    const int32_t *list, *blk_sample;
+    const double *omega, *gx;
 };
 
 // ---------------------------------------------------------------- the run
@@ -416,7 +460,12 @@ __global__ void __launch_bounds__(MAXT) k_onchip(StepArgs a, const OnchipArgs p)
     const int copy = NS * Q + EXTRA;
     S* G = TWICE ? F + copy : F;               // the copy that is written
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t blk = blockIdx.x;
+    const int64_t blk = p.list ? ld_const(p.list + blockIdx.x) : (int)blockIdx.x;
+    if (p.blk_sample) {
+        const int s = ld_const(p.blk_sample + blk);
+        a.omega = ld_const(p.omega + s);
+        a.gx = ld_const(p.gx + s);
+    }
     const S* __restrict__ fin = (const S*)a.fin;
     uint32_t node[K], w[K][9], key[K], s0[K], s1[K];
     const bool sr = sizeof(S) == 2 && a.stochastic;
@@ -488,8 +537,27 @@ __global__ void __launch_bounds__(MAXT) k_onchip(StepArgs a, const OnchipArgs p)
                 put_word(buf, dst[r], v[r], tag);
             }
         }
-        for (uint32_t e = s0[k] + (k == 0 ? RL * 64 : 0); e < s1[k]; e += 64)
-            put_word(buf, p.ent_dst[e + lane], from[p.ent_lds[e + lane] & 0xffffu], tag);
+        for (uint32_t b = s0[k] + (k == 0 ? RL * 64 : 0); b < s1[k]; b += 64 * 4) {
+            uint32_t c[4], d[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (b + r * 64 >= s1[k]) break;
+                c[r] = p.ent_lds[b + r * 64 + lane];
+                d[r] = p.ent_dst[b + r * 64 + lane];
+            }
+            S v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (b + r * 64 >= s1[k]) break;
+                v[r] = from[c[r] & 0xffffu];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (b + r * 64 >= s1[k]) break;
+                put_word(buf, d[r], v[r], tag);
+            }
+        }
     };
     // Up to N rows of entries from e0: all are waited for, then stored to `to`.
     auto receive_rows = [&](auto count, uint32_t e0, uint32_t e1, S* to, uint32_t tag, uint64_t limit, auto cell_of) {
@@ -688,7 +756,7 @@ static void with_kernel(const plb_ctx* c, const OnchipPlan* p, F f)
     else small ? f(k_onchip<__half, 1, true, 512>) : f(k_onchip<__half, 1, true, 1024>);
 }
 
-static int build_onchip(plb_ctx* c, std::vector<OnchipSample>& samples, int G, int NS)
+static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, int NS)
 {
     OnchipPlan* p = new OnchipPlan();
     c->chip = p;
@@ -701,20 +769,25 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample>& samples, int G, i
     p->twice = fits_twice(c, NS);
     const int ng = NS / 64;
     const int64_t Ntot = c->N;
-    int64_t words = 0;
+    int64_t words = 0, rank = 0;
     std::vector<int32_t> block_sample(G);
     for (size_t k = 0; k < samples.size(); k++) {
-        samples[k].word0 = words;
-        const int b = samples[k].bits[0] + samples[k].bits[1] + samples[k].bits[2];
-        words += std::max<int64_t>(1, ((int64_t)1 << b) / 64);
-        for (int q = 0; q < samples[k].nblocks; q++) block_sample[samples[k].block0 + q] = (int32_t)k;
+        OnchipSample& smp = samples[k];
+        smp.word0 = words;
+        smp.rank0 = rank;
+        smp.words = smp.nblocks ? std::max<int64_t>(1, ((int64_t)1 << (smp.bits[0] + smp.bits[1] + smp.bits[2])) / 64) : 0;
+        words += smp.words;
+        if (smp.nblocks) rank += smp.n;
+        for (int q = 0; q < smp.nblocks; q++) block_sample[smp.block0 + q] = (int32_t)k;
     }
+    p->samples = samples;
     // arrays of the plan
     const int64_t slots = (int64_t)G * NS, groups = (int64_t)G * ng;
-    PLB_HIP(hipMalloc(&p->fixed, sizeof(uint32_t) * (slots * 10 + groups + 1)));
+    PLB_HIP(hipMalloc(&p->fixed, sizeof(uint32_t) * (slots * 10 + groups + 1 + G)));
     p->node = (uint32_t*)p->fixed;
     p->idx = p->node + slots;
     p->seg = p->idx + 9 * slots;
+    p->blk_sample = (int32_t*)(p->seg + groups + 1);
     // scratch of the build
     DevBuf<char> scratch;
     size_t need = 0;
@@ -723,8 +796,7 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample>& samples, int G, i
         need += (bytes + 255) / 256 * 256;
         return at;
     };
-    const size_t o_smp = part(sizeof(OnchipSample) * samples.size()), o_bs = part(sizeof(int32_t) * G),
-                 o_bits = part(8 * (size_t)words), o_wpre = part(4 * (size_t)(words + 1)), o_order = part(4 * Ntot),
+    const size_t o_smp = part(sizeof(OnchipSample) * samples.size()), o_bits = part(8 * (size_t)words), o_wpre = part(4 * (size_t)(words + 1)), o_order = part(4 * Ntot),
                  o_blk = part(2 * Ntot), o_slot = part(4 * Ntot), o_T = part(4 * 18 * Ntot), o_M = part(4 * 18 * Ntot),
                  o_cnt = part(4 * groups), o_err = part(4);
     PLB_HIP(scratch.alloc((int64_t)need));
@@ -734,7 +806,8 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample>& samples, int G, i
     b.nsamples = (int)samples.size();
     b.Ntot = Ntot;
     b.xyz = c->node_xyz;
-    b.xyz_of = c->key_perm ? c->perm : nullptr;  // batches keep coordinates in V order
+    const bool batch = c->key_perm != nullptr;
+    b.xyz_of = batch ? c->perm : nullptr;  // batches keep coordinates in V order
     b.vid = c->perm;
     b.node_of_v = c->inv_perm;
     b.bits = (unsigned long long*)(base + o_bits);
@@ -752,14 +825,15 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample>& samples, int G, i
     b.G = G;
     b.NS = NS;
     PLB_HIP(hipMemcpyAsync(base + o_smp, samples.data(), sizeof(OnchipSample) * samples.size(), hipMemcpyHostToDevice, s));
-    PLB_HIP(hipMemcpyAsync(base + o_bs, block_sample.data(), sizeof(int32_t) * G, hipMemcpyHostToDevice, s));
+    PLB_HIP(hipMemcpyAsync(p->blk_sample, block_sample.data(), sizeof(int32_t) * G, hipMemcpyHostToDevice, s));
+    PLB_HIP(hipMemsetAsync(p->node, 0xff, sizeof(uint32_t) * slots, s));
     PLB_HIP(hipMemsetAsync(b.bits, 0, 8 * (size_t)words, s));
     PLB_HIP(hipMemsetAsync(b.M, 0xff, 4 * 18 * (size_t)Ntot, s));
     PLB_HIP(hipMemsetAsync(b.order, 0xff, 4 * (size_t)Ntot, s));
     PLB_HIP(hipMemsetAsync(b.err, 0, sizeof(int), s));
     const dim3 per_node(nblk(Ntot, 256)), t256(256);
     hipLaunchKernelGGL(k_onchip_bits, per_node, t256, 0, s, b);
-    hipLaunchKernelGGL(k_onchip_scan<true>, dim3(1), dim3(1024), 0, s, b.bits, b.wpre, words);
+    hipLaunchKernelGGL(k_onchip_words, dim3((unsigned)samples.size()), dim3(1024), 0, s, b);
     hipLaunchKernelGGL(k_onchip_rank, per_node, t256, 0, s, b);
     const StepArgs a = make_args(c, 0, false);
     const int idx = c->cfg.index_kind;
@@ -774,9 +848,9 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample>& samples, int G, i
         else PLB_LINKS(PLB_LAYOUT_AOSOA, PLB_INDEX_I32);
     }
 #undef PLB_LINKS
-    hipLaunchKernelGGL(k_onchip_slots, dim3(G), dim3(std::min(1024, NS)), 0, s, b, (const int32_t*)(base + o_bs));
+    hipLaunchKernelGGL(k_onchip_slots, dim3(G), dim3(std::min(1024, NS)), 0, s, b, p->blk_sample, p->T);
     hipLaunchKernelGGL(k_onchip_groups<0>, dim3(nblk(groups, 4)), t256, 0, s, b);
-    hipLaunchKernelGGL(k_onchip_scan<false>, dim3(1), dim3(1024), 0, s, b.cnt, b.seg, groups);
+    hipLaunchKernelGGL(k_onchip_segs, dim3(1), dim3(1024), 0, s, b, groups);
     PLB_HIP(hipGetLastError());
     uint32_t E = 0;
     int err = 0;
@@ -793,13 +867,16 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample>& samples, int G, i
         b.ent_dst = p->ent_dst = p->ent_lds + E;
         p->recv = (char*)p->exchange + lists;
         // no number a run will wait for
-        PLB_HIP(hipMemsetAsync(p->recv, 0, 2 * word * E, s));
+        p->recv_bytes = 2 * word * E;
+        PLB_HIP(hipMemsetAsync(p->recv, 0, p->recv_bytes, s));
     }
     hipLaunchKernelGGL(k_onchip_groups<1>, dim3(nblk(groups, 4)), t256, 0, s, b);
     if (E) hipLaunchKernelGGL(k_onchip_dst, dim3(nblk(E, 256)), t256, 0, s, b, (int64_t)E);
     PLB_HIP(hipGetLastError());
-    PLB_HIP(hipMalloc(&p->macros_alt, sizeof(double) * 4 * c->Npad));
-    PLB_HIP(hipMemsetAsync(p->macros_alt, 0, sizeof(double) * 4 * c->Npad, s));
+    if (!batch) {
+        PLB_HIP(hipMalloc(&p->macros_alt, sizeof(double) * 4 * c->Npad));
+        PLB_HIP(hipMemsetAsync(p->macros_alt, 0, sizeof(double) * 4 * c->Npad, s));
+    }
     PLB_HIP(hipStreamSynchronize(s));  // the scratch goes back
     int rc = PLB_OK;
     with_kernel(c, p, [&](auto* kern) {
@@ -814,7 +891,7 @@ static int plan_single(plb_ctx* c)
 {
     int cus = 0;
     PLB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
-    const int64_t per = std::max<int64_t>(256, (c->N + cus - 1) / cus);
+    const int64_t per = std::max<int64_t>(ONCHIP_MIN_SLOTS, (c->N + cus - 1) / cus);
     const int NS = (int)std::min<int64_t>(65536, (per + 63) / 64 * 64);
     if (!fits(c, NS)) return PLB_ERR_RANGE;
     OnchipSample smp = {};
@@ -849,13 +926,11 @@ bool onchip_ready(plb_ctx* c, int64_t nsteps)
     return c->chip_state == 1;
 }
 
-int launch_onchip(plb_ctx* c, int64_t it0, int64_t n, uint32_t* serial)
+// One launch of `blocks` blocks (list: which) for steps it0 .. it0 + n - 1.
+static hipError_t launch(plb_ctx* c, const StepArgs& a0, OnchipArgs o, int64_t n, int blocks)
 {
     OnchipPlan* p = c->chip;
-    *serial = 0;
-    std::swap(c->macros, p->macros_alt);
-    StepArgs a = make_args(c, it0, false);
-    OnchipArgs o = {};
+    StepArgs a = a0;
     o.node = p->node;
     o.idx = p->idx;
     o.seg = p->seg;
@@ -868,8 +943,6 @@ int launch_onchip(plb_ctx* c, int64_t it0, int64_t n, uint32_t* serial)
     o.nstride = Q * 64;
     o.dstride = o.soa ? c->Npad : 64;
     o.nsteps = n;
-    o.tag = p->tag;
-    o.serial = ++p->serial ? p->serial : ++p->serial;
     int khz = 0;
     (void)hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device);
     if (khz < 1000) khz = 100000;
@@ -879,15 +952,29 @@ int launch_onchip(plb_ctx* c, int64_t it0, int64_t n, uint32_t* serial)
     with_kernel(c, p, [&](auto* kern) {
         void* args[] = {(void*)&a, (void*)&o};
         const size_t lds = lds_bytes(c, p->NS, p->twice);
-        if (p->G > 1) {
-            e = hipLaunchCooperativeKernel((const void*)kern, dim3(p->G), dim3(p->T), args, (unsigned)lds, c->stream);
+        if (blocks > 1) {
+            e = hipLaunchCooperativeKernel((const void*)kern, dim3(blocks), dim3(p->T), args, (unsigned)lds, c->stream);
         } else {
             hipLaunchKernelGGL(kern, dim3(1), dim3(p->T), lds, c->stream, a, o);
             e = hipGetLastError();
         }
     });
-    if (e != hipSuccess) {  // refused before anything ran: one launch per step
-        (void)hipGetLastError();
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
+static uint32_t next_serial(OnchipPlan* p) { return ++p->serial ? p->serial : ++p->serial; }
+
+int launch_onchip(plb_ctx* c, int64_t it0, int64_t n, uint32_t* serial)
+{
+    OnchipPlan* p = c->chip;
+    *serial = 0;
+    std::swap(c->macros, p->macros_alt);
+    OnchipArgs o = {};
+    o.tag = p->tag;
+    o.serial = next_serial(p);
+    if (launch(c, make_args(c, it0, false), o, n, p->G) != hipSuccess) {
+        // refused before anything ran: one launch per step
         std::swap(c->macros, p->macros_alt);
         c->chip_state = -1;
         return PLB_OK;
@@ -897,5 +984,134 @@ int launch_onchip(plb_ctx* c, int64_t it0, int64_t n, uint32_t* serial)
     c->cur ^= 1;
     return PLB_OK;
 }
+
+// ---------------------------------------------------------------- batches
+// Samples that fit share the launches: as many samples as have room on the
+// chip at once run to the next check, then the next ones.  First fit, largest
+// sample first: launch[k] = the samples of launch k.
+void onchip_pack(const std::vector<int>& blocks, int cus, std::vector<std::vector<int>>* launches)
+{
+    std::vector<int> order, room;
+    for (size_t k = 0; k < blocks.size(); k++)
+        if (blocks[k] > 0) order.push_back((int)k);
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return blocks[x] > blocks[y]; });
+    launches->clear();
+    for (int s : order) {
+        size_t l = 0;
+        while (l < room.size() && room[l] < blocks[s]) l++;
+        if (l == room.size()) {
+            room.push_back(cus);
+            launches->emplace_back();
+        }
+        room[l] -= blocks[s];
+        (*launches)[l].push_back(s);
+    }
+}
+
+// Time of a step of a launch with blocks of NS slots, in ns: fits of 64^3 to
+// 112^3 noise and sphere masks (FP32: 2.6 us at 512 slots, 3.3 at 1024, and
+// about 7 for two nodes per thread; FP64: 4.2 at 512, 6.1 at 1024).
+static int64_t step_ns(const plb_ctx* c, int NS)
+{
+    if (c->cfg.precision == PLB_FP64) return NS <= 512 ? 3900 + NS / 2 : 3700 + NS * 9 / 4;
+    if (c->cfg.precision == PLB_FP32) return NS <= 1024 ? 2100 + NS * 8 / 7 : 6000 + NS * 4 / 9;
+    return NS <= 1024 ? 2500 + NS : 8000;
+}
+
+bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::vector<int64_t>& n,
+                        const std::vector<int>& nx, const std::vector<int>& ny, const std::vector<int>& nz,
+                        int64_t steps)
+{
+    if (c->chip_state != 0 || steps < 128) return c->chip_state == 1 && steps >= 16;
+    c->chip_state = -1;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) return false;
+    int most = 0;
+    for (int NS = 64; NS <= 4096 && fits(c, NS); NS += 64)
+        if (NS <= 1024 || NS % 128 == 0) most = NS;
+    std::vector<OnchipSample> samples(n.size());
+    std::vector<int> blocks(n.size());
+    std::vector<std::vector<int>> launches;
+    int G = 0;
+    auto divide = [&](int NS) {
+        G = 0;
+        for (size_t k = 0; k < n.size(); k++) {
+            OnchipSample& s = samples[k];
+            s = {};
+            s.off = off[k];
+            s.n = n[k];
+            const int d[3] = {nx[k], ny[k], nz[k]};
+            for (int q = 0; q < 3; q++) s.bits[q] = log2_ceil(d[q]);
+            const bool in = n[k] > 0 && n[k] <= (int64_t)most * cus && s.bits[0] + s.bits[1] + s.bits[2] <= 26;
+            s.block0 = G;
+            s.nblocks = in ? (int)((n[k] + NS - 1) / NS) : 0;
+            if (s.nblocks > cus) return false;  // this sample needs larger blocks
+            blocks[k] = s.nblocks;
+            G += s.nblocks;
+        }
+        onchip_pack(blocks, cus, &launches);
+        return true;
+    };
+    // larger blocks: fewer launches for a step of the whole batch, each longer
+    int NS = 0;
+    int64_t cost = 0;
+    for (int q = ONCHIP_MIN_SLOTS; q <= most; q += q < 1024 ? 64 : 128) {
+        if (!divide(q)) continue;
+        const int64_t w = (int64_t)launches.size() * step_ns(c, q);
+        if (NS == 0 || w < cost) {
+            NS = q;
+            cost = w;
+        }
+    }
+    if (NS == 0 || !divide(NS)) return false;
+    if (G == 0 || G > 65535) return false;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const int rc = build_onchip(c, samples, G, NS);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (rc) {
+        (void)hipGetLastError();
+        onchip_destroy(c);
+        return false;
+    }
+    c->chip_state = 1;
+    return true;
+}
+
+int onchip_blocks(const plb_ctx* c, int sample, int* block0)
+{
+    const OnchipSample& s = c->chip->samples[sample];
+    *block0 = s.block0;
+    return s.nblocks;
+}
+
+// A new run of the batch: no number of an earlier one is left in the buffers.
+int onchip_batch_begin(plb_ctx* c)
+{
+    if (c->chip->recv_bytes) PLB_HIP(hipMemsetAsync(c->chip->recv, 0, c->chip->recv_bytes, c->stream));
+    c->chip->tag = 16;
+    return PLB_OK;
+}
+
+// The samples of `list`, n steps from buffer c->cur to the buffer that n
+// single steps end in.  Launches of one interval use the same step numbers.
+int launch_onchip_batch(plb_ctx* c, int64_t it0, int64_t n, const int32_t* list, int blocks, const double* omega,
+                        const double* gx)
+{
+    StepArgs a = make_args(c, it0, false);
+    a.fout = c->f[c->cur ^ (int)(n & 1)];  // a block reads and writes its own nodes only
+    OnchipArgs o = {};
+    o.tag = c->chip->tag;
+    o.serial = next_serial(c->chip);
+    o.list = list;
+    o.blk_sample = c->chip->blk_sample;
+    o.omega = omega;
+    o.gx = gx;
+    if (launch(c, a, o, n, blocks) == hipSuccess) return PLB_OK;
+    c->chip_state = -1;  // refused before anything ran
+    return PLB_ERR_HIP;
+}
+
+void onchip_batch_next(plb_ctx* c, int64_t n) { c->chip->tag += (uint32_t)n + 2; }
 
 }  // namespace plb

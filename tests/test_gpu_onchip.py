@@ -115,3 +115,53 @@ def test_records_that_contradict_each_other(plb, what):
     kw = dict(tau=0.8, gx=1e-5, bb_mode=1)
     with plb.Lattice.from_V(V, start, flag.shape, **kw) as a, plb.Lattice.from_V(V, start, flag.shape, **kw) as b:
         same(a, b, [130, 20])
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2])
+@pytest.mark.parametrize("persistent", [False, True])
+def test_batch_on_chip(plb, precision, persistent):
+    """Samples on chip (checks 16 steps or more apart) against launches per step
+    (checks 15 apart): macros bit for bit; one sample has no pores, one does not
+    fit the chip in FP64, and the samples take more than one launch."""
+    rng = np.random.default_rng(12)
+    flags = [mask_of(int(0.55 * np.prod(d)), d, k) for k, d in
+             enumerate([(20, 21, 22), (64, 62, 60), (9, 70, 8), (80, 78, 81), (30, 30, 30)])]
+    flags.insert(2, np.zeros((5, 5, 5), np.uint8))
+    taus = [0.6 + 0.1 * k for k in range(6)]
+    gxs = [10.0 ** -(5 + 0.2 * k) for k in range(6)]
+    kw = dict(precision=precision, bb_mode=1, fp16_rounding=1, block_size=128, brick=(1, 16, 1), **SHAPE)
+    a, b = plb.Batch(flags, taus, gxs, **kw), plb.Batch(flags, taus, gxs, **kw)
+    for every, steps in ((50, 150), (33, 145)):
+        ra = a.run(steps, every, 0.0, persistent=persistent)
+        rb = b.run(steps, 15, 0.0)
+        assert np.array_equal(ra[0], rb[0]) and ra[1] == rb[1]
+        assert all(np.array_equal(a.read_macros(s), b.read_macros(s)) for s in range(6))
+        assert a.reduce() == b.reduce()
+    a.close()
+    b.close()
+
+
+def test_batch_stops_and_trips(plb):
+    """Samples that stop at their own steps, as single lattices do; and a
+    density-guard trip, which ends as it does with one launch per step."""
+    flags = [mask_of(4000 + 900 * k, (20, 22, 24), 20 + k) for k in range(4)]
+    kw = dict(precision=0, bb_mode=1, block_size=128, brick=(24, 8, 1), **SHAPE)
+    taus, gxs = [0.7, 0.8, 1.0, 1.2], [1e-5, 2e-5, 1e-6, 3e-6]
+    b = plb.Batch(flags, taus, gxs, **kw)
+    steps, _, _ = b.run(2000, 20, 1e-3)
+    assert 0 < steps.min() < steps.max() < 2000
+    for s in range(4):
+        with plb.Lattice.from_flag(flags[s], tau=taus[s], gx=gxs[s], **kw) as lat:
+            n, r = lat.run_to_convergence(0, 2000, 20, 1e-3)
+            assert n == steps[s] and np.array_equal(lat.read_macros(), b.read_macros(s))
+    b.close()
+    gxs[2] = 0.05
+    taus[2] = 0.51
+    a, b = plb.Batch(flags, taus, gxs, **kw), plb.Batch(flags, taus, gxs, **kw)
+    for x, every in ((a, 50), (b, 10)):
+        with pytest.raises(plb.PlbError) as e:
+            x.run(200, every, 0.0)
+        assert e.value.code == plb.ERR_DENSITY
+    assert a.last_fault() == b.last_fault() and a.last_fault()[0] == 2
+    a.close()
+    b.close()
