@@ -13,7 +13,7 @@
 
 #include <algorithm>
 
-#include "plb_internal.hpp"
+#include "plb_xfer.hpp"
 
 using namespace plb;
 
@@ -119,6 +119,8 @@ int plb::fp16_scale_log2_for(double gx)
 
 int plb::ctx_begin(plb_ctx* c, const plb_config* cfg, int nx, int ny, int nz, int num_p)
 {
+    xfer_context(1);
+    c->counted = true;
     c->cfg = *cfg;
     c->nx = nx;
     c->ny = ny;
@@ -193,6 +195,7 @@ extern "C" void plb_destroy(plb_ctx* c)
         if (g) (void)hipGraphExecDestroy(g);
     if (c->it_dev) (void)hipFree(c->it_dev);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    if (c->counted) xfer_context(-1);
     delete c;
 }
 
@@ -458,33 +461,29 @@ extern "C" double plb_bytes_per_update(const plb_ctx* c)
     return 2.0 * Q * (double)c->elem + idx + (key ? c->key_bytes : 0.0);
 }
 
-static const int64_t CHUNK_NODES = 1 << 20;
-
-
 extern "C" int plb_read_macros(plb_ctx* c, double* rho, double* ux, double* uy, double* uz)
 {
     if (!c) return PLB_ERR_INVALID;
     Range range("plb_read_macros");
     PLB_HIP(hipSetDevice(c->device));
     if (const int rcs = settle_for_read(c)) return rcs;
-    double* outs[4] = {rho, ux, uy, uz};
-    const int64_t chunk = std::min<int64_t>(std::max<int64_t>(c->N, 1), 8 * CHUNK_NODES);
-    double* d = nullptr;
-    PLB_HIP(hipMalloc(&d, sizeof(double) * chunk));
-    int rc = PLB_OK;
-    for (int comp = 0; comp < 4 && !rc; comp++) {
-        if (!outs[comp]) continue;
-        for (int64_t b = 0; b < c->N && !rc; b += chunk) {
-            const int64_t n = std::min(chunk, c->N - b);
-            rc = launch_read_macros(c, comp, b, n, d);
-            if (!rc && hipMemcpyAsync(outs[comp] + b, d, sizeof(double) * n, hipMemcpyDeviceToHost,
-                                      c->stream) != hipSuccess)
-                rc = PLB_ERR_HIP;
-            if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = PLB_ERR_HIP;
+    return read_macros_range(c, 0, c->N, rho, ux, uy, uz);
+}
+
+// The macros that are asked for, of V-order nodes first .. first + n - 1.
+int plb::read_macros_range(plb_ctx* c, int64_t first, int64_t n, double* rho, double* ux, double* uy, double* uz)
+{
+    double* const outs[4] = {rho, ux, uy, uz};
+    std::vector<char*> arrays;
+    MacroList list;
+    for (int k = 0; k < 4; k++)
+        if (outs[k]) {
+            list.comp[list.n++] = k;
+            arrays.push_back((char*)outs[k]);
         }
-    }
-    (void)hipFree(d);
-    return rc;
+    return download(c->device, c->stream, n, sizeof(double), arrays, [&](int64_t b, int64_t m, void* d) {
+        return launch_read_macros(c, list, first + b, m, (double*)d);
+    });
 }
 
 extern "C" int plb_read_populations(plb_ctx* c, double* f_aos)
@@ -492,20 +491,8 @@ extern "C" int plb_read_populations(plb_ctx* c, double* f_aos)
     if (!c || (!f_aos && c->N)) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
     if (const int rcs = settle_for_read(c)) return rcs;
-    const int64_t chunk = std::min<int64_t>(std::max<int64_t>(c->N, 1), CHUNK_NODES);
-    double* d = nullptr;
-    PLB_HIP(hipMalloc(&d, sizeof(double) * Q * chunk));
-    int rc = PLB_OK;
-    for (int64_t b = 0; b < c->N && !rc; b += chunk) {
-        const int64_t n = std::min(chunk, c->N - b);
-        rc = launch_read_pop(c, b, n, d);
-        if (!rc && hipMemcpyAsync(f_aos + b * Q, d, sizeof(double) * Q * n, hipMemcpyDeviceToHost,
-                                  c->stream) != hipSuccess)
-            rc = PLB_ERR_HIP;
-        if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = PLB_ERR_HIP;
-    }
-    (void)hipFree(d);
-    return rc;
+    return download(c->device, c->stream, c->N, sizeof(double) * Q, {(char*)f_aos},
+                    [&](int64_t b, int64_t m, void* d) { return launch_read_pop(c, b, m, (double*)d); });
 }
 
 extern "C" int plb_write_populations(plb_ctx* c, const double* f_aos)
@@ -513,21 +500,9 @@ extern "C" int plb_write_populations(plb_ctx* c, const double* f_aos)
     if (!c || (!f_aos && c->N)) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
     if (const int rcs = settle_for_read(c)) return rcs;
-    const int64_t chunk = std::min<int64_t>(std::max<int64_t>(c->N, 1), CHUNK_NODES);
-    double* d = nullptr;
-    PLB_HIP(hipMalloc(&d, sizeof(double) * Q * chunk));
-    int rc = PLB_OK;
-    for (int64_t b = 0; b < c->N && !rc; b += chunk) {
-        const int64_t n = std::min(chunk, c->N - b);
-        if (hipMemcpyAsync(d, f_aos + b * Q, sizeof(double) * Q * n, hipMemcpyHostToDevice,
-                           c->stream) != hipSuccess)
-            rc = PLB_ERR_HIP;
-        if (!rc) rc = launch_write_pop(c, b, n, d);
-        if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = PLB_ERR_HIP;
-    }
-    (void)hipFree(d);
-    if (!rc) rc = clear_fault(c);
-    return rc;
+    const int rc = upload(c->device, c->stream, c->N, sizeof(double) * Q, f_aos,
+                          [&](int64_t b, int64_t m, void* d) { return launch_write_pop(c, b, m, (const double*)d); });
+    return rc ? rc : clear_fault(c);
 }
 
 extern "C" int plb_get_state_info(const plb_ctx* c, plb_state_info* out)
@@ -542,64 +517,34 @@ extern "C" int plb_get_state_info(const plb_ctx* c, plb_state_info* out)
     return PLB_OK;
 }
 
-// Stored elements between host AoS [n][19] and the device layout, through a
-// device staging chunk.
-static int copy_state(plb_ctx* c, void* host, bool to_device)
+// Stored elements between host AoS [n][19] and the device layout.
+extern "C" int plb_read_state(plb_ctx* c, void* buf)
 {
-    if (!c || (!host && c->N)) return PLB_ERR_INVALID;
+    if (!c || (!buf && c->N)) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
     if (const int rcs = settle_for_read(c)) return rcs;
-    const int64_t chunk = std::min<int64_t>(std::max<int64_t>(c->N, 1), CHUNK_NODES);
-    const size_t rec = Q * c->elem;
-    void* d = nullptr;
-    PLB_HIP(hipMalloc(&d, rec * chunk));
-    int rc = PLB_OK;
-    char* h = (char*)host;
-    for (int64_t b = 0; b < c->N && !rc; b += chunk) {
-        const int64_t n = std::min(chunk, c->N - b);
-        if (to_device) {
-            if (hipMemcpyAsync(d, h + b * rec, rec * n, hipMemcpyHostToDevice, c->stream) != hipSuccess)
-                rc = PLB_ERR_HIP;
-            if (!rc) rc = launch_copy_state(c, b, n, d, true);
-        } else {
-            rc = launch_copy_state(c, b, n, d, false);
-            if (!rc && hipMemcpyAsync(h + b * rec, d, rec * n, hipMemcpyDeviceToHost, c->stream) != hipSuccess)
-                rc = PLB_ERR_HIP;
-        }
-        if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = PLB_ERR_HIP;
-    }
-    (void)hipFree(d);
-    return rc;
+    return download(c->device, c->stream, c->N, Q * c->elem, {(char*)buf},
+                    [&](int64_t b, int64_t m, void* d) { return launch_copy_state(c, b, m, d, false); });
 }
-
-extern "C" int plb_read_state(plb_ctx* c, void* buf) { return copy_state(c, buf, false); }
 
 extern "C" int plb_write_state(plb_ctx* c, const void* buf)
 {
-    int rc = copy_state(c, const_cast<void*>(buf), true);
-    if (!rc) rc = clear_fault(c);
-    return rc;
+    if (!c || (!buf && c->N)) return PLB_ERR_INVALID;
+    PLB_HIP(hipSetDevice(c->device));
+    if (const int rcs = settle_for_read(c)) return rcs;
+    const int rc = upload(c->device, c->stream, c->N, Q * c->elem, buf,
+                          [&](int64_t b, int64_t m, void* d) { return launch_copy_state(c, b, m, d, true); });
+    return rc ? rc : clear_fault(c);
 }
 
 extern "C" int plb_read_table(plb_ctx* c, int32_t* tab)
 {
     if (!c || (!tab && c->N)) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
-    const int64_t chunk = std::min<int64_t>(std::max<int64_t>(c->N, 1), CHUNK_NODES);
-    int32_t* d = nullptr;
-    PLB_HIP(hipMalloc(&d, sizeof(int32_t) * (Q - 1) * chunk));
-    int rc = PLB_OK;
-    for (int64_t b = 0; b < c->N && !rc; b += chunk) {
-        const int64_t n = std::min(chunk, c->N - b);
-        rc = launch_read_table(c, b, n, d);
-        for (int j = 0; j < Q - 1 && !rc; j++)
-            if (hipMemcpyAsync(tab + (int64_t)j * c->N + b, d + (int64_t)j * n,
-                               sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream) != hipSuccess)
-                rc = PLB_ERR_HIP;
-        if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = PLB_ERR_HIP;
-    }
-    (void)hipFree(d);
-    return rc;
+    std::vector<char*> rows;
+    for (int j = 0; j < Q - 1; j++) rows.push_back((char*)(tab + (int64_t)j * c->N));
+    return download(c->device, c->stream, c->N, sizeof(int32_t), rows,
+                    [&](int64_t b, int64_t m, void* d) { return launch_read_table(c, b, m, (int32_t*)d); });
 }
 
 extern "C" int plb_reduce(plb_ctx* c, plb_reduction* out)

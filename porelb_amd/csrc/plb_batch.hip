@@ -587,26 +587,7 @@ extern "C" int plb_batch_read_macros(plb_batch* b, int sample, double* rho, doub
     if (!b || sample < 0 || sample >= b->S) return PLB_ERR_INVALID;
     plb_ctx* c = b->c;
     PLB_HIP(hipSetDevice(c->device));
-    const int64_t n = b->n[sample], off = b->off[sample];
-    if (n == 0) return PLB_OK;
-    double* outs[4] = {rho, ux, uy, uz};
-    const int64_t chunk = std::min<int64_t>(n, (int64_t)8 << 20);
-    double* d = nullptr;
-    PLB_HIP(hipMalloc(&d, sizeof(double) * chunk));
-    int rc = PLB_OK;
-    for (int comp = 0; comp < 4 && !rc; comp++) {
-        if (!outs[comp]) continue;
-        for (int64_t k = 0; k < n && !rc; k += chunk) {
-            const int64_t m = std::min(chunk, n - k);
-            rc = launch_read_macros(c, comp, off + k, m, d);
-            if (!rc && hipMemcpyAsync(outs[comp] + k, d, sizeof(double) * m, hipMemcpyDeviceToHost,
-                                      c->stream) != hipSuccess)
-                rc = PLB_ERR_HIP;
-            if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = PLB_ERR_HIP;
-        }
-    }
-    (void)hipFree(d);
-    return rc;
+    return read_macros_range(c, b->off[sample], b->n[sample], rho, ux, uy, uz);
 }
 
 extern "C" int plb_batch_reduce(plb_batch* b, plb_reduction* out)

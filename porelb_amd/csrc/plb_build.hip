@@ -28,7 +28,7 @@
 
 #include <algorithm>
 
-#include "plb_internal.hpp"
+#include "plb_xfer.hpp"
 
 namespace plb {
 
@@ -109,7 +109,8 @@ __device__ __forceinline__ int64_t pore_id(const uint64_t* bits, const uint64_t*
     return (int64_t)wpre[w] + __popcll(bits[w] & below);
 }
 
-// flag (u8, x fastest) -> bits + per-word counts.  blockDim multiple of 64.
+// flag (u8, x fastest) -> bits + per-word counts.  blockDim multiple of 64;
+// a chunk of the mask starts on a word.
 __global__ void k_flag_bits(const uint8_t* __restrict__ flag, int64_t nvox, int64_t nwords,
                             uint64_t* __restrict__ bits, uint64_t* __restrict__ wcount, int* err)
 {
@@ -228,7 +229,8 @@ __global__ void k_slab_starts(GridArgs a, int num_p, int32_t* start)
 
 // ---------------------------------------------------------------- from V records
 struct VArgs {
-    const uint64_t* V;  // records as 19 words
+    const uint64_t* V;  // records of nodes first .. last - 1 as 19 words
+    int64_t first, last;
     int64_t N;
     const int32_t* start;
     int num_p;
@@ -254,9 +256,9 @@ __device__ __forceinline__ int owner_rank(const int32_t* start, int num_p, int64
 
 __global__ void k_table_from_V(VArgs a)
 {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= a.N) return;
-    const uint64_t* rec = a.V + g * 19;
+    const int64_t g = a.first + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= a.last) return;
+    const uint64_t* rec = a.V + (g - a.first) * 19;
     const uint64_t w0 = rec[0];
     const int x = (int)(w0 & 0xffff), y = (int)((w0 >> 16) & 0xffff), z = (int)((w0 >> 32) & 0xffff);
     // check_V (porelb.c:115-141), applied to every rank's records.
@@ -764,36 +766,34 @@ int build_table_from_V(plb_ctx* c, const plb_node_info* V, int64_t n)
     DevBuf<int32_t> dstart, tabref;
     DevBuf<int> derr;
     int herr = 0;
-    {
-        DevBuf<uint64_t> dV;  // 152-byte records as 19 words; freed before the final table exists
-        PLB_HIP(dV.alloc(n * 19));
-        PLB_HIP(dstart.alloc(c->num_p));
-        PLB_HIP(tabref.alloc((Q - 1) * n));
-        PLB_HIP(xyz.alloc(n));
-        PLB_HIP(derr.alloc(1));
-        PLB_HIP(hipMemsetAsync(derr, 0, sizeof(int), s));
-        if (n) PLB_HIP(hipMemcpyAsync(dV, V, sizeof(plb_node_info) * n, hipMemcpyHostToDevice, s));
-        PLB_HIP(hipMemcpyAsync(dstart, c->V_sub_start.data(), sizeof(int32_t) * c->num_p,
-                               hipMemcpyHostToDevice, s));
-        if (n) {
-            VArgs a;
-            a.V = dV;
-            a.N = n;
-            a.start = dstart;
-            a.num_p = c->num_p;
-            a.nx = c->nx;
-            a.ny = c->ny;
-            a.nz = c->nz;
-            a.mode = c->cfg.bb_mode;
-            a.tab = tabref;
-            a.xyz = xyz;
-            a.err = derr;
-            hipLaunchKernelGGL(k_table_from_V, dim3(nblk(n, 256)), dim3(256), 0, s, a);
-            PLB_HIP(hipGetLastError());
-        }
-        PLB_HIP(hipMemcpyAsync(&herr, derr, sizeof(int), hipMemcpyDeviceToHost, s));
-        PLB_HIP(hipStreamSynchronize(s));
-    }
+    PLB_HIP(dstart.alloc(c->num_p));
+    PLB_HIP(tabref.alloc((Q - 1) * n));
+    PLB_HIP(xyz.alloc(n));
+    PLB_HIP(derr.alloc(1));
+    PLB_HIP(hipMemsetAsync(derr, 0, sizeof(int), s));
+    PLB_HIP(hipMemcpyAsync(dstart, c->V_sub_start.data(), sizeof(int32_t) * c->num_p, hipMemcpyHostToDevice, s));
+    VArgs a;
+    a.N = n;
+    a.start = dstart;
+    a.num_p = c->num_p;
+    a.nx = c->nx;
+    a.ny = c->ny;
+    a.nz = c->nz;
+    a.mode = c->cfg.bb_mode;
+    a.tab = tabref;
+    a.xyz = xyz;
+    a.err = derr;
+    const int rc = upload(c->device, s, n, sizeof(plb_node_info), V, [&](int64_t first, int64_t m, void* d) {
+        a.V = (const uint64_t*)d;
+        a.first = first;
+        a.last = first + m;
+        hipLaunchKernelGGL(k_table_from_V, dim3(nblk(m, 256)), dim3(256), 0, s, a);
+        PLB_HIP(hipGetLastError());
+        return PLB_OK;
+    });
+    if (rc) return rc;
+    PLB_HIP(hipMemcpyAsync(&herr, derr, sizeof(int), hipMemcpyDeviceToHost, s));
+    PLB_HIP(hipStreamSynchronize(s));
     return herr ? herr : finalize_table(c, tabref, xyz);
 }
 
@@ -810,20 +810,23 @@ static int index_flag(const uint8_t* flag, int nx, int ny, int nz, hipStream_t s
     uint64_t last_pre = 0, last_cnt = 0;
     int herr = 0;
     {
-        DevBuf<uint8_t> dflag;
         DevBuf<uint64_t> cnt;
         DevBuf<int> derr;
-        PLB_HIP(dflag.alloc(fi.nvox));
         PLB_HIP(fi.bits.alloc(fi.nwords));
         PLB_HIP(cnt.alloc(fi.nwords));
         PLB_HIP(fi.wpre.alloc(fi.nwords));
         PLB_HIP(derr.alloc(1));
         PLB_HIP(hipMemsetAsync(derr, 0, sizeof(int), s));
-        PLB_HIP(hipMemcpyAsync(dflag, flag, fi.nvox, hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(k_flag_bits, dim3(nblk(fi.nvox, 256)), dim3(256), 0, s, dflag.p, fi.nvox,
-                           fi.nwords, fi.bits.p, cnt.p, derr.p);
-        PLB_HIP(hipGetLastError());
-        int rc = exclusive_scan_u64(cnt, fi.wpre, fi.nwords, s);
+        int device = 0;
+        PLB_HIP(hipGetDevice(&device));
+        int rc = upload(device, s, fi.nvox, 1, flag, [&](int64_t first, int64_t m, void* d) {
+            hipLaunchKernelGGL(k_flag_bits, dim3(nblk(m, 256)), dim3(256), 0, s, (const uint8_t*)d, m, (m + 63) / 64,
+                               fi.bits.p + first / 64, cnt.p + first / 64, derr.p);
+            PLB_HIP(hipGetLastError());
+            return PLB_OK;
+        });
+        if (rc) return rc;
+        rc = exclusive_scan_u64(cnt, fi.wpre, fi.nwords, s);
         if (rc) return rc;
         PLB_HIP(hipMemcpyAsync(&last_pre, fi.wpre.p + fi.nwords - 1, 8, hipMemcpyDeviceToHost, s));
         PLB_HIP(hipMemcpyAsync(&last_cnt, cnt.p + fi.nwords - 1, 8, hipMemcpyDeviceToHost, s));
@@ -924,7 +927,7 @@ int copy_table_offset(int layout, const int32_t* tabref, int64_t n, int64_t off,
 using namespace plb;
 
 // Device preprocess on its own stream; the stream is destroyed on every path.
-static int preprocess_on(hipStream_t s, const uint8_t* flag, int nx, int ny, int nz, int num_p,
+static int preprocess_on(int device, hipStream_t s, const uint8_t* flag, int nx, int ny, int nz, int num_p,
                          plb_node_info* V_out, int32_t* V_sub_start_out, int64_t* n_nodes_out)
 {
     FlagIndex fi;
@@ -946,21 +949,15 @@ static int preprocess_on(hipStream_t s, const uint8_t* flag, int nx, int ny, int
     if (V_sub_start_out)
         PLB_HIP(hipMemcpyAsync(V_sub_start_out, dstart, sizeof(int32_t) * num_p, hipMemcpyDeviceToHost, s));
     if (V_out && fi.N) {
-        // Records are produced in chunks so the device copy stays bounded.
-        const int64_t chunk = 16 * 1024 * 1024;
-        DevBuf<plb_node_info> dV;
-        PLB_HIP(dV.alloc(fi.N < chunk ? fi.N : chunk));
-        for (int64_t b0 = 0; b0 < fi.N; b0 += chunk) {
-            const int64_t m = (fi.N - b0 < chunk) ? fi.N - b0 : chunk;
+        rc = download(device, s, fi.N, sizeof(plb_node_info), {(char*)V_out}, [&](int64_t first, int64_t m, void* d) {
             GridArgs ac = a;
-            ac.xyz = fi.xyz.p + b0;
+            ac.xyz = fi.xyz.p + first;
             ac.N = m;
-            hipLaunchKernelGGL(k_V_from_bits, dim3(nblk(m, 256)), dim3(256), 0, s, ac, dstart.p,
-                               (uint64_t*)dV.p);
+            hipLaunchKernelGGL(k_V_from_bits, dim3(nblk(m, 256)), dim3(256), 0, s, ac, dstart.p, (uint64_t*)d);
             PLB_HIP(hipGetLastError());
-            PLB_HIP(hipMemcpyAsync(V_out + b0, dV, sizeof(plb_node_info) * m, hipMemcpyDeviceToHost, s));
-            PLB_HIP(hipStreamSynchronize(s));
-        }
+            return PLB_OK;
+        });
+        if (rc) return rc;
     }
     PLB_HIP(hipStreamSynchronize(s));
     return PLB_OK;
@@ -981,7 +978,7 @@ extern "C" int plb_preprocess(const uint8_t* flag, int nx, int ny, int nz, int n
     PLB_HIP(hipSetDevice(device));
     hipStream_t s;
     PLB_HIP(hipStreamCreate(&s));
-    const int rc = preprocess_on(s, flag, nx, ny, nz, num_p, V_out, V_sub_start_out, n_nodes_out);
+    const int rc = preprocess_on(device, s, flag, nx, ny, nz, num_p, V_out, V_sub_start_out, n_nodes_out);
     (void)hipStreamDestroy(s);
     return rc;
 }

@@ -118,6 +118,7 @@ struct Segment {
 struct plb_ctx {
     plb_config cfg;
     int device = 0;
+    bool counted = false;       // among the contexts that keep the transfer slots
     int lds_per_cu = 0;         // bytes of LDS per CU (occupancy cap of the step kernel)
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -258,7 +259,11 @@ int launch_step_batch(plb_ctx* c, int64_t it, bool write_macros, const int32_t* 
 int launch_init_eq(plb_ctx* c);
 int launch_read_pop(plb_ctx* c, int64_t first, int64_t n, double* dout);
 int launch_write_pop(plb_ctx* c, int64_t first, int64_t n, const double* din);
-int launch_read_macros(plb_ctx* c, int comp, int64_t first, int64_t n, double* dout);
+struct MacroList {           // which of rho, ux, uy, uz
+    int n = 0, comp[4] = {0, 0, 0, 0};
+};
+int launch_read_macros(plb_ctx* c, const MacroList& list, int64_t first, int64_t n, double* dout);
+int read_macros_range(plb_ctx* c, int64_t first, int64_t n, double* rho, double* ux, double* uy, double* uz);
 int launch_copy_state(plb_ctx* c, int64_t first, int64_t n, void* aos, bool to_device);
 int launch_read_table(plb_ctx* c, int64_t first, int64_t n, int32_t* dout);
 int launch_reduce_range(plb_ctx* c, int buf, int64_t first, int64_t n, bool with_mass,
