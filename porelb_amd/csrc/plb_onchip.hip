@@ -468,11 +468,13 @@ __global__ void __launch_bounds__(MAXT) k_onchip(StepArgs a, const OnchipArgs p)
     }
     const S* __restrict__ fin = (const S*)a.fin;
     uint32_t node[K], w[K][9], key[K], s0[K], s1[K];
+    bool any[K];   // whether the wave has nodes in its k-th group
     const bool sr = sizeof(S) == 2 && a.stochastic;
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const int slot = k * T + tid;
         node[k] = p.node[blk * NS + slot];
+        any[k] = k == 0 || __builtin_amdgcn_ballot_w64(node[k] != EMPTY) != 0;
 #pragma unroll
         for (int q = 0; q < 9; q++) w[k][q] = p.idx[(blk * 9 + q) * NS + slot];
         const int64_t g = blk * (NS / 64) + k * (T / 64) + wave;
@@ -668,6 +670,7 @@ __global__ void __launch_bounds__(MAXT) k_onchip(StepArgs a, const OnchipArgs p)
         if constexpr (TWICE) {
 #pragma unroll
             for (int k = 0; k < K; k++) {
+                if (!any[k]) break;
                 update(k, [&](int j) { return cell_at(k, j); });
                 if (!last) send(k, G, tag + 1);
                 if constexpr (K > 1) __builtin_amdgcn_sched_barrier(0);  // one node's values at a time
@@ -678,12 +681,15 @@ __global__ void __launch_bounds__(MAXT) k_onchip(StepArgs a, const OnchipArgs p)
         } else {
             S raw[K][Q];
 #pragma unroll
-            for (int k = 0; k < K; k++)
+            for (int k = 0; k < K; k++) {
+                if (!any[k]) break;
 #pragma unroll
                 for (int j = 0; j < Q; j++) raw[k][j] = cell_at(k, j);
+            }
             __syncthreads();  // every gather is done
 #pragma unroll
             for (int k = 0; k < K; k++) {
+                if (!any[k]) break;
                 update(k, [&](int j) { return raw[k][j]; });
                 if (!last) send(k, G, tag + 1);
                 if constexpr (K > 1) __builtin_amdgcn_sched_barrier(0);
@@ -734,14 +740,19 @@ static size_t lds_bytes(const plb_ctx* c, int NS, bool twice)
 {
     return ((size_t)Q * NS + EXTRA) * c->elem * (twice ? 2 : 1);
 }
+// Two nodes per thread: always 1024 threads, of which the second nodes may keep
+// only some waves busy (1 037 nodes: 576 threads took 6.0 to 7.8 us a step, 1024 take 5.0 to 5.5).
+static int slots_for(int nodes) { return nodes > 1024 ? 2048 : (nodes + 63) / 64 * 64; }
 static bool fits_twice(const plb_ctx* c, int NS) { return lds_bytes(c, NS, true) + 64 <= (size_t)c->lds_per_cu; }
-static bool fits(const plb_ctx* c, int NS)
+static bool fits(const plb_ctx* c, int nodes)
 {
     // FP16 blocks of more than 2048 slots (3 nodes per thread, one copy) spill:
     // 22 us a step for 629 146 nodes, against 16.8 us with one launch per step.
     const int most = c->cfg.precision == PLB_FP64 ? 1024 : 2048;
+    if (nodes > most) return false;
+    const int NS = slots_for(nodes);
     if (c->cfg.precision == PLB_FP16 && !fits_twice(c, NS)) return false;
-    return NS <= most && lds_bytes(c, NS, false) + 64 <= (size_t)c->lds_per_cu;
+    return lds_bytes(c, NS, false) + 64 <= (size_t)c->lds_per_cu;
 }
 
 template <typename F>
@@ -762,10 +773,9 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
     c->chip = p;
     hipStream_t s = c->stream;
     p->G = G;
-    p->K = (NS + 1023) / 1024;
-    p->NS = (NS + 64 * p->K - 1) / (64 * p->K) * (64 * p->K);
-    p->T = p->NS / p->K;
-    NS = p->NS;
+    p->K = NS > 1024 ? 2 : 1;
+    p->NS = NS = slots_for(NS);
+    p->T = NS / p->K;
     p->twice = fits_twice(c, NS);
     const int ng = NS / 64;
     const int64_t Ntot = c->N;
@@ -1008,14 +1018,14 @@ void onchip_pack(const std::vector<int>& blocks, int cus, std::vector<std::vecto
     }
 }
 
-// Time of a step of a launch with blocks of NS slots, in ns: fits of 64^3 to
-// 112^3 noise and sphere masks (FP32: 2.6 us at 512 slots, 3.3 at 1024, and
-// about 7 for two nodes per thread; FP64: 4.2 at 512, 6.1 at 1024).
+// Time of a step of a launch with blocks of up to NS nodes, in ns: fits of 64^3 to
+// 112^3 noise and sphere masks (FP32: 2.6 us at 512 nodes, 3.3 at 1024, 4.9 at
+// 1152 and 6.8 at 2048; FP64: 4.2 at 512, 6.1 at 1024).
 static int64_t step_ns(const plb_ctx* c, int NS)
 {
     if (c->cfg.precision == PLB_FP64) return NS <= 512 ? 3900 + NS / 2 : 3700 + NS * 9 / 4;
-    if (c->cfg.precision == PLB_FP32) return NS <= 1024 ? 2100 + NS * 8 / 7 : 6000 + NS * 4 / 9;
-    return NS <= 1024 ? 2500 + NS : 8000;
+    if (c->cfg.precision == PLB_FP32) return NS <= 1024 ? 2100 + NS * 8 / 7 : 2600 + NS * 2;
+    return NS <= 1024 ? 2500 + NS : 1500 + NS * 20 / 7;
 }
 
 bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::vector<int64_t>& n,
@@ -1027,8 +1037,7 @@ bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) return false;
     int most = 0;
-    for (int NS = 64; NS <= 4096 && fits(c, NS); NS += 64)
-        if (NS <= 1024 || NS % 128 == 0) most = NS;
+    for (int q = 64; q <= 4096 && fits(c, q); q += 64) most = q;
     std::vector<OnchipSample> samples(n.size());
     std::vector<int> blocks(n.size());
     std::vector<std::vector<int>> launches;
@@ -1055,7 +1064,7 @@ bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::
     // larger blocks: fewer launches for a step of the whole batch, each longer
     int NS = 0;
     int64_t cost = 0;
-    for (int q = ONCHIP_MIN_SLOTS; q <= most; q += q < 1024 ? 64 : 128) {
+    for (int q = ONCHIP_MIN_SLOTS; q <= most; q += 64) {
         if (!divide(q)) continue;
         const int64_t w = (int64_t)launches.size() * step_ns(c, q);
         if (NS == 0 || w < cost) {
