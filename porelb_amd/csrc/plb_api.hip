@@ -152,21 +152,21 @@ int plb::ctx_begin(plb_ctx* c, const plb_config* cfg, int nx, int ny, int nz, in
 int plb::ctx_alloc_state(plb_ctx* c)
 {
     const size_t nf = (size_t)c->Npad * Q * c->elem;
-    PLB_HIP(hipMalloc(&c->f[0], nf));
+    PLB_HIP(c->mem.take(&c->f[0], nf));
     if (c->cfg.stream_mode == PLB_STREAM_AA)
         c->f[1] = c->f[0];  // one buffer; c->cur is the AA phase
     else
-        PLB_HIP(hipMalloc(&c->f[1], nf));
-    PLB_HIP(hipMalloc(&c->macros, sizeof(double) * 4 * c->Npad));
+        PLB_HIP(c->mem.take(&c->f[1], nf));
+    PLB_HIP(c->mem.take(&c->macros, 4 * c->Npad));
     PLB_HIP(hipMemsetAsync(c->macros, 0, sizeof(double) * 4 * c->Npad, c->stream));
-    PLB_HIP(hipMalloc(&c->fault, 2 * sizeof(unsigned long long)));
+    PLB_HIP(c->mem.take(&c->fault, 2));
     PLB_HIP(hipMemsetAsync(c->fault, 0xff, 2 * sizeof(unsigned long long), c->stream));
     PLB_HIP(hipHostMalloc((void**)&c->host_words, 2 * sizeof(unsigned long long), hipHostMallocDefault));
     int dev_cus = 256;
     (void)hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, c->device);
     c->red_blocks = std::max(1, std::min<int>(dev_cus * 4, (int)((c->N + 255) / 256)));
-    PLB_HIP(hipMalloc(&c->red, sizeof(double) * (2 * c->red_blocks + 2)));
-    PLB_HIP(hipMalloc(&c->it_dev, sizeof(int64_t)));
+    PLB_HIP(c->mem.take(&c->red, 2 * c->red_blocks + 2));
+    PLB_HIP(c->mem.take(&c->it_dev, 1));
     PLB_HIP(hipStreamSynchronize(c->stream));
     if (c->cfg.precision == PLB_FP16 && c->cfg.fp16_rounding == PLB_ROUND_STOCHASTIC) {
         c->key_bytes = 4.0;
@@ -183,17 +183,13 @@ extern "C" void plb_destroy(plb_ctx* c)
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
     }
-    void* ptrs[] = {c->f[0], c->f[1] != c->f[0] ? c->f[1] : nullptr, c->tab, c->tdesc, c->toff, c->toff16, c->twide, c->bm, c->vox, c->perm,
-                    c->inv_perm, c->key_perm, c->kseg, c->node_xyz, c->macros, c->fault, c->red, c->reserve};
-    for (void* p : ptrs)
-        if (p) (void)hipFree(p);
     if (c->host_words) (void)hipHostFree(c->host_words);
     onchip_destroy(c);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     for (hipGraphExec_t& g : c->gexec)
         if (g) (void)hipGraphExecDestroy(g);
-    if (c->it_dev) (void)hipFree(c->it_dev);
+    if (c->reserve) (void)hipFree(c->reserve);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     if (c->counted) xfer_context(-1);
     delete c;

@@ -107,7 +107,7 @@ static int batch_build(plb_batch* b, const plb_config* cfg, const plb_sample* sm
             if (scfg.ordering == PLB_ORDER_PENCIL) scfg.brick[0] = smp[s].nx;
             int32_t* t2 = nullptr;
             rc = compute_order(scfg, smp[s].nx, smp[s].ny, smp[s].nz, ns, xyzs[s], c->stream, &invs[s],
-                               nullptr, nullptr);
+                               nullptr, nullptr, nullptr, nullptr, nullptr);
             if (!rc && hipMalloc(&t2, sizeof(int32_t) * (Q - 1) * ns) != hipSuccess) rc = PLB_ERR_NOMEM;
             if (!rc) rc = permute_ref_table(tabs[s], ns, invs[s], t2, c->stream);
             if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = PLB_ERR_HIP;
@@ -126,13 +126,13 @@ static int batch_build(plb_batch* b, const plb_config* cfg, const plb_sample* sm
     if (!rc) {
         c->N = total;
         c->Npad = total;
-        hipError_t e = hipMalloc(&c->tab, sizeof(int32_t) * (Q - 1) * total);
+        hipError_t e = c->mem.take(&c->tab, (Q - 1) * total);
         if (e == hipSuccess) e = hipMemsetAsync(c->tab, 0, sizeof(int32_t) * (Q - 1) * total, c->stream);
-        if (e == hipSuccess) e = hipMalloc(&c->node_xyz, sizeof(uint64_t) * total);
-        if (e == hipSuccess) e = hipMalloc(&c->inv_perm, sizeof(uint32_t) * total);
-        if (e == hipSuccess) e = hipMalloc(&c->key_perm, sizeof(uint32_t) * total);
+        if (e == hipSuccess) e = c->mem.take(&c->node_xyz, total);
+        if (e == hipSuccess) e = c->mem.take(&c->inv_perm, total);
+        if (e == hipSuccess) e = c->mem.take(&c->key_perm, total);
         if (e == hipSuccess) e = hipMemsetAsync(c->key_perm, 0, sizeof(uint32_t) * total, c->stream);
-        if (e == hipSuccess) e = hipMalloc(&c->perm, sizeof(uint32_t) * total);
+        if (e == hipSuccess) e = c->mem.take(&c->perm, total);
         if (e == hipSuccess) e = hipMemsetAsync(c->perm, 0, sizeof(uint32_t) * total, c->stream);
         if (e != hipSuccess) rc = e == hipErrorOutOfMemory ? PLB_ERR_NOMEM : PLB_ERR_HIP;
     }
@@ -157,7 +157,7 @@ static int batch_build(plb_batch* b, const plb_config* cfg, const plb_sample* sm
         if (invs[s]) (void)hipFree(invs[s]);
     }
     c->index_bytes = (Q - 1) * 4.0;
-    if (!rc && cfg->index_kind == PLB_INDEX_TILE8) rc = compress_tile8(c);
+    if (!rc && cfg->index_kind == PLB_INDEX_TILE8) rc = compress_tile8(c, &c->mem);
     return rc;
 }
 

@@ -74,15 +74,58 @@ __global__ void k_scan_add(uint64_t* out, const uint64_t* boff, int64_t n)
     if (i < n) out[i] += boff[i / SCAN_PER_BLOCK];
 }
 
-int exclusive_scan_u64(const uint64_t* in, uint64_t* out, int64_t n, hipStream_t s)
+// The whole scan by one block: up to SCAN_ONE values, where the three launches
+// and the partial sums of the blocks would cost more (74 664 values: 17 us).
+constexpr int64_t SCAN_ONE = (int64_t)1 << 17;
+__global__ void __launch_bounds__(1024)
+k_scan_one(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, int64_t n)
+{
+    constexpr int PER = 8;
+    __shared__ uint64_t wsum[16];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    uint64_t carry = 0;
+    for (int64_t b = 0; b < n; b += 1024 * PER) {
+        uint64_t v[PER], sum = 0;
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int64_t i = b + (int64_t)tid * PER + k;
+            v[k] = i < n ? in[i] : 0;
+            sum += v[k];
+        }
+        uint64_t inc = sum;
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) {
+            const uint64_t t = __shfl_up(inc, m, 64);
+            if (lane >= m) inc += t;
+        }
+        if (lane == 63) wsum[w] = inc;
+        __syncthreads();
+        uint64_t before = 0, total = 0;
+        for (int q = 0; q < 16; q++) {
+            if (q < w) before += wsum[q];
+            total += wsum[q];
+        }
+        uint64_t e = carry + before + inc - sum;
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int64_t i = b + (int64_t)tid * PER + k;
+            if (i < n) out[i] = e;
+            e += v[k];
+        }
+        carry += total;
+        __syncthreads();
+    }
+}
+
+static int exclusive_scan_u64(const uint64_t* in, uint64_t* out, int64_t n, hipStream_t s)
 {
     if (n <= 0) return PLB_OK;
-    int64_t nb = (n + SCAN_PER_BLOCK - 1) / SCAN_PER_BLOCK;
-    if (nb == 1) {
-        hipLaunchKernelGGL(k_scan_block, dim3(1), dim3(SCAN_T), 0, s, in, out, nullptr, n);
+    if (n <= SCAN_ONE) {
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, in, out, n);
         PLB_HIP(hipGetLastError());
         return PLB_OK;
     }
+    int64_t nb = (n + SCAN_PER_BLOCK - 1) / SCAN_PER_BLOCK;
     DevBuf<uint64_t> bsum, boff;
     PLB_HIP(bsum.alloc(nb));
     PLB_HIP(boff.alloc(nb));
@@ -160,6 +203,20 @@ __device__ __forceinline__ int64_t lin(const GridArgs& a, int x, int y, int z)
 }
 __device__ __forceinline__ int wrap(int v, int n) { return (v + n) % n; }
 
+// Pull entry (g, j) of the node at x, y, z on rank p, in V order.
+__device__ __forceinline__ int32_t entry_from_bits(const GridArgs& a, int mode, int j, int64_t g, int x, int y, int z, int p)
+{
+    const int zu = wrap(z - EZ[j], a.nz);
+    const int64_t vu = lin(a, wrap(x - EX[j], a.nx), wrap(y - EY[j], a.ny), zu);
+    const bool up = is_pore(a.bits, vu);
+    if (mode == PLB_BB_HALFWAY) return up ? (int32_t)pore_id(a.bits, a.wpre, vu) : TAB_BOUNCE;
+    const int64_t vd = lin(a, wrap(x + EX[j], a.nx), wrap(y + EY[j], a.ny), wrap(z + EZ[j], a.nz));
+    const bool dn = is_pore(a.bits, vd);
+    const int64_t uid = up ? pore_id(a.bits, a.wpre, vu) : -1;
+    if (up && (dn || (zu / a.slab) != p || uid > g)) return (int32_t)uid;
+    return dn ? TAB_CONST : TAB_BOUNCE;
+}
+
 // Pull table straight from the voxel bitmask (V order, [18][N]).
 __global__ void k_table_from_bits(GridArgs a, int mode, int32_t* __restrict__ tab)
 {
@@ -169,25 +226,30 @@ __global__ void k_table_from_bits(GridArgs a, int mode, int32_t* __restrict__ ta
     unpack(a.xyz[g], x, y, z);
     const int p = z / a.slab;
 #pragma unroll
+    for (int j = 1; j < Q; j++) tab[(int64_t)(j - 1) * a.N + g] = entry_from_bits(a, mode, j, g, x, y, z, p);
+}
+
+// The same in the lattice's node order and layout (a.xyz in that order too):
+// no V-order table is written and permuted.
+template <int LAYOUT>
+__global__ void k_order_table_from_bits(GridArgs a, int mode, const uint32_t* __restrict__ perm,
+                                        const uint32_t* __restrict__ inv_perm, int64_t npad, int32_t* __restrict__ tab)
+{
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= npad) return;
+    if (k >= a.N) {
+        for (int j = 0; j < Q - 1; j++) tab[tpos<LAYOUT>(j, k, npad)] = 0;
+        return;
+    }
+    int x, y, z;
+    unpack(a.xyz[k], x, y, z);
+    const int p = z / a.slab;
+    const int64_t g = perm ? (int64_t)perm[k] : k;
+#pragma unroll
     for (int j = 1; j < Q; j++) {
-        const int64_t vd = lin(a, wrap(x + EX[j], a.nx), wrap(y + EY[j], a.ny), wrap(z + EZ[j], a.nz));
-        const int zu = wrap(z - EZ[j], a.nz);
-        const int64_t vu = lin(a, wrap(x - EX[j], a.nx), wrap(y - EY[j], a.ny), zu);
-        const bool up = is_pore(a.bits, vu);
-        int32_t t;
-        if (mode == PLB_BB_HALFWAY) {
-            t = up ? (int32_t)pore_id(a.bits, a.wpre, vu) : TAB_BOUNCE;
-        } else {
-            const bool dn = is_pore(a.bits, vd);
-            const int64_t uid = up ? pore_id(a.bits, a.wpre, vu) : -1;
-            if (up && (dn || (zu / a.slab) != p || uid > g))
-                t = (int32_t)uid;
-            else if (!dn)
-                t = TAB_BOUNCE;
-            else
-                t = TAB_CONST;
-        }
-        tab[(int64_t)(j - 1) * a.N + g] = t;
+        int32_t t = entry_from_bits(a, mode, j, g, x, y, z, p);
+        if (t >= 0 && inv_perm) t = (int32_t)inv_perm[t];
+        tab[tpos<LAYOUT>(j - 1, k, npad)] = t;
     }
 }
 
@@ -337,6 +399,43 @@ __global__ void k_brick_bits(const uint64_t* __restrict__ xyz, int64_t N, BrickA
     atomicOr(bits + (v >> 6), 1ull << (v & 63));
 }
 
+// The same bits where the mask is at hand: every word gathers its 64 voxels, so
+// there is no atomic per node (265 421 nodes: 19 us with atomics).
+__global__ void k_brick_words(const uint64_t* __restrict__ flag_bits, BrickArgs b, int64_t nvb, uint64_t* __restrict__ bits,
+                              uint64_t* __restrict__ cnt)
+{
+    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    bool pore = false;
+    if (v < nvb) {
+        const int64_t vol = (int64_t)b.bx * b.by * b.bz;
+        int64_t brick = v / vol;
+        int64_t in = v - brick * vol;
+        uint32_t kx, ky, kz;
+        if (b.zfast) {
+            kz = (uint32_t)(brick % b.nbz);
+            brick /= b.nbz;
+            ky = (uint32_t)(brick % b.nby);
+            kx = (uint32_t)(brick / b.nby);
+        } else {
+            kx = (uint32_t)(brick % b.nbx);
+            brick /= b.nbx;
+            ky = (uint32_t)(brick % b.nby);
+            kz = (uint32_t)(brick / b.nby);
+        }
+        const uint32_t lx = (uint32_t)(in % b.bx);
+        in /= b.bx;
+        const uint32_t x = kx * b.bx + lx, y = ky * b.by + (uint32_t)(in % b.by),
+                       z = kz * b.bz + (uint32_t)(in / b.by);
+        if (x < (uint32_t)b.nx && y < (uint32_t)b.ny && z < (uint32_t)b.nz)
+            pore = is_pore(flag_bits, ((int64_t)z * b.ny + y) * b.nx + x);
+    }
+    const uint64_t m = __builtin_amdgcn_ballot_w64(pore);
+    if ((threadIdx.x & 63) == 0 && v < nvb) {
+        bits[v >> 6] = m;
+        cnt[v >> 6] = __popcll(m);
+    }
+}
+
 __global__ void k_popc_words(const uint64_t* bits, uint64_t* cnt, int64_t nw)
 {
     const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -378,9 +477,12 @@ static unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); 
 
 // Node order of a lattice: inv_perm[g] = internal id of V-order node g,
 // perm = its inverse, xyz_int = coordinates in internal order.  For the
-// reference order nothing is allocated (identity).
+// reference order nothing is allocated (identity).  The maps come from `keep`,
+// the rest from `scratch` (null: allocations of their own); flag_bits = the mask
+// as bits in V order, where there is one.
 int compute_order(const plb_config& cfg, int nx, int ny, int nz, int64_t N, const uint64_t* xyz_ref,
-                  hipStream_t s, uint32_t** inv_perm, uint32_t** perm, uint64_t* xyz_int)
+                  hipStream_t s, uint32_t** inv_perm, uint32_t** perm, uint64_t* xyz_int, Arena* keep, Arena* scratch,
+                  const uint64_t* flag_bits)
 {
     *inv_perm = nullptr;
     if (perm) *perm = nullptr;
@@ -405,27 +507,33 @@ int compute_order(const plb_config& cfg, int nx, int ny, int nz, int64_t N, cons
     const int64_t nw = (nvb + 63) / 64;
     DevBuf<uint64_t> bits, cnt, wpre, xyz_tmp;
     DevBuf<uint32_t> inv, p;
-    PLB_HIP(bits.alloc(nw));
-    PLB_HIP(cnt.alloc(nw));
-    PLB_HIP(wpre.alloc(nw));
-    PLB_HIP(hipMemsetAsync(bits, 0, sizeof(uint64_t) * nw, s));
-    hipLaunchKernelGGL(k_brick_bits, dim3(nblk(N, 256)), dim3(256), 0, s, xyz_ref, N, b,
-                       (unsigned long long*)bits.p);
-    hipLaunchKernelGGL(k_popc_words, dim3(nblk(nw, 256)), dim3(256), 0, s, bits.p, cnt.p, nw);
+    PLB_HIP(bits.alloc(nw, scratch));
+    PLB_HIP(cnt.alloc(nw, scratch));
+    PLB_HIP(wpre.alloc(nw, scratch));
+    if (flag_bits) {
+        hipLaunchKernelGGL(k_brick_words, dim3(nblk(nw * 64, 256)), dim3(256), 0, s, flag_bits, b, nvb, bits.p, cnt.p);
+    } else {
+        PLB_HIP(hipMemsetAsync(bits, 0, sizeof(uint64_t) * nw, s));
+        hipLaunchKernelGGL(k_brick_bits, dim3(nblk(N, 256)), dim3(256), 0, s, xyz_ref, N, b,
+                           (unsigned long long*)bits.p);
+        hipLaunchKernelGGL(k_popc_words, dim3(nblk(nw, 256)), dim3(256), 0, s, bits.p, cnt.p, nw);
+    }
     PLB_HIP(hipGetLastError());
     int rc = exclusive_scan_u64(cnt, wpre, nw, s);
     if (rc) return rc;
-    // Every node must own a voxel of its own: two records with the same
-    // coordinates would get the same internal id, race on its table row and
-    // leave another id unassigned.  The set bits count the distinct voxels.
-    uint64_t last[2] = {0, 0};
-    PLB_HIP(hipMemcpyAsync(&last[0], wpre.p + nw - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-    PLB_HIP(hipMemcpyAsync(&last[1], cnt.p + nw - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-    PLB_HIP(hipStreamSynchronize(s));
-    if ((int64_t)(last[0] + last[1]) != N) return PLB_ERR_BOUNDS;
-    PLB_HIP(inv.alloc(N));
-    PLB_HIP(p.alloc(N));
-    if (!xyz_int) PLB_HIP(xyz_tmp.alloc(N));
+    if (!flag_bits) {
+        // Every node must own a voxel of its own: two records with the same
+        // coordinates would get the same internal id, race on its table row and
+        // leave another id unassigned.  The set bits count the distinct voxels.
+        uint64_t last[2] = {0, 0};
+        PLB_HIP(hipMemcpyAsync(&last[0], wpre.p + nw - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+        PLB_HIP(hipMemcpyAsync(&last[1], cnt.p + nw - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+        PLB_HIP(hipStreamSynchronize(s));
+        if ((int64_t)(last[0] + last[1]) != N) return PLB_ERR_BOUNDS;
+    }
+    PLB_HIP(inv.alloc(N, keep));
+    PLB_HIP(p.alloc(N, keep));
+    if (!xyz_int) PLB_HIP(xyz_tmp.alloc(N, scratch));
     hipLaunchKernelGGL(k_brick_ids, dim3(nblk(N, 256)), dim3(256), 0, s, xyz_ref, N, b, bits.p, wpre.p,
                        inv.p, p.p, xyz_int ? xyz_int : xyz_tmp.p);
     PLB_HIP(hipGetLastError());
@@ -447,16 +555,54 @@ int permute_ref_table(const int32_t* tabref, int64_t n, const uint32_t* inv_perm
     return PLB_OK;
 }
 
-int finalize_table(plb_ctx* c, int32_t* tabref, const uint64_t* xyz_ref)
+static int build_bitmap(plb_ctx* c, Arena* scratch);
+
+// What the context and the build need for n nodes, taken at once for small lattices.
+static int reserve_for(plb_ctx* c, int64_t n, Arena* scratch)
+{
+    if (n > RESERVE_NODES) return PLB_OK;
+    const int64_t npad = std::max<int64_t>(64, (n + 63) / 64 * 64), tiles = npad / 64, nk = tiles * (Q - 1);
+    const bool tile8 = c->cfg.index_kind == PLB_INDEX_TILE8, i32 = c->cfg.index_kind == PLB_INDEX_I32;
+    const size_t slack = 64 * 256;
+    size_t keep = (size_t)npad * Q * c->elem * (c->cfg.stream_mode == PLB_STREAM_AA ? 1 : 2) + 32 * (size_t)npad +
+                  16 * (size_t)npad /* coordinates and order */ + 16 * (size_t)tiles /* FP16 keys */ + 65536 + slack;
+    size_t temp = 8 * (size_t)n + 6 * 8 * (size_t)(npad / 8) + slack;
+    if (tile8) keep += 4 * (size_t)nk + 18 * (size_t)npad;
+    if (i32) keep += 72 * (size_t)npad;
+    if (tile8) temp += 72 * (size_t)npad + 16 * (size_t)nk;
+    if (c->cfg.index_kind == PLB_INDEX_BITMAP) keep += 5 * (size_t)npad;
+    PLB_HIP(c->mem.reserve(keep));
+    PLB_HIP(scratch->reserve(temp));
+    return PLB_OK;
+}
+
+// The int32 table's place: the context's own, or only until it is encoded.
+static int take_table(plb_ctx* c, Arena* scratch)
+{
+    Arena& from = c->cfg.index_kind == PLB_INDEX_I32 ? c->mem : *scratch;
+    PLB_HIP(from.take(&c->tab, (Q - 1) * c->Npad));
+    return PLB_OK;
+}
+
+static int encode_table(plb_ctx* c, Arena* scratch)
+{
+    c->index_bytes = (Q - 1) * 4.0;
+    if (c->cfg.index_kind == PLB_INDEX_TILE8) return compress_tile8(c, scratch);
+    if (c->cfg.index_kind == PLB_INDEX_BITMAP) return build_bitmap(c, scratch);
+    return PLB_OK;
+}
+
+static int finalize_table(plb_ctx* c, int32_t* tabref, const uint64_t* xyz_ref, Arena* scratch)
 {
     const int64_t N = c->N;
     hipStream_t s = c->stream;
     const int64_t tab_elems = (Q - 1) * c->Npad;
-    PLB_HIP(hipMalloc(&c->tab, sizeof(int32_t) * tab_elems));
+    int rc = take_table(c, scratch);
+    if (rc) return rc;
     PLB_HIP(hipMemsetAsync(c->tab, 0, sizeof(int32_t) * tab_elems, s));
-    PLB_HIP(hipMalloc(&c->node_xyz, sizeof(uint64_t) * (N ? N : 1)));
-    int rc = compute_order(c->cfg, c->nx, c->ny, c->nz, N, xyz_ref, s, &c->inv_perm, &c->perm,
-                           c->node_xyz);
+    PLB_HIP(c->mem.take(&c->node_xyz, N));
+    rc = compute_order(c->cfg, c->nx, c->ny, c->nz, N, xyz_ref, s, &c->inv_perm, &c->perm, c->node_xyz, &c->mem,
+                       scratch, nullptr);
     if (rc) return rc;
     if (N > 0) {
         if (c->cfg.layout == PLB_LAYOUT_SOA)
@@ -468,10 +614,7 @@ int finalize_table(plb_ctx* c, int32_t* tabref, const uint64_t* xyz_ref)
         PLB_HIP(hipGetLastError());
     }
     PLB_HIP(hipStreamSynchronize(s));
-    c->index_bytes = (Q - 1) * 4.0;
-    if (c->cfg.index_kind == PLB_INDEX_TILE8) return compress_tile8(c);
-    if (c->cfg.index_kind == PLB_INDEX_BITMAP) return build_bitmap(c);
-    return PLB_OK;
+    return encode_table(c, scratch);
 }
 
 // ---------------------------------------------------------------- TILE8 index
@@ -555,14 +698,14 @@ k_tile8_write(const int32_t* __restrict__ tab, int64_t Npad, int64_t N,
 }
 
 // Replaces the int32 table of a context by the TILE8 encoding.
-int compress_tile8(plb_ctx* c)
+int compress_tile8(plb_ctx* c, Arena* scratch)
 {
     hipStream_t s = c->stream;
     const int64_t T = c->Npad / 64;
     const int64_t nk = T * (Q - 1);
     DevBuf<uint64_t> wide, slot;
-    PLB_HIP(wide.alloc(nk));
-    PLB_HIP(slot.alloc(nk));
+    PLB_HIP(wide.alloc(nk, scratch));
+    PLB_HIP(slot.alloc(nk, scratch));
     if (c->cfg.layout == PLB_LAYOUT_SOA)
         hipLaunchKernelGGL(k_tile8_flags<PLB_LAYOUT_SOA>, dim3((unsigned)T), dim3(64), 0, s, c->tab,
                            c->Npad, c->N, wide.p);
@@ -577,10 +720,10 @@ int compress_tile8(plb_ctx* c)
     PLB_HIP(hipMemcpyAsync(&last_wide, wide.p + nk - 1, 8, hipMemcpyDeviceToHost, s));
     PLB_HIP(hipStreamSynchronize(s));
     c->n_wide = (int64_t)(last_slot + last_wide);
-    PLB_HIP(hipMalloc(&c->tdesc, sizeof(int32_t) * nk));
-    PLB_HIP(hipMalloc(&c->toff, sizeof(uint32_t) * T * TILE8_FULL * 64));
-    PLB_HIP(hipMalloc(&c->toff16, sizeof(uint16_t) * T * 64));
-    PLB_HIP(hipMalloc(&c->twide, sizeof(int32_t) * 64 * (c->n_wide ? c->n_wide : 1)));
+    PLB_HIP(c->mem.take(&c->tdesc, nk));
+    PLB_HIP(c->mem.take(&c->toff, T * TILE8_FULL * 64));
+    PLB_HIP(c->mem.take(&c->toff16, T * 64));
+    PLB_HIP(c->mem.take(&c->twide, 64 * c->n_wide));
     if (c->cfg.layout == PLB_LAYOUT_SOA)
         hipLaunchKernelGGL(k_tile8_write<PLB_LAYOUT_SOA>, dim3((unsigned)T), dim3(64), 0, s, c->tab,
                            c->Npad, c->N, wide.p, slot.p, c->tdesc, c->toff, c->toff16, c->twide);
@@ -589,7 +732,7 @@ int compress_tile8(plb_ctx* c)
                            c->Npad, c->N, wide.p, slot.p, c->tdesc, c->toff, c->toff16, c->twide);
     PLB_HIP(hipGetLastError());
     PLB_HIP(hipStreamSynchronize(s));
-    (void)hipFree(c->tab);
+    scratch->give(c->tab);
     c->tab = nullptr;
     c->index_bytes = c->N ? ((double)T * (TILE8_FULL * 256 + 128) + (double)nk * 4 + (double)c->n_wide * 256) /
                                 (double)c->N
@@ -645,7 +788,7 @@ int build_key_runs(plb_ctx* c)
     DevBuf<unsigned long long> marked;
     PLB_HIP(marked.alloc(1));
     PLB_HIP(hipMemsetAsync(marked.p, 0, sizeof(unsigned long long), c->stream));
-    PLB_HIP(hipMalloc(&c->kseg, sizeof(uint4) * T));
+    PLB_HIP(c->mem.take(&c->kseg, T));
     hipLaunchKernelGGL(k_key_runs, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, c->stream, key, c->N, T,
                        c->kseg, marked.p);
     PLB_HIP(hipGetLastError());
@@ -703,8 +846,8 @@ __global__ void k_bm_check(const uint2* bm, const uint32_t* vox, int64_t N, int*
     if (!((wd.x >> b) & 1u) || (int64_t)id != g) *err = 1;
 }
 
-// Replaces the int32 table of a context by the BITMAP index.
-int build_bitmap(plb_ctx* c)
+// Replaces the int32 table of a context, if there is one, by the BITMAP index.
+static int build_bitmap(plb_ctx* c, Arena* scratch)
 {
     hipStream_t s = c->stream;
     const plb_config& cfg = c->cfg;
@@ -722,15 +865,15 @@ int build_bitmap(plb_ctx* c)
     DevBuf<uint32_t> bits;
     DevBuf<uint64_t> cnt, pre;
     DevBuf<int> derr;
-    PLB_HIP(bits.alloc(nw));
-    PLB_HIP(cnt.alloc(nw));
-    PLB_HIP(pre.alloc(nw));
-    PLB_HIP(derr.alloc(1));
+    PLB_HIP(bits.alloc(nw, scratch));
+    PLB_HIP(cnt.alloc(nw, scratch));
+    PLB_HIP(pre.alloc(nw, scratch));
+    PLB_HIP(derr.alloc(1, scratch));
     PLB_HIP(hipMemsetAsync(bits, 0, sizeof(uint32_t) * nw, s));
     PLB_HIP(hipMemsetAsync(derr, 0, sizeof(int), s));
-    PLB_HIP(hipMalloc(&c->vox, sizeof(uint32_t) * c->Npad));
+    PLB_HIP(c->mem.take(&c->vox, c->Npad));
     PLB_HIP(hipMemsetAsync(c->vox, 0, sizeof(uint32_t) * c->Npad, s));
-    PLB_HIP(hipMalloc(&c->bm, sizeof(uint2) * nw));
+    PLB_HIP(c->mem.take(&c->bm, nw));
     PencilMap m;
     m.nx = (uint32_t)c->nx;
     m.nz = (uint32_t)c->nz;
@@ -751,7 +894,7 @@ int build_bitmap(plb_ctx* c)
     PLB_HIP(hipMemcpyAsync(&herr, derr, sizeof(int), hipMemcpyDeviceToHost, s));
     PLB_HIP(hipStreamSynchronize(s));
     if (herr) return PLB_ERR_INVALID;  // node order and voxel order disagree
-    (void)hipFree(c->tab);
+    if (c->tab) scratch->give(c->tab);
     c->tab = nullptr;
     c->py = (int)py;
     c->n_bm_words = nw;
@@ -762,6 +905,7 @@ int build_bitmap(plb_ctx* c)
 int build_table_from_V(plb_ctx* c, const plb_node_info* V, int64_t n)
 {
     hipStream_t s = c->stream;
+    Arena scratch(s);
     DevBuf<uint64_t> xyz;
     DevBuf<int32_t> dstart, tabref;
     DevBuf<int> derr;
@@ -783,7 +927,9 @@ int build_table_from_V(plb_ctx* c, const plb_node_info* V, int64_t n)
     a.tab = tabref;
     a.xyz = xyz;
     a.err = derr;
-    const int rc = upload(c->device, s, n, sizeof(plb_node_info), V, [&](int64_t first, int64_t m, void* d) {
+    int rc = reserve_for(c, n, &scratch);
+    if (rc) return rc;
+    rc = upload(c->device, s, n, sizeof(plb_node_info), V, [&](int64_t first, int64_t m, void* d) {
         a.V = (const uint64_t*)d;
         a.first = first;
         a.last = first + m;
@@ -794,7 +940,7 @@ int build_table_from_V(plb_ctx* c, const plb_node_info* V, int64_t n)
     if (rc) return rc;
     PLB_HIP(hipMemcpyAsync(&herr, derr, sizeof(int), hipMemcpyDeviceToHost, s));
     PLB_HIP(hipStreamSynchronize(s));
-    return herr ? herr : finalize_table(c, tabref, xyz);
+    return herr ? herr : finalize_table(c, tabref, xyz, &scratch);
 }
 
 // Device-side mask analysis shared by plb_create_from_flag and plb_preprocess.
@@ -803,7 +949,7 @@ struct FlagIndex {
     int64_t N = 0, nvox = 0, nwords = 0;
 };
 
-static int index_flag(const uint8_t* flag, int nx, int ny, int nz, hipStream_t s, FlagIndex& fi)
+static int index_flag(const uint8_t* flag, int nx, int ny, int nz, hipStream_t s, FlagIndex& fi, Arena* scratch = nullptr)
 {
     fi.nvox = (int64_t)nx * ny * nz;
     fi.nwords = (fi.nvox + 63) / 64;
@@ -812,10 +958,11 @@ static int index_flag(const uint8_t* flag, int nx, int ny, int nz, hipStream_t s
     {
         DevBuf<uint64_t> cnt;
         DevBuf<int> derr;
-        PLB_HIP(fi.bits.alloc(fi.nwords));
-        PLB_HIP(cnt.alloc(fi.nwords));
-        PLB_HIP(fi.wpre.alloc(fi.nwords));
-        PLB_HIP(derr.alloc(1));
+        if (scratch && fi.nvox <= 16 * RESERVE_NODES) PLB_HIP(scratch->reserve(3 * 8 * (size_t)fi.nwords + 4096));
+        PLB_HIP(fi.bits.alloc(fi.nwords, scratch));
+        PLB_HIP(cnt.alloc(fi.nwords, scratch));
+        PLB_HIP(fi.wpre.alloc(fi.nwords, scratch));
+        PLB_HIP(derr.alloc(1, scratch));
         PLB_HIP(hipMemsetAsync(derr, 0, sizeof(int), s));
         int device = 0;
         PLB_HIP(hipGetDevice(&device));
@@ -882,15 +1029,49 @@ int build_ref_from_flag(const uint8_t* flag, int nx, int ny, int nz, int num_p, 
 
 int build_table_from_flag(plb_ctx* c, const uint8_t* flag)
 {
-    DevBuf<int32_t> tabref;
-    DevBuf<uint64_t> xyz;
-    int64_t n = 0;
-    int rc = build_ref_from_flag(flag, c->nx, c->ny, c->nz, c->num_p, c->cfg.bb_mode, c->stream,
-                                 &tabref.p, &xyz.p, &n, &c->V_sub_start);
+    hipStream_t s = c->stream;
+    Arena mask_mem(s), scratch(s);  // before the buffers that come from them
+    FlagIndex fi;
+    int rc = index_flag(flag, c->nx, c->ny, c->nz, s, fi, &mask_mem);
     if (rc) return rc;
-    c->N = n;
-    c->Npad = std::max<int64_t>(64, (n + 63) / 64 * 64);
-    return finalize_table(c, tabref, xyz);
+    c->N = fi.N;
+    c->Npad = std::max<int64_t>(64, (fi.N + 63) / 64 * 64);
+    rc = reserve_for(c, fi.N, &scratch);
+    if (rc) return rc;
+    GridArgs a;
+    a.bits = fi.bits;
+    a.wpre = fi.wpre;
+    a.xyz = fi.xyz;
+    a.N = fi.N;
+    a.nx = c->nx;
+    a.ny = c->ny;
+    a.nz = c->nz;
+    a.slab = c->nz / c->num_p;
+    DevBuf<int32_t> dstart;
+    PLB_HIP(dstart.alloc(c->num_p, &scratch));
+    hipLaunchKernelGGL(k_slab_starts, dim3(nblk(c->num_p, 64)), dim3(64), 0, s, a, c->num_p, dstart.p);
+    c->V_sub_start.assign(c->num_p, 0);
+    PLB_HIP(hipMemcpyAsync(c->V_sub_start.data(), dstart, sizeof(int32_t) * c->num_p, hipMemcpyDeviceToHost, s));
+    PLB_HIP(c->mem.take(&c->node_xyz, fi.N));
+    rc = compute_order(c->cfg, c->nx, c->ny, c->nz, fi.N, fi.xyz, s, &c->inv_perm, &c->perm, c->node_xyz, &c->mem,
+                       &scratch, fi.bits);
+    if (rc) return rc;
+    if (c->cfg.index_kind != PLB_INDEX_BITMAP) {
+        rc = take_table(c, &scratch);
+        if (rc) return rc;
+        a.xyz = c->node_xyz;
+        const dim3 grid(nblk(c->Npad, 256));
+        if (c->cfg.layout == PLB_LAYOUT_SOA)
+            hipLaunchKernelGGL(k_order_table_from_bits<PLB_LAYOUT_SOA>, grid, dim3(256), 0, s, a, c->cfg.bb_mode, c->perm,
+                               c->inv_perm, c->Npad, c->tab);
+        else
+            hipLaunchKernelGGL(k_order_table_from_bits<PLB_LAYOUT_AOSOA>, grid, dim3(256), 0, s, a, c->cfg.bb_mode,
+                               c->perm, c->inv_perm, c->Npad, c->tab);
+        PLB_HIP(hipGetLastError());
+    }
+    rc = encode_table(c, &scratch);
+    PLB_HIP(hipStreamSynchronize(s));
+    return rc;
 }
 
 template <int LAYOUT>

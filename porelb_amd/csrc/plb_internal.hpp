@@ -105,6 +105,106 @@ __host__ __device__ __forceinline__ uint64_t pack_xyz(uint64_t x, uint64_t y, ui
 }  // namespace plb
 
 namespace plb {
+// Device memory that may come from, and go to, the kept blocks (plb_mem.hip).
+// dev_free: the work that uses the block has been waited for.
+hipError_t dev_alloc(void** p, size_t bytes);
+void dev_free(void* p);
+
+// Device memory with one owner.  reserve() takes one block that take() cuts
+// pieces from; what does not fit, or comes without a reserve, gets an
+// allocation of its own, and give() frees only that.  An allocation costs 25 to
+// 60 us and its release up to 200, so a small lattice is built in three reserves;
+// a large one (RESERVE_NODES) takes its arrays one by one, as it did, so that its
+// peak memory is not the sum of what it needs at different times.
+constexpr int64_t RESERVE_NODES = (int64_t)4 << 20;
+class Arena {
+public:
+    // stream: waited for before anything goes back (null: the owner has done so)
+    explicit Arena(hipStream_t stream = nullptr) : stream_(stream) {}
+    Arena(const Arena&) = delete;
+    Arena& operator=(const Arena&) = delete;
+    ~Arena()
+    {
+        if (stream_ && !own_.empty()) (void)hipStreamSynchronize(stream_);
+        for (void* p : own_) dev_free(p);
+    }
+    static size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+    hipError_t reserve(size_t bytes)
+    {
+        void* p = nullptr;
+        const hipError_t e = dev_alloc(&p, bytes);
+        if (e != hipSuccess) return e;
+        own_.push_back(p);
+        base_ = (char*)p;
+        size_ = bytes;
+        used_ = 0;
+        return hipSuccess;
+    }
+    hipError_t take(void** p, size_t bytes)
+    {
+        const size_t need = rounded(bytes ? bytes : 1);
+        if (base_ && used_ + need <= size_) {
+            *p = base_ + used_;
+            used_ += need;
+            return hipSuccess;
+        }
+        const hipError_t e = dev_alloc(p, need);
+        if (e == hipSuccess) own_.push_back(*p);
+        else *p = nullptr;
+        return e;
+    }
+    template <typename T>
+    hipError_t take(T** p, int64_t n)
+    {
+        return take((void**)p, sizeof(T) * (size_t)(n > 0 ? n : 1));
+    }
+    void give(void* p)
+    {
+        for (size_t k = 0; k < own_.size(); k++)
+            if (own_[k] == p && p != base_) {
+                if (stream_) (void)hipStreamSynchronize(stream_);
+                dev_free(p);
+                own_.erase(own_.begin() + k);
+                return;
+            }
+    }
+
+private:
+    std::vector<void*> own_;
+    hipStream_t stream_ = nullptr;
+    char* base_ = nullptr;
+    size_t size_ = 0, used_ = 0;
+};
+
+// Owner of a temporary device array: freed (or given back to its arena) on every return path.
+template <typename T>
+struct DevBuf {
+    T* p = nullptr;
+    Arena* from = nullptr;
+    DevBuf() = default;
+    DevBuf(const DevBuf&) = delete;
+    DevBuf& operator=(const DevBuf&) = delete;
+    ~DevBuf()
+    {
+        if (!p) return;
+        if (from) from->give(p);
+        else (void)hipFree(p);
+    }
+    hipError_t alloc(int64_t n, Arena* arena = nullptr)
+    {
+        from = arena;
+        if (arena) return arena->take(&p, n);
+        return hipMalloc((void**)&p, sizeof(T) * (size_t)(n > 0 ? n : 1));
+    }
+    T* release()
+    {
+        T* q = p;
+        p = nullptr;
+        return q;
+    }
+    operator T*() const { return p; }
+};
+
 struct OnchipPlan;
 // One plb_step_async call that plb_sync has not settled yet.
 struct Segment {
@@ -122,6 +222,7 @@ struct plb_ctx {
     int lds_per_cu = 0;         // bytes of LDS per CU (occupancy cap of the step kernel)
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    plb::Arena mem;             // every device array below except the placement reserve
     int64_t N = 0, Npad = 0;
     int nx = 0, ny = 0, nz = 0, num_p = 1;
     std::vector<int32_t> V_sub_start;
@@ -189,26 +290,6 @@ struct Range {
     Range& operator=(const Range&) = delete;
 };
 
-// Owner of a temporary device array: freed on every return path.
-template <typename T>
-struct DevBuf {
-    T* p = nullptr;
-    DevBuf() = default;
-    DevBuf(const DevBuf&) = delete;
-    DevBuf& operator=(const DevBuf&) = delete;
-    ~DevBuf()
-    {
-        if (p) (void)hipFree(p);
-    }
-    hipError_t alloc(int64_t n) { return hipMalloc((void**)&p, sizeof(T) * (size_t)(n > 0 ? n : 1)); }
-    T* release()
-    {
-        T* q = p;
-        p = nullptr;
-        return q;
-    }
-    operator T*() const { return p; }
-};
 }  // namespace plb
 
 
@@ -246,8 +327,6 @@ int build_table_from_flag(plb_ctx* c, const uint8_t* flag);
 int launch_step(plb_ctx* c, int64_t it, bool write_macros, const int64_t* it_base = nullptr);
 int launch_graph_steps(plb_ctx* c, int64_t it0, int64_t G);
 int launch_reduce(plb_ctx* c, double* host_out2);
-int exclusive_scan_u64(const uint64_t* in, uint64_t* out, int64_t n, hipStream_t s);
-int finalize_table(plb_ctx* c, int32_t* tabref, const uint64_t* xyz_ref);
 int build_ref_from_flag(const uint8_t* flag, int nx, int ny, int nz, int num_p, int mode,
                         hipStream_t s, int32_t** tabref_out, uint64_t** xyz_out, int64_t* n_out,
                         std::vector<int32_t>* start_out);
@@ -273,11 +352,11 @@ int launch_sample_sums(plb_ctx* c, const int32_t* d_active, int n_active, const 
                        double* d_partial, double* d_out);
 int check_cfg(const plb_config* cfg);
 int fp16_scale_log2_for(double gx);
-int compress_tile8(plb_ctx* c);
+int compress_tile8(plb_ctx* c, Arena* scratch);
 int build_key_runs(plb_ctx* c);
-int build_bitmap(plb_ctx* c);
 int compute_order(const plb_config& cfg, int nx, int ny, int nz, int64_t N, const uint64_t* xyz_ref,
-                  hipStream_t s, uint32_t** inv_perm, uint32_t** perm, uint64_t* xyz_int);
+                  hipStream_t s, uint32_t** inv_perm, uint32_t** perm, uint64_t* xyz_int, Arena* keep, Arena* scratch,
+                  const uint64_t* flag_bits);
 int permute_ref_table(const int32_t* tabref, int64_t n, const uint32_t* inv_perm, int32_t* out,
                       hipStream_t s);
 int ctx_begin(plb_ctx* c, const plb_config* cfg, int nx, int ny, int nz, int num_p);

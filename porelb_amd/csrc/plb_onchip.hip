@@ -70,7 +70,8 @@ struct OnchipPlan {
     void* recv = nullptr;
     size_t recv_bytes = 0;
     std::vector<OnchipSample> samples;
-    double* macros_alt = nullptr;
+    double* macros_own = nullptr;  // a second macros array; runs write the two by turns
+    double* macros_alt = nullptr;  // the one the next run writes
     uint32_t tag = 16;     // step number the next run starts with
     uint32_t serial = 0;   // of the last run
 };
@@ -722,8 +723,9 @@ void onchip_destroy(plb_ctx* c)
 {
     OnchipPlan* p = c->chip;
     if (!p) return;
-    for (void* q : {p->fixed, p->exchange, (void*)p->macros_alt})
-        if (q) (void)hipFree(q);
+    (void)hipStreamSynchronize(c->stream);
+    for (void* q : {p->fixed, p->exchange, (void*)p->macros_own})
+        if (q) dev_free(q);
     delete p;
     c->chip = nullptr;
 }
@@ -793,12 +795,13 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
     p->samples = samples;
     // arrays of the plan
     const int64_t slots = (int64_t)G * NS, groups = (int64_t)G * ng;
-    PLB_HIP(hipMalloc(&p->fixed, sizeof(uint32_t) * (slots * 10 + groups + 1 + G)));
+    PLB_HIP(dev_alloc(&p->fixed, sizeof(uint32_t) * (slots * 10 + groups + 1 + G)));
     p->node = (uint32_t*)p->fixed;
     p->idx = p->node + slots;
     p->seg = p->idx + 9 * slots;
     p->blk_sample = (int32_t*)(p->seg + groups + 1);
     // scratch of the build
+    Arena mem(s);
     DevBuf<char> scratch;
     size_t need = 0;
     auto part = [&](size_t bytes) {
@@ -809,7 +812,7 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
     const size_t o_smp = part(sizeof(OnchipSample) * samples.size()), o_bits = part(8 * (size_t)words), o_wpre = part(4 * (size_t)(words + 1)), o_order = part(4 * Ntot),
                  o_blk = part(2 * Ntot), o_slot = part(4 * Ntot), o_T = part(4 * 18 * Ntot), o_M = part(4 * 18 * Ntot),
                  o_cnt = part(4 * groups), o_err = part(4);
-    PLB_HIP(scratch.alloc((int64_t)need));
+    PLB_HIP(scratch.alloc((int64_t)need, &mem));
     char* const base = scratch.p;
     OnchipBuild b = {};
     b.samples = (const OnchipSample*)(base + o_smp);
@@ -872,7 +875,7 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
     if (E) {
         const size_t word = c->cfg.precision == PLB_FP16 ? 4 : c->cfg.precision == PLB_FP32 ? 8 : 16;
         const size_t lists = (8 * (size_t)E + 255) / 256 * 256;
-        PLB_HIP(hipMalloc(&p->exchange, lists + 2 * word * E));
+        PLB_HIP(dev_alloc(&p->exchange, lists + 2 * word * E));
         b.ent_lds = p->ent_lds = (uint32_t*)p->exchange;
         b.ent_dst = p->ent_dst = p->ent_lds + E;
         p->recv = (char*)p->exchange + lists;
@@ -884,7 +887,8 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
     if (E) hipLaunchKernelGGL(k_onchip_dst, dim3(nblk(E, 256)), t256, 0, s, b, (int64_t)E);
     PLB_HIP(hipGetLastError());
     if (!batch) {
-        PLB_HIP(hipMalloc(&p->macros_alt, sizeof(double) * 4 * c->Npad));
+        PLB_HIP(dev_alloc((void**)&p->macros_own, sizeof(double) * 4 * c->Npad));
+        p->macros_alt = p->macros_own;
         PLB_HIP(hipMemsetAsync(p->macros_alt, 0, sizeof(double) * 4 * c->Npad, s));
     }
     PLB_HIP(hipStreamSynchronize(s));  // the scratch goes back
@@ -1018,14 +1022,12 @@ void onchip_pack(const std::vector<int>& blocks, int cus, std::vector<std::vecto
     }
 }
 
-// Time of a step of a launch with blocks of up to NS nodes, in ns: fits of 64^3 to
-// 112^3 noise and sphere masks (FP32: 2.6 us at 512 nodes, 3.3 at 1024, 4.9 at
-// 1152 and 6.8 at 2048; FP64: 4.2 at 512, 6.1 at 1024).
+// Time of a step of a launch that fills the chip with blocks of up to NS nodes,
+// in ns: fits of 64^3 to 112^3 masks (FP32: 2.6 us at 320 nodes, 3.5 at 640,
+// 5.0 at 1152, 6.5 at 1664; FP64: 4.1 at 320, 6.7 at 640; FP16: 2.7, 3.5, 4.9, 6.5).
 static int64_t step_ns(const plb_ctx* c, int NS)
 {
-    if (c->cfg.precision == PLB_FP64) return NS <= 512 ? 3900 + NS / 2 : 3700 + NS * 9 / 4;
-    if (c->cfg.precision == PLB_FP32) return NS <= 1024 ? 2100 + NS * 8 / 7 : 2600 + NS * 2;
-    return NS <= 1024 ? 2500 + NS : 1500 + NS * 20 / 7;
+    return c->cfg.precision == PLB_FP64 ? 1600 + 8 * NS : 1650 + NS * 29 / 10;
 }
 
 bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::vector<int64_t>& n,

@@ -51,7 +51,7 @@ static void staging_free(Staging* s)
     if (!s) return;
     (void)hipSetDevice(s->device);
     if (s->host) (void)hipHostFree(s->host);
-    if (s->dev) (void)hipFree(s->dev);
+    dev_free(s->dev);
     for (hipEvent_t e : s->copied)
         if (e) (void)hipEventDestroy(e);
     delete s;
@@ -80,7 +80,7 @@ static hipError_t staging_new(int device, Staging** out)
     Staging* s = new Staging();
     s->device = device;
     hipError_t e = hipHostMalloc((void**)&s->host, SLOT * SLOTS, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipMalloc((void**)&s->dev, SLOT * SLOTS);
+    if (e == hipSuccess) e = dev_alloc((void**)&s->dev, SLOT * SLOTS);
     for (int k = 0; k < SLOTS && e == hipSuccess; k++) e = hipEventCreateWithFlags(&s->copied[k], hipEventDisableTiming);
     if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -249,12 +249,13 @@ static int move(int device, hipStream_t s, int64_t n, size_t item, const std::ve
     if (!threaded) {
         // One long copy per array and pass: the copy engine reaches its rate
         // from a few MB on.
+        Arena passes(s);
         DevBuf<char> big;
         char* room = st.dev;
         size_t have = SLOT * SLOTS;
         if (bytes > have) {
             const size_t want = std::min(bytes + 64 * row, LONG_PASS);
-            if (hipMalloc((void**)&big.p, want) == hipSuccess) {
+            if (big.alloc((int64_t)want, &passes) == hipSuccess) {
                 room = big.p;
                 have = want;
             } else {
