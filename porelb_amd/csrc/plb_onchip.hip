@@ -32,9 +32,15 @@
 // and loaded as one atomic (FP32: 8 bytes, FP64: two halves of 8 bytes, FP16: 4
 // bytes), and the receiver polls that word: no flag, no fence, one trip through
 // memory (0.9 us per round between 256 blocks, against 5.1 us for a grid barrier
-// with agent fences).  Blocks with more than 64 x T/64 slots send their
-// boundary nodes' values before they update the interior ones, so the trip
-// overlaps the update.
+// with agent fences).  Where a thread has two nodes, the block's shared nodes are
+// the first ones if they are no more than the threads, and their values leave
+// before the second ones are updated, so the trip overlaps that update.  The
+// entries of a wave are ordered by the wave at the other end, the same way on
+// both sides, so a row of 64 words leaves as a few stretches and not as 64
+// partial cache lines: 4.5 -> 4.0 us a step for 91 750 FP64 nodes, 4.9 -> 4.0 for
+// 265 421 FP32 ones, 3.2 -> 2.7 for 8 064 FP64 ones.  (Entry lists of a whole
+// block, dealt out to its waves: fewer pieces, but a second block barrier and
+// sends that wait for the slowest wave; 2.8, 4.7 and 4.6 us.)
 //
 // Ends.  Blocks wait for each other, so the launch is cooperative, and every
 // wait is bounded: a block that waits too long (50 ms for the first exchange,
@@ -80,6 +86,8 @@ constexpr uint32_t EMPTY = 0xffffffffu;
 // Cells behind the NS rows of F: the constants of directions 1..6 and 7..18,
 // and one that takes what is dropped on arrival.
 constexpr int EXTRA = 3, DROP = 2;
+// Directions come in pairs: 1, 2 | 3, 4 | ...
+__device__ __forceinline__ uint32_t opposite(uint32_t j) { return ((j - 1u) ^ 1u) + 1u; }
 
 // ---------------------------------------------------------------- plan
 __device__ __forceinline__ int64_t morton(uint64_t p, const OnchipSample& s)
@@ -107,7 +115,9 @@ struct OnchipBuild {
     uint16_t* blk;              // internal id -> block
     uint32_t* slot_of;          // internal id -> block * NS + slot
     int32_t* T;                 // [18][Ntot] pull sources
-    uint32_t* M;                // [18][Ntot] node that pulls population re[j]; later the shared link's entry
+    uint32_t* M;                // [18][Ntot] node that pulls population re[j]
+    uint32_t* at;               // [18][Ntot] the shared link's entry
+    const int32_t* block_sample;
     int* err;                   // the table is not that of a lattice (records that contradict each other)
     uint32_t* cnt;              // entries per group of 64 slots
     uint32_t *node, *idx, *seg, *ent_lds, *ent_dst;
@@ -239,11 +249,11 @@ __device__ __forceinline__ uint32_t partner(const OnchipBuild& b, int64_t k, int
 
 // Slot order of one block's nodes: key (no shared link, V id), sorted in LDS.
 constexpr int SORT_MAX = 4096;
-__global__ void __launch_bounds__(1024) k_onchip_slots(const OnchipBuild b, const int32_t* block_sample, int T)
+__global__ void __launch_bounds__(1024) k_onchip_slots(const OnchipBuild b, int T)
 {
     __shared__ uint32_t key[SORT_MAX];
     const int blk = blockIdx.x;
-    const OnchipSample s = b.samples[block_sample[blk]];
+    const OnchipSample s = b.samples[b.block_sample[blk]];
     const int64_t lb = blk - s.block0;
     const int64_t r0 = (lb * s.n + s.nblocks - 1) / s.nblocks, r1 = ((lb + 1) * s.n + s.nblocks - 1) / s.nblocks;
     const int n = (int)(r1 - r0);
@@ -311,19 +321,28 @@ __global__ void __launch_bounds__(1024) k_onchip_slots(const OnchipBuild b, cons
     }
 }
 
-// Entries of each group of 64 slots, in the order (direction, slot).
+// Entries of each group of 64 slots.  Their order is (block and group at the
+// other end, direction and slot as the end with the lower number has them), so
+// the links that two groups share have the same order in both lists: what a
+// wave sends as one row of 64 words goes to a few stretches of the receive
+// buffers.  (In the order (direction, slot) a row went to 18 pieces of 64 bytes
+// on average, in this one to 11, 8 being the least.)
 // FILL 0: counts them; 1: writes the entries and the index words.
+constexpr int GROUP_KEYS = 2048;   // 64 slots x 18 directions
 template <int FILL>
 __global__ void __launch_bounds__(256) k_onchip_groups(const OnchipBuild b)
 {
+    __shared__ uint32_t keys[FILL ? 4 : 1][FILL ? GROUP_KEYS : 1];
     const int lane = threadIdx.x & 63;
-    const int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int ng = b.NS / 64;
-    if (g >= (int64_t)b.G * ng) return;
-    const int blk = (int)(g / ng);
-    const uint32_t slot = (uint32_t)(g % ng) * 64 + lane;
-    const uint32_t k = b.node[g * 64 + lane];
-    uint32_t e = FILL ? b.seg[g] : 0u, lo = 0;
+    const uint32_t NS = (uint32_t)b.NS;
+    const int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), groups = (int64_t)b.G * ng;
+    const bool in = g < groups;
+    const int blk = in ? (int)(g / ng) : 0;
+    const uint32_t first = in ? (uint32_t)(g % ng) * 64 : 0u, slot = first + lane;
+    const uint32_t k = in ? b.node[g * 64 + lane] : EMPTY;
+    uint32_t* const key = keys[FILL ? threadIdx.x >> 6 : 0];
+    uint32_t n = 0, lo = 0;
 #pragma unroll
     for (int j = 1; j < Q; j++) {
         int32_t t = TAB_CONST;
@@ -331,35 +350,73 @@ __global__ void __launch_bounds__(256) k_onchip_groups(const OnchipBuild b)
         if (k != EMPTY) with = partner(b, k, j, (uint16_t)blk, t);
         const uint64_t m = __builtin_amdgcn_ballot_w64(with != EMPTY);
         if constexpr (FILL) {
-            const uint32_t own = slot * Q + RE[j];
             const bool in_block = t >= 0 && b.blk[t] == (uint16_t)blk;
-            uint32_t pos = own;
-            if (in_block) pos = b.slot_of[t] % (uint32_t)b.NS * Q + j;
-            else if (t == TAB_CONST) pos = (uint32_t)b.NS * Q + (j > 6 ? 1u : 0u);
+            uint32_t pos = slot * Q + RE[j];
+            if (in_block) pos = b.slot_of[t] % NS * Q + j;
+            else if (t == TAB_CONST) pos = NS * Q + (j > 6 ? 1u : 0u);
             if (k == EMPTY) pos = 0;
             // words 0..8 hold directions 1, 2 | 3, 4 | ... | 17, 18
             if (j & 1) lo = pos;
-            else b.idx[((int64_t)blk * 9 + (j / 2 - 1)) * b.NS + slot] = lo | (pos << 16);
+            else if (in) b.idx[((int64_t)blk * 9 + (j / 2 - 1)) * NS + slot] = lo | (pos << 16);
             if (with != EMPTY) {
-                const uint32_t at = e + __popcll(m & ((1ull << lane) - 1ull));
-                const uint32_t to = t >= 0 && !in_block ? own : (uint32_t)b.NS * Q + DROP;
-                b.ent_lds[at] = own | (to << 16);
-                b.ent_dst[at] = with;                      // the partner node until k_onchip_dst
-                b.M[(int64_t)(j - 1) * b.Ntot + k] = at;   // read by this lane only, above
+                const int other = b.blk[with];
+                const uint32_t there = b.slot_of[with] % NS;
+                const uint32_t block0 = (uint32_t)b.samples[b.block_sample[blk]].block0;
+                const uint32_t dir = blk < other ? (uint32_t)j : (uint32_t)RE[j];
+                const uint32_t at = blk < other ? slot : there;
+                key[n + __popcll(m & ((1ull << lane) - 1ull))] =
+                    ((uint32_t)other - block0) << 16 | (there >> 6) << 11 | dir << 6 | (at & 63u);
             }
         }
-        e += (uint32_t)__popcll(m);
+        n += (uint32_t)__popcll(m);
     }
-    // Whole rows of 64, so that the exchange needs no lane masks: the rest are
-    // entries a block sends to itself and drops.
-    if constexpr (FILL) {
-        if (e + lane < b.seg[g + 1]) {
-            const uint32_t drop = (uint32_t)b.NS * Q + DROP;
-            b.ent_lds[e + lane] = drop | (drop << 16);
-            b.ent_dst[e + lane] = e + lane;
-        }
+    if constexpr (FILL == 0) {
+        // Whole rows of 64, so that the exchange needs no lane masks: the rest
+        // are entries a block sends to itself and drops.
+        if (in && lane == 0) b.cnt[g] = (n + 63u) & ~63u;
     } else {
-        if (lane == 0) b.cnt[g] = (e + 63u) & ~63u;
+        uint32_t P = 64;
+        while (P < n) P <<= 1;
+        for (uint32_t q = n + lane; q < P; q += 64) key[q] = EMPTY;
+        // one wave sorts its own keys: LDS operations of a wave stay in order
+        auto fence = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+        fence();
+        for (uint32_t size = 2; n && size <= P; size <<= 1)
+            for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+                for (uint32_t q = lane; q < P / 2; q += 64) {
+                    const uint32_t a = 2 * q - (q & (stride - 1)), c = a + stride;
+                    const uint32_t x = key[a], y = key[c];
+                    if ((x > y) == ((a & size) == 0)) {
+                        key[a] = y;
+                        key[c] = x;
+                    }
+                }
+                fence();
+            }
+        if (!in) return;
+        const uint32_t e0 = b.seg[g], e1 = b.seg[g + 1];
+        const int block0 = b.samples[b.block_sample[blk]].block0;
+        for (uint32_t q = lane; e0 + q < e1; q += 64) {
+            const uint32_t e = e0 + q;
+            if (q >= n) {
+                b.ent_lds[e] = (NS * Q + DROP) * 0x10001u;
+                b.ent_dst[e] = e;
+                continue;
+            }
+            const int other = block0 + (int)(key[q] >> 16);
+            uint32_t j = (key[q] >> 6) & 31u, mine = first + (key[q] & 63u);
+            int32_t t;
+            if (other < blk) {   // the key has the other end's direction and slot
+                const uint32_t far = ((key[q] >> 11) & 31u) * 64 + (key[q] & 63u);
+                mine = b.slot_of[partner(b, b.node[(int64_t)other * NS + far], (int)j, (uint16_t)other, t)] % NS;
+                j = opposite(j);
+            }
+            const uint32_t me = b.node[(int64_t)blk * NS + mine], own = mine * Q + opposite(j);
+            const uint32_t with = partner(b, me, (int)j, (uint16_t)blk, t);
+            b.ent_lds[e] = own | (t >= 0 ? own : NS * Q + DROP) << 16;
+            b.ent_dst[e] = with;                            // the partner node until k_onchip_dst
+            b.at[(int64_t)(j - 1) * b.Ntot + me] = e;
+        }
     }
 }
 
@@ -370,7 +427,7 @@ __global__ void k_onchip_dst(const OnchipBuild b, int64_t E)
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= E) return;
     const uint32_t cell = b.ent_lds[e] & 0xffffu;
-    if (cell < (uint32_t)b.NS * Q) b.ent_dst[e] = b.M[(int64_t)(cell % Q - 1) * b.Ntot + b.ent_dst[e]];
+    if (cell < (uint32_t)b.NS * Q) b.ent_dst[e] = b.at[(int64_t)(cell % Q - 1) * b.Ntot + b.ent_dst[e]];
 }
 
 // ---------------------------------------------------------------- exchange words
@@ -810,7 +867,7 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
         return at;
     };
     const size_t o_smp = part(sizeof(OnchipSample) * samples.size()), o_bits = part(8 * (size_t)words), o_wpre = part(4 * (size_t)(words + 1)), o_order = part(4 * Ntot),
-                 o_blk = part(2 * Ntot), o_slot = part(4 * Ntot), o_T = part(4 * 18 * Ntot), o_M = part(4 * 18 * Ntot),
+                 o_blk = part(2 * Ntot), o_slot = part(4 * Ntot), o_T = part(4 * 18 * Ntot), o_M = part(4 * 18 * Ntot), o_at = part(4 * 18 * Ntot),
                  o_cnt = part(4 * groups), o_err = part(4);
     PLB_HIP(scratch.alloc((int64_t)need, &mem));
     char* const base = scratch.p;
@@ -830,6 +887,8 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
     b.slot_of = (uint32_t*)(base + o_slot);
     b.T = (int32_t*)(base + o_T);
     b.M = (uint32_t*)(base + o_M);
+    b.at = (uint32_t*)(base + o_at);
+    b.block_sample = p->blk_sample;
     b.cnt = (uint32_t*)(base + o_cnt);
     b.err = (int*)(base + o_err);
     b.node = p->node;
@@ -861,7 +920,7 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
         else PLB_LINKS(PLB_LAYOUT_AOSOA, PLB_INDEX_I32);
     }
 #undef PLB_LINKS
-    hipLaunchKernelGGL(k_onchip_slots, dim3(G), dim3(std::min(1024, NS)), 0, s, b, p->blk_sample, p->T);
+    hipLaunchKernelGGL(k_onchip_slots, dim3(G), dim3(std::min(1024, NS)), 0, s, b, p->T);
     hipLaunchKernelGGL(k_onchip_groups<0>, dim3(nblk(groups, 4)), t256, 0, s, b);
     hipLaunchKernelGGL(k_onchip_segs, dim3(1), dim3(1024), 0, s, b, groups);
     PLB_HIP(hipGetLastError());
