@@ -266,6 +266,16 @@ __device__ __forceinline__ int64_t out_pos(const StepArgs& a, int64_t i, const i
     }
 }
 
+// Stores of the step kernels: non-temporal, or plain where the next step finds
+// the populations in the memory-side cache (KEEP).
+template <bool KEEP, typename S>
+__device__ __forceinline__ void st_dev(S* p, S v)
+{
+    if constexpr (KEEP) *p = v;
+    else if constexpr (sizeof(S) == 2) __builtin_nontemporal_store(__half_as_ushort(v), (unsigned short*)p);
+    else __builtin_nontemporal_store(v, p);
+}
+
 // FP64 collision in the reference's evaluation order (porelb.c:326-362) on
 // the streamed populations f of node i; put(j, value) takes the results.
 template <typename Put>
@@ -300,7 +310,7 @@ __device__ __forceinline__ void relax_f64(const StepArgs& a, int64_t i, const do
     }
 }
 
-template <int LAYOUT, int MODE = 0>
+template <int LAYOUT, int MODE = 0, bool KEEP = false>
 __device__ __forceinline__ void collide_f64(const StepArgs& a, int64_t i, const int32_t t[Q],
                                             double f[Q], unsigned long long fk)
 {
@@ -311,7 +321,7 @@ __device__ __forceinline__ void collide_f64(const StepArgs& a, int64_t i, const 
             if (t[j] == TAB_CONST) f[j] = TP[j] * a.rho0 * 1.0;  // feq(rho0, u=0) = initial f1
     }
     relax_f64(a, i, f, fk, [&](int j, double o) {
-        __builtin_nontemporal_store(o, fout + out_pos<LAYOUT, MODE>(a, i, t, j));
+        st_dev<KEEP>(fout + out_pos<LAYOUT, MODE>(a, i, t, j), o);
     });
 }
 
@@ -329,11 +339,6 @@ __device__ __forceinline__ S to_stored(float v)
 {
     if constexpr (sizeof(S) == 2) return __float2half_rn(v);
     else return v;
-}
-__device__ __forceinline__ void st_dev(float* p, float v) { __builtin_nontemporal_store(v, p); }
-__device__ __forceinline__ void st_dev(__half* p, __half v)
-{
-    __builtin_nontemporal_store(__half_as_ushort(v), (unsigned short*)p);
 }
 
 // Stochastic rounding of FP16 stores.  v_cvt_sr_f16_f32 rounds up with
@@ -446,7 +451,7 @@ __device__ __forceinline__ void relax_shift(const StepArgs& a, int64_t i, const 
     }
 }
 
-template <typename S, int LAYOUT, int MODE = 0>
+template <typename S, int LAYOUT, int MODE = 0, bool KEEP = false>
 __device__ __forceinline__ void collide_shift(const StepArgs& a, int64_t i, const int32_t t[Q],
                                               const S raw[Q], unsigned long long fk, uint32_t key)
 {
@@ -463,8 +468,8 @@ __device__ __forceinline__ void collide_shift(const StepArgs& a, int64_t i, cons
     }
     S* __restrict__ onode = fout + fpos<LAYOUT>(0, i, a.Npad);
     relax_shift<S>(a, i, ds, fk, key, [&](int j, S v) {
-        if constexpr (MODE == 0) st_dev(onode + fpos<LAYOUT>(j, 0, a.Npad), v);
-        else st_dev(fout + out_pos<LAYOUT, MODE>(a, i, t, j), v);
+        if constexpr (MODE == 0) st_dev<KEEP>(onode + fpos<LAYOUT>(j, 0, a.Npad), v);
+        else st_dev<KEEP>(fout + out_pos<LAYOUT, MODE>(a, i, t, j), v);
     });
 }
 
@@ -490,17 +495,17 @@ __device__ __forceinline__ uint32_t sr_key(const StepArgs& a, int64_t i)
     return (uint32_t)i;
 }
 
-template <typename S, int LAYOUT, int MODE = 0>
+template <typename S, int LAYOUT, int MODE = 0, bool KEEP = false>
 __device__ __forceinline__ void collide_any(const StepArgs& a, int64_t i, const int32_t t[Q], S raw[Q],
                                             unsigned long long fk, uint32_t key)
 {
     if constexpr (sizeof(S) == 8)
-        collide_f64<LAYOUT, MODE>(a, i, t, (double*)raw, fk);
+        collide_f64<LAYOUT, MODE, KEEP>(a, i, t, (double*)raw, fk);
     else
-        collide_shift<S, LAYOUT, MODE>(a, i, t, raw, fk, key);
+        collide_shift<S, LAYOUT, MODE, KEEP>(a, i, t, raw, fk, key);
 }
 
-template <typename S, int LAYOUT, int IDX, bool CONST_DESC = false>
+template <typename S, int LAYOUT, int IDX, bool CONST_DESC = false, bool KEEP = false>
 __device__ __forceinline__ void node_any(const StepArgs& a, int64_t i, unsigned long long fk)
 {
     Entries<IDX> e;
@@ -509,7 +514,7 @@ __device__ __forceinline__ void node_any(const StepArgs& a, int64_t i, unsigned 
     S raw[Q];
     gather<S, LAYOUT>(a, i, e.t, raw);
     const uint32_t key = sr_key<S>(a, i);
-    collide_any<S, LAYOUT>(a, i, e.t, raw, fk, key);
+    collide_any<S, LAYOUT, 0, KEEP>(a, i, e.t, raw, fk, key);
 }
 
 // Pull sources t[1..18] of internal node k, decoded by one lane on its own

@@ -37,6 +37,25 @@ __global__ void __launch_bounds__(1024) k_step(const StepArgs a)
     node_any<S, LAYOUT, IDX>(with_step(a), i, *a.fault);
 }
 
+// The same with plain stores, for FP64 and FP32 lattices whose two buffers and
+// index fit the 256 MB memory-side cache but not the L2s (8 x 4 MB): non-temporal
+// stores go past that cache, and the next step then reads from HBM what this one
+// wrote.  us a step, plain against non-temporal: FP64 7.1 / 6.5 at 78 643 nodes
+// (25 MB), 11.1 / 13.2 at 153 600 (50 MB), 17.2 / 19.5 at 265 421 (86 MB), 36.9 /
+// 40.3 at 629 146 (204 MB), 77.8 / 74.6 at 1 228 800 (398 MB); FP32 6.9 / 6.8 at
+// 153 600 (26 MB), 10.8 / 11.9 at 265 421 (46 MB), 21.5 / 22.5 at 629 146 (108 MB),
+// 40.2 / 41.2 at 1 228 800 (211 MB), 71.8 / 68.8 at 2 123 366 (365 MB).  FP16
+// (bound by L2 requests) gains at no size.
+template <typename S, int LAYOUT, int IDX>
+__global__ void __launch_bounds__(1024) k_step_keep(const StepArgs a)
+{
+    const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t i = blk * blockDim.x + threadIdx.x;
+    if (i >= a.N) return;
+    node_any<S, LAYOUT, IDX, false, true>(with_step(a), i, *a.fault);
+}
+constexpr double KEEP_ABOVE = 32e6, KEEP_MOST = 256e6;
+
 // Single lattice, one buffer, AA pattern (half-way bounce-back).  The
 // buffer alternates between two forms of the post-collision populations
 // f*_j(y) of the last step: after a neighbour step (and at rest), f*_j(y)
@@ -781,6 +800,28 @@ static unsigned step_lds_bytes(const plb_ctx* c, int bs)
     return (unsigned)(share / 512 * 512);
 }
 
+static bool keep_stores(const plb_ctx* c)
+{
+    const double bytes = (2.0 * Q * c->elem + c->index_bytes) * (double)c->N;
+    return c->cfg.precision != PLB_FP16 && bytes > KEEP_ABOVE && bytes <= KEEP_MOST;
+}
+
+static void launch_keep(const plb_ctx* c, const StepArgs& a, dim3 grid, dim3 block, unsigned lds)
+{
+    auto run = [&](auto* kern) { hipLaunchKernelGGL(kern, grid, block, lds, c->stream, a); };
+    auto with = [&](auto layout, auto idx) {
+        constexpr int L = decltype(layout)::value, I = decltype(idx)::value;
+        c->cfg.precision == PLB_FP64 ? run(k_step_keep<double, L, I>) : run(k_step_keep<float, L, I>);
+    };
+    auto with_idx = [&](auto layout) {
+        if (c->cfg.index_kind == PLB_INDEX_I32) with(layout, std::integral_constant<int, PLB_INDEX_I32>{});
+        else if (c->cfg.index_kind == PLB_INDEX_TILE8) with(layout, std::integral_constant<int, PLB_INDEX_TILE8>{});
+        else with(layout, std::integral_constant<int, PLB_INDEX_BITMAP>{});
+    };
+    if (c->cfg.layout == PLB_LAYOUT_SOA) with_idx(std::integral_constant<int, PLB_LAYOUT_SOA>{});
+    else with_idx(std::integral_constant<int, PLB_LAYOUT_AOSOA>{});
+}
+
 int launch_step(plb_ctx* c, int64_t it, bool write_macros, const int64_t* it_base)
 {
     if (c->N == 0) {  // a mask without pores: nothing to update
@@ -804,6 +845,8 @@ int launch_step(plb_ctx* c, int64_t it, bool write_macros, const int64_t* it_bas
         const int64_t threads = (c->N + 127) / 128 * 64;
         PLB_DISPATCH3(c->cfg.precision, c->cfg.layout, c->cfg.index_kind, k_step2,
                       dim3(nblk(threads, bs)), dim3(bs), lds, c->stream, a);
+    } else if (keep_stores(c)) {
+        launch_keep(c, a, dim3(nblk(c->N, bs)), dim3(bs), lds);
     } else {
         PLB_DISPATCH3(c->cfg.precision, c->cfg.layout, c->cfg.index_kind, k_step, dim3(nblk(c->N, bs)),
                       dim3(bs), lds, c->stream, a);
