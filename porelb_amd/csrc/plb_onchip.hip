@@ -1181,11 +1181,15 @@ void onchip_pack(const std::vector<int>& blocks, int cus, std::vector<std::vecto
 }
 
 // Time of a step of a launch that fills the chip with blocks of up to NS nodes,
-// in ns: fits of 64^3 to 112^3 masks (FP32: 2.6 us at 320 nodes, 3.5 at 640,
-// 5.0 at 1152, 6.5 at 1664; FP64: 4.1 at 320, 6.7 at 640; FP16: 2.7, 3.5, 4.9, 6.5).
+// in ns: fits of 64^3 to 119^3 noise masks and sphere packs (FP32: 2.2 us at 359
+// nodes, 3.8 to 4.2 at 1152, 4.9 to 5.5 at 1664, 5.5 to 5.9 at 1975; FP64: 3.6 at 359,
+// 5.2 at 600, 6.3 at 1005; FP16: 4.2 to 4.8 at 1152, 6.2 to 7.3 at 2000).  Above 1024
+// nodes a thread has two.
 static int64_t step_ns(const plb_ctx* c, int NS)
 {
-    return c->cfg.precision == PLB_FP64 ? 1600 + 8 * NS : 1650 + NS * 29 / 10;
+    if (c->cfg.precision == PLB_FP64) return 2600 + NS * 37 / 10;
+    if (NS <= 1024) return 1900 + NS * 6 / 5;
+    return c->cfg.precision == PLB_FP32 ? 1900 + NS * 37 / 20 : 1000 + NS * 14 / 5;
 }
 
 bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::vector<int64_t>& n,
