@@ -266,14 +266,20 @@ __device__ __forceinline__ int64_t out_pos(const StepArgs& a, int64_t i, const i
     }
 }
 
-// Stores of the step kernels: non-temporal, or plain where the next step finds
-// the populations in the memory-side cache (KEEP).
+// Stores of the step kernels: non-temporal, or (KEEP, and `keep` of the wave)
+// plain, where the next step is to find them in the memory-side cache.
 template <bool KEEP, typename S>
-__device__ __forceinline__ void st_dev(S* p, S v)
+__device__ __forceinline__ void st_dev(S* p, S v, bool keep)
 {
-    if constexpr (KEEP) *p = v;
-    else if constexpr (sizeof(S) == 2) __builtin_nontemporal_store(__half_as_ushort(v), (unsigned short*)p);
-    else __builtin_nontemporal_store(v, p);
+    if (KEEP && keep) {
+        asm volatile("");   // or the compiler makes one plain store of the two
+        *p = v;
+        asm volatile("");
+    } else if constexpr (sizeof(S) == 2) {
+        __builtin_nontemporal_store(__half_as_ushort(v), (unsigned short*)p);
+    } else {
+        __builtin_nontemporal_store(v, p);
+    }
 }
 
 // FP64 collision in the reference's evaluation order (porelb.c:326-362) on
@@ -312,7 +318,7 @@ __device__ __forceinline__ void relax_f64(const StepArgs& a, int64_t i, const do
 
 template <int LAYOUT, int MODE = 0, bool KEEP = false>
 __device__ __forceinline__ void collide_f64(const StepArgs& a, int64_t i, const int32_t t[Q],
-                                            double f[Q], unsigned long long fk)
+                                            double f[Q], unsigned long long fk, bool keep)
 {
     double* __restrict__ fout = (double*)a.fout;
     if constexpr (MODE == 0) {  // constant entries: reference bounce order, two buffers only
@@ -321,7 +327,7 @@ __device__ __forceinline__ void collide_f64(const StepArgs& a, int64_t i, const 
             if (t[j] == TAB_CONST) f[j] = TP[j] * a.rho0 * 1.0;  // feq(rho0, u=0) = initial f1
     }
     relax_f64(a, i, f, fk, [&](int j, double o) {
-        st_dev<KEEP>(fout + out_pos<LAYOUT, MODE>(a, i, t, j), o);
+        st_dev<KEEP>(fout + out_pos<LAYOUT, MODE>(a, i, t, j), o, keep);
     });
 }
 
@@ -453,7 +459,7 @@ __device__ __forceinline__ void relax_shift(const StepArgs& a, int64_t i, const 
 
 template <typename S, int LAYOUT, int MODE = 0, bool KEEP = false>
 __device__ __forceinline__ void collide_shift(const StepArgs& a, int64_t i, const int32_t t[Q],
-                                              const S raw[Q], unsigned long long fk, uint32_t key)
+                                              const S raw[Q], unsigned long long fk, uint32_t key, bool keep)
 {
     S* __restrict__ fout = (S*)a.fout;
     float ds[Q];
@@ -468,8 +474,8 @@ __device__ __forceinline__ void collide_shift(const StepArgs& a, int64_t i, cons
     }
     S* __restrict__ onode = fout + fpos<LAYOUT>(0, i, a.Npad);
     relax_shift<S>(a, i, ds, fk, key, [&](int j, S v) {
-        if constexpr (MODE == 0) st_dev<KEEP>(onode + fpos<LAYOUT>(j, 0, a.Npad), v);
-        else st_dev<KEEP>(fout + out_pos<LAYOUT, MODE>(a, i, t, j), v);
+        if constexpr (MODE == 0) st_dev<KEEP>(onode + fpos<LAYOUT>(j, 0, a.Npad), v, keep);
+        else st_dev<KEEP>(fout + out_pos<LAYOUT, MODE>(a, i, t, j), v, keep);
     });
 }
 
@@ -497,16 +503,16 @@ __device__ __forceinline__ uint32_t sr_key(const StepArgs& a, int64_t i)
 
 template <typename S, int LAYOUT, int MODE = 0, bool KEEP = false>
 __device__ __forceinline__ void collide_any(const StepArgs& a, int64_t i, const int32_t t[Q], S raw[Q],
-                                            unsigned long long fk, uint32_t key)
+                                            unsigned long long fk, uint32_t key, bool keep = false)
 {
     if constexpr (sizeof(S) == 8)
-        collide_f64<LAYOUT, MODE, KEEP>(a, i, t, (double*)raw, fk);
+        collide_f64<LAYOUT, MODE, KEEP>(a, i, t, (double*)raw, fk, keep);
     else
-        collide_shift<S, LAYOUT, MODE, KEEP>(a, i, t, raw, fk, key);
+        collide_shift<S, LAYOUT, MODE, KEEP>(a, i, t, raw, fk, key, keep);
 }
 
 template <typename S, int LAYOUT, int IDX, bool CONST_DESC = false, bool KEEP = false>
-__device__ __forceinline__ void node_any(const StepArgs& a, int64_t i, unsigned long long fk)
+__device__ __forceinline__ void node_any(const StepArgs& a, int64_t i, unsigned long long fk, bool keep = false)
 {
     Entries<IDX> e;
     issue_entries<LAYOUT, IDX, CONST_DESC>(a, i, e);
@@ -514,7 +520,7 @@ __device__ __forceinline__ void node_any(const StepArgs& a, int64_t i, unsigned 
     S raw[Q];
     gather<S, LAYOUT>(a, i, e.t, raw);
     const uint32_t key = sr_key<S>(a, i);
-    collide_any<S, LAYOUT, 0, KEEP>(a, i, e.t, raw, fk, key);
+    collide_any<S, LAYOUT, 0, KEEP>(a, i, e.t, raw, fk, key, keep);
 }
 
 // Pull sources t[1..18] of internal node k, decoded by one lane on its own

@@ -37,24 +37,28 @@ __global__ void __launch_bounds__(1024) k_step(const StepArgs a)
     node_any<S, LAYOUT, IDX>(with_step(a), i, *a.fault);
 }
 
-// The same with plain stores, for FP64 and FP32 lattices whose two buffers and
-// index fit the 256 MB memory-side cache but not the L2s (8 x 4 MB): non-temporal
-// stores go past that cache, and the next step then reads from HBM what this one
-// wrote.  us a step, plain against non-temporal: FP64 7.1 / 6.5 at 78 643 nodes
-// (25 MB), 11.1 / 13.2 at 153 600 (50 MB), 17.2 / 19.5 at 265 421 (86 MB), 36.9 /
-// 40.3 at 629 146 (204 MB), 77.8 / 74.6 at 1 228 800 (398 MB); FP32 6.9 / 6.8 at
-// 153 600 (26 MB), 10.8 / 11.9 at 265 421 (46 MB), 21.5 / 22.5 at 629 146 (108 MB),
-// 40.2 / 41.2 at 1 228 800 (211 MB), 71.8 / 68.8 at 2 123 366 (365 MB).  FP16
-// (bound by L2 requests) gains at no size.
+// The same with plain stores for `keep` of 16 groups of 16 blocks, for FP64 and
+// FP32 lattices that do not fit the L2s (8 x 4 MB) but whose two buffers and index
+// fit the 256 MB memory-side cache, all or in part: non-temporal stores go past
+// that cache, and the next step then reads from HBM what this one wrote.  Of a
+// lattice beyond 208 MB, the share that takes KEEP_BYTES is kept; the rest passes
+// by.  (Keeping everything there pushes out what is still to be read.)  us a step
+// against non-temporal stores alone: FP64 14.8 / 16.1 at 204 442 nodes (66 MB), 37.5 /
+// 40.5 at 629 146 (204 MB), 47.6 / 52.3 at 823 200 (267 MB), 60.5 / 65.0 at 1 053 542
+// (341 MB), 95.2 / 99.3 at 1 635 533 (530 MB); FP32 15.7 / 16.6 at 421 478 (72 MB),
+// 39.2 / 41.7 at 1 228 800 (211 MB), 64.5 / 69.7 at 2 123 366 (365 MB), 99.3 / 103.8 at
+// 3 194 400 (549 MB), 138.8 / 138.7 at 4 251 746 (731 MB).  Below 32 MB plain stores
+// lose (FP64 7.1 / 6.5 at 78 643 nodes), and FP16, bound by L2 requests, gains at no
+// size.
 template <typename S, int LAYOUT, int IDX>
-__global__ void __launch_bounds__(1024) k_step_keep(const StepArgs a)
+__global__ void __launch_bounds__(1024) k_step_keep(const StepArgs a, int keep)
 {
     const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
     const int64_t i = blk * blockDim.x + threadIdx.x;
     if (i >= a.N) return;
-    node_any<S, LAYOUT, IDX, false, true>(with_step(a), i, *a.fault);
+    node_any<S, LAYOUT, IDX, false, true>(with_step(a), i, *a.fault, (int)((blk >> 4) & 15) < keep);
 }
-constexpr double KEEP_ABOVE = 32e6, KEEP_MOST = 256e6;
+constexpr double KEEP_ABOVE = 32e6, KEEP_ALL = 208e6, KEEP_MOST = 600e6, KEEP_BYTES = 115e6;
 
 // Single lattice, one buffer, AA pattern (half-way bounce-back).  The
 // buffer alternates between two forms of the post-collision populations
@@ -800,15 +804,17 @@ static unsigned step_lds_bytes(const plb_ctx* c, int bs)
     return (unsigned)(share / 512 * 512);
 }
 
-static bool keep_stores(const plb_ctx* c)
+// Groups of 16 whose stores are plain; 0: k_step.
+static int keep_stores(const plb_ctx* c)
 {
     const double bytes = (2.0 * Q * c->elem + c->index_bytes) * (double)c->N;
-    return c->cfg.precision != PLB_FP16 && bytes > KEEP_ABOVE && bytes <= KEEP_MOST;
+    if (c->cfg.precision == PLB_FP16 || bytes <= KEEP_ABOVE || bytes > KEEP_MOST) return 0;
+    return bytes <= KEEP_ALL ? 16 : (int)(16.0 * KEEP_BYTES / bytes + 0.5);
 }
 
-static void launch_keep(const plb_ctx* c, const StepArgs& a, dim3 grid, dim3 block, unsigned lds)
+static void launch_keep(const plb_ctx* c, const StepArgs& a, int keep, dim3 grid, dim3 block, unsigned lds)
 {
-    auto run = [&](auto* kern) { hipLaunchKernelGGL(kern, grid, block, lds, c->stream, a); };
+    auto run = [&](auto* kern) { hipLaunchKernelGGL(kern, grid, block, lds, c->stream, a, keep); };
     auto with = [&](auto layout, auto idx) {
         constexpr int L = decltype(layout)::value, I = decltype(idx)::value;
         c->cfg.precision == PLB_FP64 ? run(k_step_keep<double, L, I>) : run(k_step_keep<float, L, I>);
@@ -845,8 +851,8 @@ int launch_step(plb_ctx* c, int64_t it, bool write_macros, const int64_t* it_bas
         const int64_t threads = (c->N + 127) / 128 * 64;
         PLB_DISPATCH3(c->cfg.precision, c->cfg.layout, c->cfg.index_kind, k_step2,
                       dim3(nblk(threads, bs)), dim3(bs), lds, c->stream, a);
-    } else if (keep_stores(c)) {
-        launch_keep(c, a, dim3(nblk(c->N, bs)), dim3(bs), lds);
+    } else if (const int keep = keep_stores(c)) {
+        launch_keep(c, a, keep, dim3(nblk(c->N, bs)), dim3(bs), lds);
     } else {
         PLB_DISPATCH3(c->cfg.precision, c->cfg.layout, c->cfg.index_kind, k_step, dim3(nblk(c->N, bs)),
                       dim3(bs), lds, c->stream, a);

@@ -1,6 +1,6 @@
 """Step kernels with plain and with non-temporal stores compute the same: lattices on both sides of the sizes
-(32 and 256 MB of populations and index) between which plain stores are used, against the two-nodes-per-thread
-kernel, which has non-temporal ones."""
+(32, 208 and 600 MB of populations and index) between which all or some blocks store plainly, against the
+two-nodes-per-thread kernel, which has non-temporal stores."""
 import numpy as np
 import pytest
 
@@ -12,14 +12,14 @@ pytestmark = pytest.mark.gpu
 # pore nodes x (2 x 19 x element + index bytes): FP64 with an int32 table 376 bytes a node, FP32 224
 @pytest.mark.parametrize("layout", [P.LAYOUT_SOA, P.LAYOUT_AOSOA])
 @pytest.mark.parametrize("precision,bb,nodes", [
-    (P.FP64, P.BB_REFCOMPAT, 85_000), (P.FP64, P.BB_REFCOMPAT, 85_207), (P.FP64, P.BB_HALFWAY, 680_000),
-    (P.FP64, P.BB_HALFWAY, 681_001), (P.FP32, P.BB_HALFWAY, 142_000), (P.FP32, P.BB_REFCOMPAT, 142_931),
-    (P.FP32, P.BB_HALFWAY, 300_001)])
+    (P.FP64, P.BB_REFCOMPAT, 85_000), (P.FP64, P.BB_REFCOMPAT, 85_207), (P.FP64, P.BB_HALFWAY, 553_100),
+    (P.FP64, P.BB_HALFWAY, 553_299), (P.FP64, P.BB_HALFWAY, 1_595_700), (P.FP64, P.BB_HALFWAY, 1_595_800),
+    (P.FP32, P.BB_HALFWAY, 142_000), (P.FP32, P.BB_REFCOMPAT, 142_931), (P.FP32, P.BB_HALFWAY, 1_200_001)])
 def test_same_as_two_nodes_per_thread(precision, bb, nodes, layout):
     rng = np.random.default_rng(nodes)
-    flag = np.zeros(100 * 101 * 99, np.uint8)
+    flag = np.zeros(120 * 121 * 119, np.uint8)
     flag[rng.permutation(flag.size)[:nodes]] = 1
-    flag = flag.reshape(99, 101, 100)
+    flag = flag.reshape(119, 121, 120)
     out = []
     for per_thread in (1, 2):
         with P.Lattice.from_flag(flag, 1, tau=0.8, gx=1e-5, precision=precision, bb_mode=bb, layout=layout,
