@@ -46,6 +46,7 @@ struct plb_batch {
     double* d_gx = nullptr;
     double* d_sums = nullptr;
     double* d_partial = nullptr;  // per-chunk u_x partial sums
+    double* sums = nullptr;       // [S][2] of plb_batch_reduce, page-locked
 };
 
 extern "C" void plb_batch_destroy(plb_batch* b)
@@ -59,6 +60,7 @@ extern "C" void plb_batch_destroy(plb_batch* b)
                     b->d_omega, b->d_gx, b->d_sums, b->d_partial};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    if (b->sums) (void)hipHostFree(b->sums);
     plb_destroy(b->c);
     delete b;
 }
@@ -597,12 +599,16 @@ extern "C" int plb_batch_reduce(plb_batch* b, plb_reduction* out)
     PLB_HIP(hipSetDevice(c->device));
     double wsum = 0.0;
     for (int j = 0; j < Q; j++) wsum += TP[j] * c->cfg.rho0;
+    // one wait for all samples
+    if (!b->sums) PLB_HIP(hipHostMalloc((void**)&b->sums, sizeof(double) * 2 * (size_t)b->S, hipHostMallocDefault));
     for (int s = 0; s < b->S; s++) {
-        double r[2] = {0.0, 0.0};
-        if (b->n[s] > 0) {
-            int rc = launch_reduce_range(c, b->sample_cur[s], b->off[s], b->n[s], true, r);
-            if (rc) return rc;
-        }
+        if (b->n[s] == 0) continue;
+        const int rc = launch_reduce_range(c, b->sample_cur[s], b->off[s], b->n[s], b->sums + 2 * s, nullptr);
+        if (rc) return rc;
+    }
+    PLB_HIP(hipStreamSynchronize(c->stream));
+    for (int s = 0; s < b->S; s++) {
+        const double r[2] = {b->n[s] ? b->sums[2 * s] : 0.0, b->n[s] ? b->sums[2 * s + 1] : 0.0};
         plb_reduction& o = out[s];
         o.mass = r[0] + (c->cfg.precision != PLB_FP64 ? wsum * (double)b->n[s] : 0.0);
         o.sum_ux = r[1];

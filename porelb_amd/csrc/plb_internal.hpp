@@ -213,6 +213,12 @@ struct Segment {
     uint32_t serial;     // on-chip run: its serial number; 0: one launch per step
     double* macros;      // macros array before it
 };
+
+// What the host waits for between calls.
+struct HostWords {
+    unsigned long long fault[2];
+    double sum[2];
+};
 }  // namespace plb
 
 struct plb_ctx {
@@ -254,7 +260,7 @@ struct plb_ctx {
     double* macros = nullptr;   // [4][Npad]
     void* reserve = nullptr;    // placement reserve (cfg.placement_reserve_gib)
     unsigned long long* fault = nullptr;  // [0] density-guard key, [1] serial of an on-chip run that gave up
-    unsigned long long* host_words = nullptr;  // page-locked copy of the two words
+    plb::HostWords* host = nullptr;  // page-locked, written by kernels
     double* red = nullptr;      // reduction partials
     int red_blocks = 0;
     double omega = 0.0;
@@ -326,7 +332,7 @@ int build_table_from_V(plb_ctx* c, const plb_node_info* V, int64_t n);
 int build_table_from_flag(plb_ctx* c, const uint8_t* flag);
 int launch_step(plb_ctx* c, int64_t it, bool write_macros, const int64_t* it_base = nullptr);
 int launch_graph_steps(plb_ctx* c, int64_t it0, int64_t G);
-int launch_reduce(plb_ctx* c, double* host_out2);
+int launch_reduce(plb_ctx* c);  // to c->host, with the fault words
 int build_ref_from_flag(const uint8_t* flag, int nx, int ny, int nz, int num_p, int mode,
                         hipStream_t s, int32_t** tabref_out, uint64_t** xyz_out, int64_t* n_out,
                         std::vector<int32_t>* start_out);
@@ -345,8 +351,8 @@ int launch_read_macros(plb_ctx* c, const MacroList& list, int64_t first, int64_t
 int read_macros_range(plb_ctx* c, int64_t first, int64_t n, double* rho, double* ux, double* uy, double* uz);
 int launch_copy_state(plb_ctx* c, int64_t first, int64_t n, void* aos, bool to_device);
 int launch_read_table(plb_ctx* c, int64_t first, int64_t n, int32_t* dout);
-int launch_reduce_range(plb_ctx* c, int buf, int64_t first, int64_t n, bool with_mass,
-                        double* out2_host);
+int launch_reduce_range(plb_ctx* c, int buf, int64_t first, int64_t n, double* sums, HostWords* words);
+int launch_fault_words(plb_ctx* c);
 int launch_sample_sums(plb_ctx* c, const int32_t* d_active, int n_active, const int32_t* chunk_sample,
                        const int64_t* sample_end, const int64_t* d_off, const int64_t* d_n, int nsamples,
                        double* d_partial, double* d_out);

@@ -625,31 +625,29 @@ __global__ void k_read_table(const StepArgs a, const uint32_t* inv_perm, const u
 constexpr int RED_T = 256;
 
 // Block partial sums over nodes [first, first+n): mass (sum of the stored
-// populations; skipped when with_mass == 0) and ux.
+// populations) and ux.
 template <typename S, int LAYOUT>
 __global__ void __launch_bounds__(RED_T)
 k_reduce_partial(const void* f, const double* ux, int64_t first, int64_t n, int64_t Npad,
-                 float inv, int with_mass, double* partial)
+                 float inv, double* partial)
 {
     __shared__ double sm[2][RED_T];
     double m = 0.0, s = 0.0;
     for (int64_t r = (int64_t)blockIdx.x * RED_T + threadIdx.x; r < n;
          r += (int64_t)gridDim.x * RED_T) {
         const int64_t i = first + r;
-        if (with_mass) {
-            double mi = 0.0;
+        double mi = 0.0;
 #pragma unroll
-            for (int j = 0; j < Q; j++) {
-                const int64_t p = fpos<LAYOUT>(j, i, Npad);
-                if constexpr (sizeof(S) == 8)
-                    mi += ((const double*)f)[p];
-                else if constexpr (sizeof(S) == 4)
-                    mi += (double)((const float*)f)[p];
-                else
-                    mi += (double)(__half2float(((const __half*)f)[p]) * inv);
-            }
-            m += mi;
+        for (int j = 0; j < Q; j++) {
+            const int64_t p = fpos<LAYOUT>(j, i, Npad);
+            if constexpr (sizeof(S) == 8)
+                mi += ((const double*)f)[p];
+            else if constexpr (sizeof(S) == 4)
+                mi += (double)((const float*)f)[p];
+            else
+                mi += (double)(__half2float(((const __half*)f)[p]) * inv);
         }
+        m += mi;
         s += ux[i];
     }
     sm[0][threadIdx.x] = m;
@@ -698,7 +696,10 @@ k_sample_sums(const double* partial, const int64_t* off, const int64_t* n, int b
     if (threadIdx.x == 0) out[s] = t;
 }
 
-__global__ void __launch_bounds__(RED_T) k_reduce_final(double* partial, int nb)
+// The sums, and the fault words when asked, go to page-locked memory: a copy
+// back to the host takes 8 us more than the kernel's own stores.
+__global__ void __launch_bounds__(RED_T)
+k_reduce_final(const double* partial, int nb, double* sums, const unsigned long long* fault, HostWords* words)
 {
     __shared__ double sm[2][RED_T];
     double m = 0.0, s = 0.0;
@@ -717,9 +718,15 @@ __global__ void __launch_bounds__(RED_T) k_reduce_final(double* partial, int nb)
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        partial[2 * nb] = sm[0][0];
-        partial[2 * nb + 1] = sm[1][0];
+        sums[0] = sm[0][0];
+        sums[1] = sm[1][0];
     }
+    if (words && threadIdx.x < 2) words->fault[threadIdx.x] = fault[threadIdx.x];
+}
+
+__global__ void k_fault_words(const unsigned long long* fault, HostWords* words)
+{
+    if (threadIdx.x < 2) words->fault[threadIdx.x] = fault[threadIdx.x];
 }
 
 // ---------------------------------------------------------------- launchers
@@ -1076,27 +1083,30 @@ int launch_read_table(plb_ctx* c, int64_t first, int64_t n, int32_t* dout)
     return PLB_OK;
 }
 
-// out2[0] = sum of stored populations (raw for FP64, deviations otherwise)
-// over nodes [first, first+n) of buffer `buf`, out2[1] = sum of ux macros.
-// Deterministic: fixed grid, fixed tree order.
-int launch_reduce_range(plb_ctx* c, int buf, int64_t first, int64_t n, bool with_mass,
-                        double* out2)
+// Enqueues sums[0] = sum of stored populations (raw for FP64, deviations
+// otherwise) over nodes [first, first+n) of buffer `buf`, sums[1] = sum of ux
+// macros; sums and words (null: none) are page-locked.  Deterministic: fixed
+// grid, fixed tree order.
+int launch_reduce_range(plb_ctx* c, int buf, int64_t first, int64_t n, double* sums, HostWords* words)
 {
     const int nb = std::max(1, std::min<int>(c->red_blocks, (int)((n + RED_T - 1) / RED_T)));
     PLB_DISPATCH(c->cfg.precision, c->cfg.layout, k_reduce_partial, dim3(nb), dim3(RED_T), 0,
-                 c->stream, c->f[buf], c->macros + c->Npad, first, n, c->Npad, c->inv_scale,
-                 with_mass ? 1 : 0, c->red);
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(RED_T), 0, c->stream, c->red, nb);
+                 c->stream, c->f[buf], c->macros + c->Npad, first, n, c->Npad, c->inv_scale, c->red);
+    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(RED_T), 0, c->stream, c->red, nb, sums, c->fault, words);
     PLB_HIP(hipGetLastError());
-    PLB_HIP(hipMemcpyAsync(out2, c->red + 2 * nb, 2 * sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
-    PLB_HIP(hipStreamSynchronize(c->stream));
     return PLB_OK;
 }
 
-int launch_reduce(plb_ctx* c, double* out2)
+int launch_reduce(plb_ctx* c)
 {
-    return launch_reduce_range(c, c->cur, 0, c->N, true, out2);
+    return launch_reduce_range(c, c->cur, 0, c->N, c->host->sum, c->host);
+}
+
+int launch_fault_words(plb_ctx* c)
+{
+    hipLaunchKernelGGL(k_fault_words, dim3(1), dim3(64), 0, c->stream, c->fault, c->host);
+    PLB_HIP(hipGetLastError());
+    return PLB_OK;
 }
 
 int launch_sample_sums(plb_ctx* c, const int32_t* d_active, int n_active, const int32_t* chunk_sample,
