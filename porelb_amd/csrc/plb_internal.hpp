@@ -344,10 +344,11 @@ int launch_step_batch(plb_ctx* c, int64_t it, bool write_macros, const int32_t* 
 int launch_init_eq(plb_ctx* c);
 int launch_read_pop(plb_ctx* c, int64_t first, int64_t n, double* dout);
 int launch_write_pop(plb_ctx* c, int64_t first, int64_t n, const double* din);
-struct MacroList {           // which of rho, ux, uy, uz
+struct MacroList {           // which of rho, ux, uy, uz, and where to
     int n = 0, comp[4] = {0, 0, 0, 0};
+    double* out[4] = {nullptr, nullptr, nullptr, nullptr};
 };
-int launch_read_macros(plb_ctx* c, const MacroList& list, int64_t first, int64_t n, double* dout);
+int launch_read_macros(plb_ctx* c, const MacroList& list, int64_t first, int64_t n);
 int read_macros_range(plb_ctx* c, int64_t first, int64_t n, double* rho, double* ux, double* uy, double* uz);
 int launch_copy_state(plb_ctx* c, int64_t first, int64_t n, void* aos, bool to_device);
 int launch_read_table(plb_ctx* c, int64_t first, int64_t n, int32_t* dout);

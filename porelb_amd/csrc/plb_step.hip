@@ -580,13 +580,13 @@ __global__ void k_copy_state_aa(const StepArgs a, int form, const uint32_t* inv_
 
 // out[q][r] = macro list.comp[q] of V-order node first + r.
 __global__ void k_read_macros(const double* __restrict__ macros, int64_t Npad, const uint32_t* __restrict__ inv_perm,
-                              int64_t first, int64_t n, MacroList list, double* __restrict__ out)
+                              int64_t first, int64_t n, MacroList list)
 {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
     const int64_t g = first + r;
     const int64_t k = inv_perm ? (int64_t)inv_perm[g] : g;
-    for (int q = 0; q < list.n; q++) out[q * n + r] = macros[list.comp[q] * Npad + k];
+    for (int q = 0; q < list.n; q++) list.out[q][r] = macros[list.comp[q] * Npad + k];
 }
 
 template <int LAYOUT, int IDX>
@@ -1053,10 +1053,10 @@ int launch_copy_state(plb_ctx* c, int64_t first, int64_t n, void* aos, bool to_d
     return PLB_OK;
 }
 
-int launch_read_macros(plb_ctx* c, const MacroList& list, int64_t first, int64_t n, double* dout)
+int launch_read_macros(plb_ctx* c, const MacroList& list, int64_t first, int64_t n)
 {
     hipLaunchKernelGGL(k_read_macros, dim3(nblk(n, 256)), dim3(256), 0, c->stream, c->macros, c->Npad, c->inv_perm,
-                       first, n, list, dout);
+                       first, n, list);
     PLB_HIP(hipGetLastError());
     return PLB_OK;
 }

@@ -1,12 +1,16 @@
 // plb_xfer.hip -- the copies between the caller's arrays and device layouts.
 //
-// A read-back gathers a chunk of nodes into a device slot, copies the slot to
-// the host, and goes on with the next chunk in another slot.  Into page-locked
-// memory the copy engine writes at the PCIe rate (53 GB/s).  Pageable memory it
-// reaches only through the runtime's own staging: 17 GB/s, and 7 GB/s into
-// memory that was never touched, because one thread takes all the page faults.
-// Such reads go through page-locked slots here, and a few threads move each
-// slot on, so the faults and the copies are shared; writes go the other way.
+// Into and out of page-locked memory the copy engine moves long passes at the
+// PCIe rate (53 GB/s).  Pageable memory it reaches only through the runtime's own
+// staging: 17 GB/s, and 7 GB/s into memory that was never touched, because one
+// thread takes all the page faults.  Such reads go through page-locked slots
+// here, and a few threads move each slot on, so the faults and the copies are
+// shared; writes go the other way.  The engine fills the slots of a read-back; a
+// write's slots are read by the kernel itself, since for 60 ms after the engine
+// has read such slots it writes page-locked memory at 28 GB/s instead of 54.
+// (Kernels on page-locked arrays otherwise: 54 GB/s for separate components, as
+// plb_read_macros has it; 24 and 4 GB/s for writes and reads of whole states,
+// whose 152-byte rows reach the bus in pieces; records 1.1 times slower.)
 //
 // The slots are kept from call to call (a page-locked allocation costs 140 us,
 // a 16 MB device allocation and its release 45 us), at most MAX_KEPT sets in
@@ -79,7 +83,7 @@ static hipError_t staging_new(int device, Staging** out)
 {
     Staging* s = new Staging();
     s->device = device;
-    hipError_t e = hipHostMalloc((void**)&s->host, SLOT * SLOTS, hipHostMallocDefault);
+    hipError_t e = hipHostMalloc((void**)&s->host, SLOT * SLOTS, hipHostMallocCoherent);
     if (e == hipSuccess) e = dev_alloc((void**)&s->dev, SLOT * SLOTS);
     for (int k = 0; k < SLOTS && e == hipSuccess; k++) e = hipEventCreateWithFlags(&s->copied[k], hipEventDisableTiming);
     if (e != hipSuccess) {
@@ -128,14 +132,14 @@ struct Lease {
     }
 };
 
-static bool page_locked(const void* p)
+bool page_locked(const void* p)
 {
     hipPointerAttribute_t a;
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
-    return a.type == hipMemoryTypeHost;
+    return a.type == hipMemoryTypeHost && a.devicePointer == a.hostPointer;  // kernels take the pointer as it is
 }
 
 // Threads that run work(chunk, thread, threads) for every chunk that is posted.
@@ -211,20 +215,14 @@ static int move(int device, hipStream_t s, int64_t n, size_t item, const std::ve
         return false;
     };
     // the kernel and the copies of m nodes from `first` on, in stream order
-    auto transfer = [&](int64_t first, int64_t m, char* dev, char* host) {
+    auto transfer = [&](int64_t first, int64_t m, char* dev) {
         if (!to_device && (rc = kernel(first, m, dev))) return false;
-        if (host) {
-            if (!check(to_device ? hipMemcpyAsync(dev, host, row * m, hipMemcpyHostToDevice, s)
-                                 : hipMemcpyAsync(host, dev, row * m, hipMemcpyDeviceToHost, s)))
+        for (size_t p = 0; p < arrays.size(); p++) {
+            char* const mine = arrays[p] + (size_t)first * item;
+            char* const part = dev + (size_t)m * p * item;
+            if (!check(to_device ? hipMemcpyAsync(part, mine, m * item, hipMemcpyHostToDevice, s)
+                                 : hipMemcpyAsync(mine, part, m * item, hipMemcpyDeviceToHost, s)))
                 return false;
-        } else {
-            for (size_t p = 0; p < arrays.size(); p++) {
-                char* const mine = arrays[p] + (size_t)first * item;
-                char* const part = dev + (size_t)m * p * item;
-                if (!check(to_device ? hipMemcpyAsync(part, mine, m * item, hipMemcpyHostToDevice, s)
-                                     : hipMemcpyAsync(mine, part, m * item, hipMemcpyDeviceToHost, s)))
-                    return false;
-            }
         }
         return !to_device || (rc = kernel(first, m, dev)) == PLB_OK;
     };
@@ -263,15 +261,18 @@ static int move(int device, hipStream_t s, int64_t n, size_t item, const std::ve
             }
         }
         const int64_t pass = whole_words(have);
-        for (int64_t first = 0; first < n && !rc; first += pass) transfer(first, std::min(pass, n - first), room, nullptr);
+        for (int64_t first = 0; first < n && !rc; first += pass) transfer(first, std::min(pass, n - first), room);
         const hipError_t e = hipStreamSynchronize(s);
         if (!rc) check(e);
         return rc;
     }
     auto chunk = [&](int64_t k) {
         const size_t at = SLOT * (k % SLOTS);
-        return transfer(k * per, std::min(per, n - k * per), st.dev + at, st.host + at) &&
-               check(hipEventRecord(st.copied[k % SLOTS], s));
+        const int64_t m = std::min(per, n - k * per);
+        rc = kernel(k * per, m, to_device ? st.host + at : st.dev + at);
+        if (rc || (!to_device && !check(hipMemcpyAsync(st.host + at, st.dev + at, row * m, hipMemcpyDeviceToHost, s))))
+            return false;
+        return check(hipEventRecord(st.copied[k % SLOTS], s));
     };
     if (to_device) {
         team->post(std::min<int64_t>(chunks, SLOTS));

@@ -10,7 +10,7 @@
 namespace plb {
 
 // Enqueues, on the copy's stream, the kernel that fills (read-backs) or takes
-// (writes) the device slot of nodes first .. first + m - 1: `item` bytes per node
+// (writes) the slot of nodes first .. first + m - 1: `item` bytes per node
 // and array, the arrays one after the other.
 using ChunkKernel = std::function<int(int64_t first, int64_t m, void* slot)>;
 
@@ -18,6 +18,9 @@ using ChunkKernel = std::function<int(int64_t first, int64_t m, void* slot)>;
 int download(int device, hipStream_t s, int64_t n, size_t item, const std::vector<char*>& arrays,
              const ChunkKernel& kernel);
 int upload(int device, hipStream_t s, int64_t n, size_t item, const void* array, const ChunkKernel& kernel);
+
+// Whether p lies in page-locked memory that kernels reach by the same pointer.
+bool page_locked(const void* p);
 
 // +1 for a context that is created, -1 for one that goes: the kept slots go with the last.
 void xfer_context(int add);
