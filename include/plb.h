@@ -167,7 +167,16 @@ int plb_init_equilibrium(plb_ctx *c);
 int plb_step(plb_ctx *c, int64_t it0, int64_t nsteps);
 
 /* As plb_step, but enqueues on the context stream and returns at once;
- * plb_sync waits and reports the density guard. */
+ * plb_sync waits and reports the density guard.
+ * Small lattices (up to 262 144 nodes in FP64, 524 288 in FP32 and FP16) run
+ * calls of 16 steps or more in one cooperative launch with the populations in
+ * the CUs' LDS, from the 128th step on (the plan for it is built in that call,
+ * which then waits for it); the results are the same bit for bit.  Such a run
+ * that cannot complete (its blocks are not all resident) or in which the
+ * density guard trips is repeated with one launch per step by the next call
+ * that waits or reads.  plb_config's launch shape (block size, nodes per
+ * thread, wave cap) is that of launches per step; graph_steps > 0 or one-buffer
+ * streaming keeps to them. */
 int plb_step_async(plb_ctx *c, int64_t it0, int64_t nsteps);
 int plb_sync(plb_ctx *c);
 
@@ -261,8 +270,10 @@ double plb_bytes_per_update(const plb_ctx *c);
 const char *plb_strerror(int code);
 
 /* Page-locked host memory (new; the reference writes from malloc'd arrays,
- * porelb.c:375-391).  plb_read_macros / plb_read_populations copy into such a
- * buffer by DMA at the full PCIe rate instead of through a staging copy.
+ * porelb.c:375-391).  plb_read_macros stores to such buffers from its kernel,
+ * and the other reads and writes move them by DMA, at the full PCIe rate;
+ * pageable memory goes through page-locked slots and a few host threads (from
+ * 3 MB on) at about half of it.
  * Returns NULL on failure; release with plb_host_free. */
 void *plb_host_alloc(size_t bytes);
 void plb_host_free(void *p);
@@ -305,8 +316,12 @@ int plb_batch_create(plb_batch **out, const plb_config *cfg, const plb_sample *s
  * sample ran; updates[0] = total node updates performed; ms = device time. */
 int plb_batch_run(plb_batch *b, int64_t max_steps, int64_t check_every, double tol,
                   int64_t *steps_done, int64_t *updates, double *ms);
-/* The same run as one persistent launch: a resident grid (cooperative
- * launch) advances every sample through the same steps, checks and
+/* The same run as one persistent launch, unless the batch runs on chip: then
+ * plb_batch_run's launches, which are shorter.  (A batch does so when its
+ * checks are 16 steps apart or more and it runs for 128 or more: the samples
+ * that fit the CUs' LDS go from check to check in shared launches, the others
+ * take one launch per step.)  Otherwise a resident grid (cooperative launch)
+ * advances every sample through the same steps, checks and
  * convergence rule as plb_batch_run, with a grid barrier between steps and
  * the per-sample u_x sums and stop decisions made on the device (no host
  * round trip per check).  The per-sample sums use the same fixed order in

@@ -373,6 +373,7 @@ bool onchip_ready(plb_ctx* c, int64_t nsteps);
 int launch_onchip(plb_ctx* c, int64_t it0, int64_t n, uint32_t* serial);
 void onchip_destroy(plb_ctx* c);
 constexpr int ONCHIP_MIN_SLOTS = 256;  // node slots of the smallest on-chip block
+constexpr int64_t ONCHIP_PLAN_STEPS = 128;   // a lattice's plan is built when it has run, or is sure to run, this many
 bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::vector<int64_t>& n,
                         const std::vector<int>& nx, const std::vector<int>& ny, const std::vector<int>& nz, int64_t steps);
 int onchip_blocks(const plb_ctx* c, int sample, int* block0);

@@ -1083,7 +1083,7 @@ bool onchip_ready(plb_ctx* c, int64_t nsteps)
     if (c->cfg.stream_mode != PLB_STREAM_PULL || c->cfg.graph_steps != 0) return false;
     if (c->chip_state == 0) {
         c->chip_steps += nsteps;
-        if (c->chip_steps < 128) return false;
+        if (c->chip_steps < ONCHIP_PLAN_STEPS) return false;
         // a capture of the caller's elsewhere in this thread is none of the plan's business
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
         (void)hipThreadExchangeStreamCaptureMode(&mode);
