@@ -36,8 +36,10 @@ constexpr int SLOTS = 4;
 constexpr size_t LONG_PASS = (size_t)64 << 20;
 constexpr int MAX_KEPT = 4;
 constexpr int MAX_THREADS = 8;
-// From here a pageable copy is worth the threads (a thread starts in about 15 us).
-constexpr size_t THREADED = (size_t)3 << 20;
+// From here a pageable copy is worth the threads (a thread starts in about 15 us),
+// and without a context the slots, which then last for one call only (250 us:
+// records of 54 000 nodes, 8 MB, 0.96 ms with them and 0.86 without).
+constexpr size_t THREADED = (size_t)3 << 20, THREADED_ALONE = 4 * THREADED;
 
 struct Staging {
     int device = 0;
@@ -77,6 +79,12 @@ void xfer_context(int add)
             }
     }
     for (Staging* s : gone) staging_free(s);
+}
+
+static bool slots_are_kept()
+{
+    std::lock_guard<std::mutex> lock(pool_mutex);
+    return contexts > 0;
 }
 
 static hipError_t staging_new(int device, Staging** out)
@@ -200,12 +208,11 @@ static int move(int device, hipStream_t s, int64_t n, size_t item, const std::ve
 {
     const size_t row = item * arrays.size(), bytes = row * (size_t)n;
     if (bytes == 0) return PLB_OK;
-    Lease lease;
-    PLB_HIP(lease.take(device));
-    Staging& st = *lease.s;
     bool locked = true;
     for (const char* a : arrays) locked = locked && page_locked(a);
-    bool threaded = !locked && bytes >= THREADED;
+    Lease lease;
+    bool threaded = !locked && bytes >= (slots_are_kept() ? THREADED : THREADED_ALONE);
+    if (threaded && lease.take(device) != hipSuccess) threaded = false;
 
     int rc = PLB_OK;
     auto check = [&](hipError_t e) {
@@ -237,7 +244,7 @@ static int move(int device, hipStream_t s, int64_t n, size_t item, const std::ve
             const int64_t a = m * t / T, b = m * (t + 1) / T;
             for (size_t p = 0; p < arrays.size(); p++) {
                 char* const mine = arrays[p] + (size_t)(first + a) * item;
-                char* const staged = st.host + SLOT * (k % SLOTS) + ((size_t)m * p + a) * item;
+                char* const staged = lease.s->host + SLOT * (k % SLOTS) + ((size_t)m * p + a) * item;
                 if (to_device) memcpy(staged, mine, (size_t)(b - a) * item);
                 else memcpy(mine, staged, (size_t)(b - a) * item);
             }
@@ -247,25 +254,22 @@ static int move(int device, hipStream_t s, int64_t n, size_t item, const std::ve
     if (!threaded) {
         // One long copy per array and pass: the copy engine reaches its rate
         // from a few MB on.
-        Arena passes(s);
-        DevBuf<char> big;
-        char* room = st.dev;
-        size_t have = SLOT * SLOTS;
-        if (bytes > have) {
-            const size_t want = std::min(bytes + 64 * row, LONG_PASS);
-            if (big.alloc((int64_t)want, &passes) == hipSuccess) {
-                room = big.p;
-                have = want;
-            } else {
-                (void)hipGetLastError();
-            }
+        char* room = nullptr;
+        size_t have = std::min(bytes + 64 * row, LONG_PASS);
+        hipError_t got = dev_alloc((void**)&room, have);
+        while (got != hipSuccess && have > SLOT) {  // little memory left: shorter passes
+            (void)hipGetLastError();
+            got = dev_alloc((void**)&room, have = std::max(SLOT, have / 4));
         }
+        PLB_HIP(got);
         const int64_t pass = whole_words(have);
         for (int64_t first = 0; first < n && !rc; first += pass) transfer(first, std::min(pass, n - first), room);
         const hipError_t e = hipStreamSynchronize(s);
+        dev_free(room);
         if (!rc) check(e);
         return rc;
     }
+    Staging& st = *lease.s;
     auto chunk = [&](int64_t k) {
         const size_t at = SLOT * (k % SLOTS);
         const int64_t m = std::min(per, n - k * per);
