@@ -37,14 +37,7 @@ __global__ void __launch_bounds__(1024) k_step(const StepArgs a)
     node_any<S, LAYOUT, IDX>(with_step(a), i, *a.fault);
 }
 
-// How k_step_keep stores: plainly in `share` of 16 groups of 16 blocks, or (tail
-// not 0) in the last `tail` of 256 parts of its sweep, which may go backwards.
-struct KeepArgs {
-    int share, tail;
-    bool back;
-};
-
-// Single lattice with plain stores of some blocks, for FP64 and
+// The same with plain stores for `keep` of 16 groups of 16 blocks, for FP64 and
 // FP32 lattices that do not fit the L2s (8 x 4 MB) but whose two buffers and index
 // fit the 256 MB memory-side cache, all or in part: non-temporal stores go past
 // that cache, and the next step then reads from HBM what this one wrote.  Of a
@@ -57,24 +50,15 @@ struct KeepArgs {
 // 3 194 400 (549 MB), 138.8 / 138.7 at 4 251 746 (731 MB).  Below 32 MB plain stores
 // lose (FP64 7.1 / 6.5 at 78 643 nodes), and FP16, bound by L2 requests, gains at no
 // size.
-// Larger still, every second step sweeps backwards (each XCD its own stretch),
-// and the last `tail` of 256 parts of a sweep, 300 MB with what they read, store
-// plainly: the next step begins with them.  FP64 285.6 / 290.7 at 5 033 165 nodes
-// (1 631 MB), 459 / 463 at 8 100 000; FP32 128.1 / 133.3 at 4 251 746 (731 MB), 151.9 /
-// 156.5 at 5 033 165 (866 MB), 203.0 / 204.5 at 6 585 600 (1 133 MB).
 template <typename S, int LAYOUT, int IDX>
-__global__ void __launch_bounds__(1024) k_step_keep(const StepArgs a, const KeepArgs k)
+__global__ void __launch_bounds__(1024) k_step_keep(const StepArgs a, int keep)
 {
-    const int64_t first = xcd_block(blockIdx.x & 7, gridDim.x), slot = blockIdx.x >> 3;
-    const int64_t len = (gridDim.x >> 3) + ((blockIdx.x & 7) < (gridDim.x & 7));
-    const int64_t blk = first + (k.back ? len - 1 - slot : slot);
+    const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
     const int64_t i = blk * blockDim.x + threadIdx.x;
     if (i >= a.N) return;
-    const bool keep = k.tail ? slot * 256 >= len * (256 - k.tail) : (int)((blk >> 4) & 15) < k.share;
-    node_any<S, LAYOUT, IDX, false, true>(with_step(a), i, *a.fault, keep);
+    node_any<S, LAYOUT, IDX, false, true>(with_step(a), i, *a.fault, (int)((blk >> 4) & 15) < keep);
 }
-constexpr double KEEP_ABOVE = 32e6, KEEP_ALL = 208e6, KEEP_SHARE = 600e6, KEEP_MOST = 3e9,
-                 KEEP_BYTES = 115e6, KEEP_TAIL = 300e6;
+constexpr double KEEP_ABOVE = 32e6, KEEP_ALL = 208e6, KEEP_MOST = 600e6, KEEP_BYTES = 115e6;
 
 // Single lattice, one buffer, AA pattern (half-way bounce-back).  The
 // buffer alternates between two forms of the post-collision populations
@@ -827,20 +811,17 @@ static unsigned step_lds_bytes(const plb_ctx* c, int bs)
     return (unsigned)(share / 512 * 512);
 }
 
-// Whether k_step_keep runs, and with what.
-static bool keep_stores(const plb_ctx* c, KeepArgs* k)
+// Groups of 16 whose stores are plain; 0: k_step.
+static int keep_stores(const plb_ctx* c)
 {
     const double bytes = (2.0 * Q * c->elem + c->index_bytes) * (double)c->N;
-    if (c->cfg.precision == PLB_FP16 || bytes <= KEEP_ABOVE || bytes > KEEP_MOST) return false;
-    *k = {16, 0, false};
-    if (bytes > KEEP_SHARE) *k = {0, (int)(256.0 * KEEP_TAIL / bytes + 0.5), c->cur != 0};
-    else if (bytes > KEEP_ALL) k->share = (int)(16.0 * KEEP_BYTES / bytes + 0.5);
-    return true;
+    if (c->cfg.precision == PLB_FP16 || bytes <= KEEP_ABOVE || bytes > KEEP_MOST) return 0;
+    return bytes <= KEEP_ALL ? 16 : (int)(16.0 * KEEP_BYTES / bytes + 0.5);
 }
 
-static void launch_keep(const plb_ctx* c, const StepArgs& a, const KeepArgs& k, dim3 grid, dim3 block, unsigned lds)
+static void launch_keep(const plb_ctx* c, const StepArgs& a, int keep, dim3 grid, dim3 block, unsigned lds)
 {
-    auto run = [&](auto* kern) { hipLaunchKernelGGL(kern, grid, block, lds, c->stream, a, k); };
+    auto run = [&](auto* kern) { hipLaunchKernelGGL(kern, grid, block, lds, c->stream, a, keep); };
     auto with = [&](auto layout, auto idx) {
         constexpr int L = decltype(layout)::value, I = decltype(idx)::value;
         c->cfg.precision == PLB_FP64 ? run(k_step_keep<double, L, I>) : run(k_step_keep<float, L, I>);
@@ -877,8 +858,8 @@ int launch_step(plb_ctx* c, int64_t it, bool write_macros, const int64_t* it_bas
         const int64_t threads = (c->N + 127) / 128 * 64;
         PLB_DISPATCH3(c->cfg.precision, c->cfg.layout, c->cfg.index_kind, k_step2,
                       dim3(nblk(threads, bs)), dim3(bs), lds, c->stream, a);
-    } else if (KeepArgs k; keep_stores(c, &k)) {
-        launch_keep(c, a, k, dim3(nblk(c->N, bs)), dim3(bs), lds);
+    } else if (const int keep = keep_stores(c)) {
+        launch_keep(c, a, keep, dim3(nblk(c->N, bs)), dim3(bs), lds);
     } else {
         PLB_DISPATCH3(c->cfg.precision, c->cfg.layout, c->cfg.index_kind, k_step, dim3(nblk(c->N, bs)),
                       dim3(bs), lds, c->stream, a);

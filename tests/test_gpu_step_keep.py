@@ -1,6 +1,6 @@
 """Step kernels with plain and with non-temporal stores compute the same: lattices on both sides of the sizes
-(32, 208, 600 and 3 000 MB of populations and index) between which all or some blocks store plainly, against
-the two-nodes-per-thread kernel, which has non-temporal stores."""
+(32, 208 and 600 MB of populations and index) between which all or some blocks store plainly, against the
+two-nodes-per-thread kernel, which has non-temporal stores."""
 import numpy as np
 import pytest
 
