@@ -274,7 +274,7 @@ static int clear_fault(plb_ctx* c)
     PLB_HIP(hipMemsetAsync(c->fault, 0xff, 2 * sizeof(unsigned long long), c->stream));
     PLB_HIP(hipStreamSynchronize(c->stream));
     c->segs.clear();
-    c->fault_seen = false;
+    c->fault_seen = c->fault_held = false;
     return PLB_OK;
 }
 
@@ -304,40 +304,60 @@ static int read_fault_words(plb_ctx* c, unsigned long long* key, unsigned long l
     return PLB_OK;
 }
 
-// Waits for the calls since the last plb_sync.  An on-chip run in which the
-// density guard tripped, or which gave up waiting for a block, has left the
-// state before it (and the macros) untouched, and everything queued behind it
-// has left the state alone: it and the calls after it are repeated with one
-// launch per step, which freeze at the end of the faulting step.
+// Waits for the calls that are queued and settles them: none is left in c->segs,
+// and c->cur is the buffer of the state.  An on-chip run in which the density
+// guard tripped, or which gave up waiting for a block, has left the state before
+// it (and the macros) untouched, and everything queued behind it has left the
+// state alone: it and the calls after it are repeated with one launch per step,
+// which freeze at the end of the faulting step.  (The queued calls' step numbers
+// rise, so a fault's step names its call.)
 static int settle(plb_ctx* c, unsigned long long* key)
 {
     unsigned long long gave_up = NO_FAULT;
     int rc = read_fault_words(c, key, &gave_up);
-    if (rc || *key == NO_FAULT) return rc;
+    if (rc) return rc;
+    auto trips = [&](const Segment& s) {
+        const int64_t fs = (int64_t)(*key >> 32);
+        return *key != HOLD_FAULT && fs >= s.it0 && fs < s.it0 + s.n;
+    };
     size_t k = 0;
-    const int64_t fs = (int64_t)(*key >> 32);
-    for (; k < c->segs.size(); k++) {
-        const Segment& s = c->segs[k];
-        if (s.serial && (s.serial == gave_up || (*key != HOLD_FAULT && fs >= s.it0 && fs < s.it0 + s.n))) break;
-    }
-    if (k == c->segs.size()) return PLB_OK;
-    if (gave_up != NO_FAULT) {
-        fprintf(stderr, "libplb: an on-chip run's blocks were not all resident; this lattice goes on with one launch per step\n");
-        c->chip_state = -1;
-    }
-    PLB_HIP(hipMemsetAsync(c->fault, 0xff, 2 * sizeof(unsigned long long), c->stream));
-    c->cur = c->segs[k].cur;
-    onchip_restore_macros(c, c->segs[k].macros);
-    for (; k < c->segs.size(); k++) {
-        Segment& s = c->segs[k];
-        s.serial = 0;
-        s.cur = c->cur;
-        for (int64_t t = 0; t < s.n; t++) {
-            rc = launch_step(c, s.it0 + t, t == s.n - 1);
-            if (rc) return rc;
+    if (*key != NO_FAULT)
+        while (k < c->segs.size() && !(c->segs[k].serial && (c->segs[k].serial == gave_up || trips(c->segs[k])))) k++;
+    if (*key != NO_FAULT && k < c->segs.size()) {
+        if (gave_up != NO_FAULT) {
+            fprintf(stderr, "libplb: an on-chip run's blocks were not all resident; this lattice goes on with one launch per step\n");
+            c->chip_state = -1;
         }
+        PLB_HIP(hipMemsetAsync(c->fault, 0xff, 2 * sizeof(unsigned long long), c->stream));
+        c->cur = c->segs[k].cur;
+        onchip_restore_macros(c, c->segs[k].macros);
+        for (; k < c->segs.size(); k++) {
+            Segment& s = c->segs[k];
+            s.serial = 0;
+            s.cur = c->cur;
+            for (int64_t t = 0; t < s.n; t++) {
+                rc = launch_step(c, s.it0 + t, t == s.n - 1);
+                if (rc) return rc;
+            }
+        }
+        rc = read_fault_words(c, key, &gave_up);
+        if (rc) return rc;
     }
-    return read_fault_words(c, key, &gave_up);
+    if (*key != NO_FAULT) {
+        // Steps after the faulting one did not run: the faulting step's output
+        // buffer holds the current state.  A fault from an earlier call made
+        // every launch of these a no-op.
+        const int64_t fs = (int64_t)(*key >> 32);
+        if (!c->segs.empty() && fs < c->segs[0].it0) c->cur = c->segs[0].cur;
+        for (const Segment& s : c->segs)
+            if (trips(s)) {
+                c->cur = s.cur ^ (int)((fs - s.it0 + 1) & 1);
+                break;
+            }
+        if (!c->fault_seen) c->fault_held = true;
+    }
+    c->segs.clear();
+    return PLB_OK;
 }
 
 // Before the state or the macros are read without a plb_sync.
@@ -356,12 +376,17 @@ extern "C" int plb_step_async(plb_ctx* c, int64_t it0, int64_t nsteps)
     if (!c || nsteps < 0 || it0 < 0 || it0 + nsteps >= ((int64_t)1 << 31)) return PLB_ERR_INVALID;
     Range range("plb_step");
     PLB_HIP(hipSetDevice(c->device));
-    // A call that goes back in time behind an unsettled on-chip run would
-    // not be held off by a fault of that run.
+    // A call whose step numbers start again would not be held off by a fault of
+    // the calls before it, and the fault's step would not tell it from them.
     if (!c->segs.empty() && it0 < c->segs.back().it0 + c->segs.back().n) {
-        int rc = settle_for_read(c);
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // it waits, also beside a capture of the caller's
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        unsigned long long key;
+        const int rc = settle(c, &key);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
         if (rc) return rc;
     }
+    if (c->fault_held) return PLB_OK;  // the state stays that of a fault until plb_sync has reported it
     Segment seg{it0, nsteps, c->cur, 0, c->macros};
     if (onchip_ready(c, nsteps)) {
         int rc = launch_onchip(c, it0, nsteps, &seg.serial);
@@ -391,22 +416,11 @@ extern "C" int plb_sync(plb_ctx* c)
     if (!c) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
     unsigned long long key = NO_FAULT;
-    int rc = settle(c, &key);
+    const int rc = settle(c, &key);
     if (rc) return rc;
-    std::vector<Segment> segs;
-    segs.swap(c->segs);
     if (key == NO_FAULT) return PLB_OK;
+    c->fault_held = false;
     c->fault_seen = true;
-    const int64_t fs = (int64_t)(key >> 32);
-    // Steps after the faulting one did not run: the faulting step's output
-    // buffer holds the current state.  A fault from an earlier call made
-    // every launch of this one a no-op.
-    if (!segs.empty() && fs < segs[0].it0) c->cur = segs[0].cur;
-    for (const Segment& s : segs)
-        if (fs >= s.it0 && fs < s.it0 + s.n) {
-            c->cur = s.cur ^ (int)((fs - s.it0 + 1) & 1);
-            break;
-        }
     return PLB_ERR_DENSITY;
 }
 

@@ -206,7 +206,7 @@ struct DevBuf {
 };
 
 struct OnchipPlan;
-// One plb_step_async call that plb_sync has not settled yet.
+// One plb_step_async call that has not been settled yet.
 struct Segment {
     int64_t it0, n;
     int cur;             // buffer of the state before it
@@ -266,8 +266,9 @@ struct plb_ctx {
     double omega = 0.0;
     float scale = 1.f, inv_scale = 1.f;  // FP16 storage scale 2^scale_log2
     int scale_log2 = 0;
-    std::vector<plb::Segment> segs;  // calls since the last plb_sync
-    bool fault_seen = false;    // the density guard tripped and the state was not replaced
+    std::vector<plb::Segment> segs;  // calls that are queued, their step numbers rising
+    bool fault_seen = false;    // plb_sync has reported a trip of the density guard, and the state was not replaced
+    bool fault_held = false;    // a trip was found that plb_sync has yet to report
     // On-chip runs of small lattices (plb_onchip.hip)
     plb::OnchipPlan* chip = nullptr;
     int chip_state = 0;         // 0: no plan yet, 1: plan ready, -1: not used for this lattice

@@ -1,0 +1,66 @@
+"""Density-guard trips in queues of asynchronous calls: the fault, the frozen
+state and the macros are those of the same calls made one by one with one
+launch per step (graph_steps longer than any call keeps a lattice to that)."""
+import pytest
+
+import numpy as np
+
+pytestmark = pytest.mark.gpu
+
+# Without the guard's trip the flow would be past it at about step 46 (FP64, counted from rest).
+GX = 0.003
+
+
+def pair(plb, precision, gx=GX):
+    flag = plb.mask_spheres((30, 32, 34), 3.0, 5.0, 0.5, 4)
+    kw = dict(tau=0.51, gx=gx, precision=precision, bb_mode=1, fp16_rounding=1, index_kind=1, layout=1, ordering=2,
+              brick=(34, 8, 1), block_size=128)
+    return plb.Lattice.from_flag(flag, **kw), plb.Lattice.from_flag(flag, graph_steps=1024, **kw)
+
+
+def warm(lat):
+    """Past the 128 steps from which calls of 16 or more run on chip."""
+    lat.step_rc(0, 130)
+    lat.init_equilibrium()
+
+
+def one_by_one(plb, lat, calls):
+    """The calls, each waited for, up to the first that trips."""
+    for it0, n in calls:
+        rc = lat.step_rc(it0, n)
+        if rc:
+            return rc
+    return 0
+
+
+def same(a, b):
+    assert a.last_fault() == b.last_fault()
+    assert np.array_equal(a.read_state(), b.read_state())
+    assert np.array_equal(a.read_macros(), b.read_macros())
+
+
+@pytest.mark.parametrize("read", ["", "read", "reduce"])
+@pytest.mark.parametrize("n", [60, 61, 30, 31])   # the trip falls into the first call, into the second
+@pytest.mark.parametrize("precision", [0, 1, 2])
+@pytest.mark.parametrize("chip", [True, False])
+def test_step_numbers_that_start_again(plb, chip, precision, n, read):
+    a, b = pair(plb, precision)
+    if not chip:
+        a = pair(plb, precision)[1]
+    L = plb.lib()
+    with a, b:
+        if chip:
+            warm(a)
+        rc = one_by_one(plb, b, [(0, n), (0, n)])
+        assert rc == plb.ERR_DENSITY
+        assert L.plb_step_async(a._h, 0, n) == 0
+        if read:
+            a.read_macros() if read == "read" else a.reduce()
+        assert L.plb_step_async(a._h, 0, n) == 0
+        assert L.plb_sync(a._h) == rc
+        same(a, b)
+        # and from rest again, on chip as before
+        a.init_equilibrium()
+        b.init_equilibrium()
+        assert a.step_rc(0, n) == b.step_rc(0, n)
+        same(a, b)
