@@ -345,13 +345,14 @@ static int settle(plb_ctx* c, unsigned long long* key)
     }
     if (*key != NO_FAULT) {
         // Steps after the faulting one did not run: the faulting step's output
-        // buffer holds the current state.  A fault from an earlier call made
-        // every launch of these a no-op.
+        // buffer holds the current state (a fault from an earlier call made
+        // every launch of these a no-op), and the macros are in the array that
+        // its call writes, also where on-chip runs behind it have swapped them.
         const int64_t fs = (int64_t)(*key >> 32);
-        if (!c->segs.empty() && fs < c->segs[0].it0) c->cur = c->segs[0].cur;
         for (const Segment& s : c->segs)
-            if (trips(s)) {
-                c->cur = s.cur ^ (int)((fs - s.it0 + 1) & 1);
+            if (fs < s.it0 + s.n) {
+                c->cur = fs < s.it0 ? s.cur : s.cur ^ (int)((fs - s.it0 + 1) & 1);
+                onchip_restore_macros(c, s.macros);
                 break;
             }
         if (!c->fault_seen) c->fault_held = true;

@@ -64,3 +64,40 @@ def test_step_numbers_that_start_again(plb, chip, precision, n, read):
         b.init_equilibrium()
         assert a.step_rc(0, n) == b.step_rc(0, n)
         same(a, b)
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2])
+def test_trip_in_front_of_a_queued_run(plb, precision):
+    """The trip falls into launches per step, before the 128th step; the call
+    queued behind them would run on chip, and is held off."""
+    a, b = pair(plb, precision)
+    L = plb.lib()
+    with a, b:
+        rc = one_by_one(plb, b, [(0, 100), (100, 100)])
+        assert rc == plb.ERR_DENSITY
+        assert L.plb_step_async(a._h, 0, 100) == 0
+        assert L.plb_step_async(a._h, 100, 100) == 0
+        assert L.plb_sync(a._h) == rc
+        same(a, b)
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2])
+def test_queued_runs_before_a_trip_and_behind_it(plb, precision):
+    """On-chip runs by turns with short calls; the trip falls into a short one."""
+    a, b = pair(plb, precision)
+    L = plb.lib()
+    with a, b:
+        warm(a)
+        b.step_rc(0, 200)
+        trip = b.last_fault()["step"]
+        b.init_equilibrium()
+        calls = [(0, trip - 5), (trip - 5, 12), (trip + 7, 40), (trip + 47, 3)]
+        rc = one_by_one(plb, b, calls)
+        assert rc == plb.ERR_DENSITY and b.last_fault()["step"] == trip
+        for it0, n in calls:
+            assert L.plb_step_async(a._h, it0, n) == 0
+        assert a.last_fault() == b.last_fault()     # a read before plb_sync
+        assert np.array_equal(a.read_macros(), b.read_macros())
+        assert L.plb_step_async(a._h, trip + 100, 60) == 0
+        assert L.plb_sync(a._h) == rc
+        same(a, b)
