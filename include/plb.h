@@ -175,10 +175,11 @@ int plb_step(plb_ctx *c, int64_t it0, int64_t nsteps);
  * that cannot complete (its blocks are not all resident) or in which the
  * density guard trips is repeated with one launch per step by the next call
  * that waits or reads.  A call whose step numbers start again, before the end
- * of one that is still queued, waits for the queued ones; after a trip that
- * plb_sync has yet to report, it leaves the state alone.  plb_config's launch shape (block size, nodes per
- * thread, wave cap) is that of launches per step; graph_steps > 0 or one-buffer
- * streaming keeps to them. */
+ * of one that is still queued, waits for the queued ones (and so does a call
+ * behind 256 that no plb_sync or read has waited for); after a trip that
+ * plb_sync has yet to report, it leaves the state alone.  plb_config's launch
+ * shape (block size, nodes per thread, wave cap) is that of launches per step;
+ * graph_steps > 0 or one-buffer streaming keeps to them. */
 int plb_step_async(plb_ctx *c, int64_t it0, int64_t nsteps);
 int plb_sync(plb_ctx *c);
 

@@ -121,6 +121,7 @@ int plb::ctx_begin(plb_ctx* c, const plb_config* cfg, int nx, int ny, int nz, in
 {
     xfer_context(1);
     c->counted = true;
+    c->segs.reserve(SEGMENTS_MOST);
     c->cfg = *cfg;
     c->nx = nx;
     c->ny = ny;
@@ -379,7 +380,7 @@ extern "C" int plb_step_async(plb_ctx* c, int64_t it0, int64_t nsteps)
     PLB_HIP(hipSetDevice(c->device));
     // A call whose step numbers start again would not be held off by a fault of
     // the calls before it, and the fault's step would not tell it from them.
-    if (!c->segs.empty() && it0 < c->segs.back().it0 + c->segs.back().n) {
+    if (c->segs.size() >= SEGMENTS_MOST || (!c->segs.empty() && it0 < c->segs.back().it0 + c->segs.back().n)) {
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // it waits, also beside a capture of the caller's
         (void)hipThreadExchangeStreamCaptureMode(&mode);
         unsigned long long key;
@@ -408,7 +409,10 @@ extern "C" int plb_step_async(plb_ctx* c, int64_t it0, int64_t nsteps)
         int rc = launch_step(c, it0 + s, s == nsteps - 1);
         if (rc) return rc;
     }
-    if (nsteps > 0) c->segs.push_back(seg);
+    // steps that go on from launches per step are of one call with them
+    Segment* const last = c->segs.empty() ? nullptr : &c->segs.back();
+    if (last && !last->serial && last->it0 + last->n == it0) last->n += nsteps;
+    else if (nsteps > 0) c->segs.push_back(seg);
     return PLB_OK;
 }
 

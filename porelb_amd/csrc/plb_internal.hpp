@@ -213,6 +213,7 @@ struct Segment {
     uint32_t serial;     // on-chip run: its serial number; 0: one launch per step
     double* macros;      // macros array before it
 };
+constexpr size_t SEGMENTS_MOST = 256;  // queued calls; one more settles them first
 
 // What the host waits for between calls.
 struct HostWords {

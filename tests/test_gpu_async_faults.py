@@ -101,3 +101,44 @@ def test_queued_runs_before_a_trip_and_behind_it(plb, precision):
         assert L.plb_step_async(a._h, trip + 100, 60) == 0
         assert L.plb_sync(a._h) == rc
         same(a, b)
+
+
+@pytest.mark.parametrize("gap", [0, 1])
+def test_queue_without_a_sync_stays_small(plb, gap):
+    """Asynchronous calls and reads, never a plb_sync: no memory for every call."""
+    def resident():
+        return int(open("/proc/self/statm").read().split()[1]) * 4096
+
+    L = plb.lib()
+    a, b = pair(plb, 1, gx=1e-6)
+    with a, b:
+        it = 0
+
+        def queue(calls):
+            nonlocal it
+            for k in range(calls):
+                assert L.plb_step_async(b._h, it, 1) == 0
+                it += 1 + gap
+                if k % 1000 == 0:
+                    b.reduce()
+
+        queue(20_000)
+        before = resident()
+        queue(400_000)
+        assert resident() - before < 4 << 20
+        assert L.plb_sync(b._h) == 0
+
+
+def test_long_queue_ends_in_the_same_state(plb):
+    """More calls than the queue holds, on chip and between, and a trip behind them."""
+    a, b = pair(plb, 0, gx=0.002)     # trips at about step 144
+    L = plb.lib()
+    with a, b:
+        warm(a)
+        # steps in a row, steps with gaps in their numbers, on-chip runs
+        calls = [(k, 1) for k in range(140)] + [(140 + 2 * k, 1) for k in range(300)] + [(800, 20), (820, 20), (840, 3)]
+        rc = one_by_one(plb, b, calls)
+        for it0, n in calls:
+            assert L.plb_step_async(a._h, it0, n) == 0
+        assert L.plb_sync(a._h) == rc == plb.ERR_DENSITY
+        same(a, b)
