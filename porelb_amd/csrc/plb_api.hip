@@ -273,6 +273,10 @@ __global__ void k_fill_macros(double* m, int64_t Npad, double rho0)
 static int clear_fault(plb_ctx* c)
 {
     PLB_HIP(hipMemsetAsync(c->fault, 0xff, 2 * sizeof(unsigned long long), c->stream));
+    if (c->chip) {
+        const int rc = onchip_clear(c);
+        if (rc) return rc;
+    }
     PLB_HIP(hipStreamSynchronize(c->stream));
     c->segs.clear();
     c->fault_seen = c->fault_held = false;

@@ -341,7 +341,6 @@ static int batch_run(plb_batch* b, int64_t max_steps, int64_t check_every, doubl
     plb_ctx* c = b->c;
     *again = false;
     int rc = plb_init_equilibrium(c);
-    if (!rc && chip) rc = onchip_batch_begin(c);
     if (rc) return rc;
     b->active.assign(b->S, 1);
     for (int s = 0; s < b->S; s++)

@@ -380,7 +380,7 @@ bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::
                         const std::vector<int>& nx, const std::vector<int>& ny, const std::vector<int>& nz, int64_t steps);
 int onchip_blocks(const plb_ctx* c, int sample, int* block0);
 void onchip_pack(const std::vector<int>& blocks, int cus, std::vector<std::vector<int>>* launches);
-int onchip_batch_begin(plb_ctx* c);
+int onchip_clear(plb_ctx* c);
 int launch_onchip_batch(plb_ctx* c, int64_t it0, int64_t n, const int32_t* list, int blocks, const double* omega,
                         const double* gx);
 void onchip_batch_next(plb_ctx* c, int64_t n);

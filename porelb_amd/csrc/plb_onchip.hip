@@ -1135,6 +1135,18 @@ static hipError_t launch(plb_ctx* c, const StepArgs& a0, OnchipArgs o, int64_t n
     return e;
 }
 
+// No step number of an earlier run is left in the buffers.  A run's numbers go on
+// from those of the run before it, whose words lie one or two numbers back when
+// it has run to its end; a run that was held off by a fault stores none, so the
+// numbers (16 bits with FP16 words) may come round to the old words.  A fault ends
+// with a new state, and so does a run of a batch begin.
+int onchip_clear(plb_ctx* c)
+{
+    if (c->chip->recv_bytes) PLB_HIP(hipMemsetAsync(c->chip->recv, 0, c->chip->recv_bytes, c->stream));
+    c->chip->tag = 16;
+    return PLB_OK;
+}
+
 static uint32_t next_serial(OnchipPlan* p) { return ++p->serial ? p->serial : ++p->serial; }
 
 int launch_onchip(plb_ctx* c, int64_t it0, int64_t n, uint32_t* serial)
@@ -1258,14 +1270,6 @@ int onchip_blocks(const plb_ctx* c, int sample, int* block0)
     const OnchipSample& s = c->chip->samples[sample];
     *block0 = s.block0;
     return s.nblocks;
-}
-
-// A new run of the batch: no number of an earlier one is left in the buffers.
-int onchip_batch_begin(plb_ctx* c)
-{
-    if (c->chip->recv_bytes) PLB_HIP(hipMemsetAsync(c->chip->recv, 0, c->chip->recv_bytes, c->stream));
-    c->chip->tag = 16;
-    return PLB_OK;
 }
 
 // The samples of `list`, n steps from buffer c->cur to the buffer that n

@@ -142,3 +142,23 @@ def test_long_queue_ends_in_the_same_state(plb):
             assert L.plb_step_async(a._h, it0, n) == 0
         assert L.plb_sync(a._h) == rc == plb.ERR_DENSITY
         same(a, b)
+
+
+@pytest.mark.parametrize("frozen", [65_530, 65_531])
+def test_runs_after_a_long_held_off_call(plb, frozen):
+    """FP16 words carry 16 bits of the step number, which a held-off call of this
+    length brings round to those that the run before it left in the buffers."""
+    a, b = pair(plb, 2)
+    good = plb.Lattice.from_flag(plb.mask_spheres((30, 32, 34), 3.0, 5.0, 0.5, 4), tau=0.51, gx=GX, precision=2, bb_mode=1)
+    L = plb.lib()
+    with a, b, good:
+        warm(a)
+        good.step(0, 20)
+        state = good.read_state()
+        for call in [(0, 200), (200, frozen)]:
+            assert L.plb_step_async(a._h, *call) == 0
+        assert L.plb_sync(a._h) == plb.ERR_DENSITY
+        a.write_state(state)
+        b.write_state(state)
+        assert a.step_rc(0, 20) == b.step_rc(0, 20)
+        same(a, b)
