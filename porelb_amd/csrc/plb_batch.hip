@@ -255,6 +255,9 @@ extern "C" int plb_batch_create(plb_batch** out, const plb_config* cfg, const pl
     return PLB_OK;
 }
 
+extern "C" int plb_test_withhold_block(plb_ctx* c, int runs);
+extern "C" int plb_test_batch_withhold_block(plb_batch* b, int runs) { return plb_test_withhold_block(b->c, runs); }
+
 extern "C" int64_t plb_batch_num_nodes(const plb_batch* b, int s)
 {
     if (!b || s < 0 || s >= b->S) return -1;
@@ -368,14 +371,16 @@ static int batch_run(plb_batch* b, int64_t max_steps, int64_t check_every, doubl
         rc = launch_sample_sums(c, b->d_active, b->n_active, b->d_block_sample, b->d_end, b->d_off, b->d_n, b->S,
                                 b->d_partial, b->d_sums);
         if (rc) return rc;
-        unsigned long long key = NO_FAULT;
+        unsigned long long words[2] = {NO_FAULT, NO_FAULT};
         PLB_HIP(hipMemcpyAsync(sums.data(), b->d_sums, sizeof(double) * b->S, hipMemcpyDeviceToHost,
                                c->stream));
-        PLB_HIP(hipMemcpyAsync(&key, c->fault, sizeof key, hipMemcpyDeviceToHost, c->stream));
+        PLB_HIP(hipMemcpyAsync(words, c->fault, sizeof words, hipMemcpyDeviceToHost, c->stream));
         PLB_HIP(hipStreamSynchronize(c->stream));
-        if (key != NO_FAULT) {
+        if (words[0] != NO_FAULT) {
             *again = chip;
-            if (key == HOLD_FAULT) c->chip_state = -1;  // blocks that were not all resident: not tried again
+            // Blocks that were not all resident: not tried again.  (Such a launch goes on
+            // to the end of its step, where it may record a trip as well.)
+            if (words[1] != NO_FAULT) c->chip_state = -1;
             return PLB_ERR_DENSITY;
         }
         bool changed = false;

@@ -274,6 +274,7 @@ struct plb_ctx {
     plb::OnchipPlan* chip = nullptr;
     int chip_state = 0;         // 0: no plan yet, 1: plan ready, -1: not used for this lattice
     int64_t chip_steps = 0;     // steps asked for in calls long enough for the on-chip run
+    int chip_withhold = 0;      // tests: runs to launch without their last block
 };
 
 // Error helpers (host).

@@ -52,6 +52,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <utility>
 
 #include "plb_device.hpp"
 
@@ -1121,6 +1122,10 @@ static hipError_t launch(plb_ctx* c, const StepArgs& a0, OnchipArgs o, int64_t n
     o.first_ticks = (uint64_t)khz * 50;
     o.wait_ticks = (uint64_t)khz * 2000;
     hipError_t e = hipErrorUnknown;
+    if (blocks > 1 && c->chip_withhold > 0) {
+        c->chip_withhold--;
+        blocks--;   // the others wait for it, and give up
+    }
     with_kernel(c, p, [&](auto* kern) {
         void* args[] = {(void*)&a, (void*)&o};
         const size_t lds = lds_bytes(c, p->NS, p->twice);
@@ -1146,6 +1151,10 @@ int onchip_clear(plb_ctx* c)
     c->chip->tag = 16;
     return PLB_OK;
 }
+
+// Tests only: launches the next `runs` runs of more than one block without the
+// last one, as if it were not resident; returns how many were still to come.
+extern "C" int plb_test_withhold_block(plb_ctx* c, int runs) { return std::exchange(c->chip_withhold, runs); }
 
 static uint32_t next_serial(OnchipPlan* p) { return ++p->serial ? p->serial : ++p->serial; }
 

@@ -1,0 +1,100 @@
+"""On-chip runs that cannot complete: a launch without its last block, as when
+that block finds no room on the chip.  The other blocks' waits end, and the run
+is repeated with one launch per step, with the results of that."""
+import ctypes as C
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPE = dict(index_kind=1, layout=1, ordering=2, block_size=128)
+
+
+def withhold(plb, obj, runs):
+    """The next `runs` launches go without a block; returns how many were still to come."""
+    name = "plb_test_batch_withhold_block" if isinstance(obj, plb.Batch) else "plb_test_withhold_block"
+    f = getattr(plb.lib(), name)
+    f.argtypes, f.restype = [C.c_void_p, C.c_int], C.c_int
+    return f(obj._h, runs)
+
+
+def same(a, b):
+    assert np.array_equal(a.read_state(), b.read_state())
+    assert np.array_equal(a.read_macros(), b.read_macros())
+
+
+def pair(plb, precision, tau=0.8, gx=1e-5):
+    flag = plb.mask_spheres((30, 32, 34), 3.0, 5.0, 0.5, 4)
+    kw = dict(tau=tau, gx=gx, precision=precision, bb_mode=1, fp16_rounding=1, brick=(34, 8, 1), **SHAPE)
+    return plb.Lattice.from_flag(flag, **kw), plb.Lattice.from_flag(flag, graph_steps=1024, **kw)
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2])
+def test_queue_with_a_run_that_gives_up(plb, precision):
+    a, b = pair(plb, precision)
+    L = plb.lib()
+    with a, b:
+        for lat in (a, b):
+            lat.step(0, 130)
+        assert L.plb_step_async(a._h, 130, 41) == 0
+        withhold(plb, a, 1)
+        for call in [(171, 40), (211, 33), (244, 7)]:
+            assert L.plb_step_async(a._h, *call) == 0
+        assert withhold(plb, a, 0) == 0
+        assert L.plb_sync(a._h) == 0
+        for call in [(130, 41), (171, 40), (211, 33), (244, 7)]:
+            b.step(*call)
+        same(a, b)
+
+
+def test_trip_in_a_run_that_gives_up(plb):
+    a, b = pair(plb, 0, 0.51, 0.003)
+    with a, b:
+        a.step_rc(0, 130)
+        a.init_equilibrium()
+        withhold(plb, a, 1)
+        assert a.step_rc(0, 130) == b.step_rc(0, 130) == plb.ERR_DENSITY
+        assert a.last_fault() == b.last_fault()
+        same(a, b)
+
+
+def batch(plb, precision, gx=1e-5):
+    flags = [plb.mask_spheres((30, 32, 34), 3.0, 5.0, 0.5, 4 + k) for k in range(3)]
+    kw = dict(precision=precision, bb_mode=1, fp16_rounding=1, brick=(34, 8, 1), **SHAPE)
+    taus, gxs = [0.8, 0.51, 0.9], [1e-5, gx, 2e-5]
+    return plb.Batch(flags, taus, gxs, **kw), plb.Batch(flags, taus, gxs, **kw)
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2])
+def test_batch_that_gives_up(plb, precision):
+    a, b = batch(plb, precision)
+    withhold(plb, a, 5)
+    ra, rb = a.run(150, 50, 0.0), b.run(150, 15, 0.0)
+    assert withhold(plb, a, 5) == 4        # one launch gave up, and the run was not tried on chip again
+    assert np.array_equal(ra[0], rb[0]) and ra[1] == rb[1]
+    for s in range(3):
+        assert np.array_equal(a.read_macros(s), b.read_macros(s))
+    assert a.reduce() == b.reduce()
+    a.run(150, 50, 0.0)
+    assert withhold(plb, a, 0) == 5        # nor was the next one
+    a.close()
+    b.close()
+
+
+def test_batch_that_gives_up_and_trips(plb):
+    """The density guard trips in the launch that gives up: it still counts as one."""
+    a, b = batch(plb, 0, 0.03)
+    withhold(plb, a, 5)
+    for x, every in ((a, 50), (b, 10)):
+        with pytest.raises(plb.PlbError) as e:
+            x.run(150, every, 0.0)
+        assert e.value.code == plb.ERR_DENSITY
+    assert a.last_fault() == b.last_fault() and a.last_fault()[0] == 1
+    assert withhold(plb, a, 5) == 4
+    with pytest.raises(plb.PlbError):
+        a.run(150, 50, 0.0)
+    assert withhold(plb, a, 0) == 5
+    a.close()
+    b.close()
