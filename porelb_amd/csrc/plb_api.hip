@@ -330,8 +330,8 @@ static int settle(plb_ctx* c, unsigned long long* key)
         while (k < c->segs.size() && !(c->segs[k].serial && (c->segs[k].serial == gave_up || trips(c->segs[k])))) k++;
     if (*key != NO_FAULT && k < c->segs.size()) {
         if (gave_up != NO_FAULT) {
-            fprintf(stderr, "libplb: an on-chip run's blocks were not all resident; this lattice goes on with one launch per step\n");
-            c->chip_state = -1;
+            rc = onchip_gave_up(c);
+            if (rc) return rc;
         }
         PLB_HIP(hipMemsetAsync(c->fault, 0xff, 2 * sizeof(unsigned long long), c->stream));
         c->cur = c->segs[k].cur;

@@ -267,7 +267,7 @@ extern "C" int64_t plb_batch_num_nodes(const plb_batch* b, int s)
 // Whether the run's samples that fit run on chip (and builds the plan).
 static bool batch_on_chip(plb_batch* b, int64_t max_steps, int64_t check_every)
 {
-    return check_every >= 16 && onchip_batch_ready(b->c, b->off, b->n, b->nx, b->ny, b->nz, max_steps);
+    return check_every >= 16 && !onchip_resting(b->c, max_steps) && onchip_batch_ready(b->c, b->off, b->n, b->nx, b->ny, b->nz, max_steps);
 }
 
 // The blocks of the active samples; with `chip`, the samples that have an
@@ -378,9 +378,11 @@ static int batch_run(plb_batch* b, int64_t max_steps, int64_t check_every, doubl
         PLB_HIP(hipStreamSynchronize(c->stream));
         if (words[0] != NO_FAULT) {
             *again = chip;
-            // Blocks that were not all resident: not tried again.  (Such a launch goes on
-            // to the end of its step, where it may record a trip as well.)
-            if (words[1] != NO_FAULT) c->chip_state = -1;
+            // (A launch that gives up goes on to the end of its step, where it may record a trip as well.)
+            if (words[1] != NO_FAULT) {
+                rc = onchip_gave_up(c);
+                if (rc) return rc;
+            }
             return PLB_ERR_DENSITY;
         }
         bool changed = false;

@@ -274,6 +274,8 @@ struct plb_ctx {
     plb::OnchipPlan* chip = nullptr;
     int chip_state = 0;         // 0: no plan yet, 1: plan ready, -1: not used for this lattice
     int64_t chip_steps = 0;     // steps asked for in calls long enough for the on-chip run
+    int64_t chip_rest = 0;      // of these steps, how many take one launch each before the next try
+    int64_t chip_pause = 16384; // chip_rest after the next run that gives up
     int chip_withhold = 0;      // tests: runs to launch without their last block
 };
 
@@ -382,6 +384,8 @@ bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::
 int onchip_blocks(const plb_ctx* c, int sample, int* block0);
 void onchip_pack(const std::vector<int>& blocks, int cus, std::vector<std::vector<int>>* launches);
 int onchip_clear(plb_ctx* c);
+int onchip_gave_up(plb_ctx* c);
+bool onchip_resting(plb_ctx* c, int64_t nsteps);
 int launch_onchip_batch(plb_ctx* c, int64_t it0, int64_t n, const int32_t* list, int blocks, const double* omega,
                         const double* gx);
 void onchip_batch_next(plb_ctx* c, int64_t n);

@@ -1077,6 +1077,27 @@ static int plan_single(plb_ctx* c)
     return build_onchip(c, samples, smp.nblocks, NS);
 }
 
+// A run gave up: some of its blocks did not start within 50 ms, because other
+// work kept the CUs.  Launches per step take over for a while, twice as long after
+// each time, so that a busy chip costs a few waits (16 384 steps of a small lattice,
+// 70 ms, take about as long as one) and a chip that is free again is used.
+int onchip_gave_up(plb_ctx* c)
+{
+    fprintf(stderr, "libplb: an on-chip run's blocks were not all resident; the next %lld steps go with one launch per step\n",
+            (long long)c->chip_pause);
+    c->chip_rest = c->chip_pause;
+    c->chip_pause *= c->chip_pause < ((int64_t)1 << 60) ? 2 : 1;
+    return onchip_clear(c);
+}
+
+// Whether a call of nsteps steps falls into such a while.
+bool onchip_resting(plb_ctx* c, int64_t nsteps)
+{
+    if (c->chip_rest <= 0) return false;
+    c->chip_rest -= nsteps;
+    return true;
+}
+
 // Whether this call of nsteps steps runs on chip; builds the plan when it pays.
 bool onchip_ready(plb_ctx* c, int64_t nsteps)
 {
@@ -1096,7 +1117,7 @@ bool onchip_ready(plb_ctx* c, int64_t nsteps)
         }
         c->chip_state = rc ? -1 : 1;
     }
-    return c->chip_state == 1;
+    return c->chip_state == 1 && !onchip_resting(c, nsteps);
 }
 
 // One launch of `blocks` blocks (list: which) for steps it0 .. it0 + n - 1.

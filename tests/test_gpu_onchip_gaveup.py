@@ -98,3 +98,66 @@ def test_batch_that_gives_up_and_trips(plb):
     assert withhold(plb, a, 0) == 5
     a.close()
     b.close()
+
+
+def test_chip_is_tried_again(plb):
+    """After a run that gave up, 16 384 steps with one launch each and then the chip
+    again; after the next one, twice as many."""
+    a, b = pair(plb, 1)
+    with a, b:
+        it = 0
+
+        def steps(n, call=512):
+            nonlocal it
+            for end in range(it + call, it + n + 1, call):
+                a.step(it, call)
+                it = end
+
+        steps(160, 160)
+        for pause in (16384, 32768):
+            withhold(plb, a, 1)
+            steps(64, 64)
+            assert withhold(plb, a, 1) == 0      # gave up
+            steps(pause)
+            assert withhold(plb, a, 0) == 1      # none on chip
+        steps(96, 96)
+        for s in range(0, it, 1000):
+            b.step(s, min(1000, it - s))
+        same(a, b)
+
+
+def test_batch_is_tried_again(plb):
+    a, b = batch(plb, 1)
+    withhold(plb, a, 5)
+    a.run(150, 50, 0.0)
+    withhold(plb, a, 5)
+    a.run(16384, 1000, 0.0)
+    assert withhold(plb, a, 5) == 5
+    a.run(150, 50, 0.0)
+    assert withhold(plb, a, 0) == 4
+    b.run(150, 15, 0.0)
+    assert a.reduce() == b.reduce()
+    a.close()
+    b.close()
+
+
+def test_lattices_on_chip_at_the_same_time(plb):
+    """Three threads with a lattice that fills the chip each, and a fourth with one
+    that does not fit it: whatever of them gives up, the results are those of each alone."""
+    flags = [plb.mask_noise((64, 64, 64), 2.0, 0.35, k) for k in range(3)] + [plb.mask_noise((128, 128, 128), 2.0, 0.4, 9)]
+
+    def work(k):
+        kw = dict(tau=0.8, gx=1e-5, precision=k % 2, bb_mode=1, brick=(flags[k].shape[2], 8, 1), **SHAPE)
+        with plb.Lattice.from_flag(flags[k], **kw) as lat:
+            for it in range(0, 2000, 200):
+                lat.step(it, 200)
+            return lat.read_state(), lat.read_macros()
+
+    alone, shared = [work(k) for k in range(4)], [None] * 4
+    threads = [threading.Thread(target=lambda k=k: shared.__setitem__(k, work(k))) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for one, other in zip(alone, shared):
+        assert np.array_equal(one[0], other[0]) and np.array_equal(one[1], other[1])
