@@ -140,13 +140,21 @@ struct Lease {
     }
 };
 
-bool page_locked(const void* p)
+// What the runtime knows of p; pageable memory it does not know.
+static hipPointerAttribute_t attributes(const void* p)
 {
-    hipPointerAttribute_t a;
+    hipPointerAttribute_t a = {};
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError();
-        return false;
+        a = {};
+        a.type = hipMemoryTypeUnregistered;
     }
+    return a;
+}
+
+bool page_locked(const void* p)
+{
+    const hipPointerAttribute_t a = attributes(p);
     return a.type == hipMemoryTypeHost && a.devicePointer == a.hostPointer;  // kernels take the pointer as it is
 }
 
@@ -208,10 +216,15 @@ static int move(int device, hipStream_t s, int64_t n, size_t item, const std::ve
 {
     const size_t row = item * arrays.size(), bytes = row * (size_t)n;
     if (bytes == 0) return PLB_OK;
-    bool locked = true;
-    for (const char* a : arrays) locked = locked && page_locked(a);
+    // Threads move host memory, if any of it is pageable; device and managed memory is left to the runtime's copies.
+    bool host = true, locked = true;
+    for (const char* a : arrays) {
+        const hipMemoryType type = attributes(a).type;
+        locked = locked && type == hipMemoryTypeHost;
+        host = host && (type == hipMemoryTypeHost || type == hipMemoryTypeUnregistered);
+    }
     Lease lease;
-    bool threaded = !locked && bytes >= (slots_are_kept() ? THREADED : THREADED_ALONE);
+    bool threaded = host && !locked && bytes >= (slots_are_kept() ? THREADED : THREADED_ALONE);
     if (threaded && lease.take(device) != hipSuccess) threaded = false;
 
     int rc = PLB_OK;

@@ -124,3 +124,45 @@ def test_order_and_table_of_large_masks(nx):
             lat.step(0, 5)
             out.append((table, lat.read_state()))
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("managed", [False, True])
+@pytest.mark.parametrize("nbytes", [1 * MB, 3 * MB + 152, 20 * MB])
+def test_device_and_managed_memory(nbytes, managed):
+    """Arrays that are not host memory, on both sides of the size from which threads move host memory."""
+    L = P.lib()
+    hip = ctypes.CDLL("libamdhip64.so")     # the one libplb.so has loaded
+    hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+    with lattice(nbytes // 152, precision=P.FP64) as lat:
+        want = state(lat, 5)
+        p, size = ctypes.c_void_p(), ctypes.c_size_t(want.nbytes)
+        assert (hip.hipMallocManaged(ctypes.byref(p), size, 1) if managed else hip.hipMalloc(ctypes.byref(p), size)) == 0
+
+        def back(n):
+            out = np.zeros(n)
+            assert hip.hipMemcpy(out.ctypes.data, p, out.nbytes, 4) == 0
+            return out
+
+        lat.write_state(want)
+        assert L.plb_read_state(lat._h, p) == 0
+        assert np.array_equal(back(want.size).reshape(want.shape), want)
+        lat.init_equilibrium()
+        assert L.plb_write_state(lat._h, p) == 0
+        assert np.array_equal(lat.read_state(), want)
+        lat.step(0, 3)
+        assert L.plb_read_populations(lat._h, p) == 0
+        assert np.array_equal(back(want.size).reshape(want.shape), lat.read_populations())
+        macros = lat.read_macros()
+        parts = [ctypes.c_void_p(p.value + 8 * lat.N * q) for q in range(4)]
+        assert L.plb_read_macros(lat._h, *parts) == 0
+        assert np.array_equal(back(4 * lat.N).reshape(4, lat.N), macros)
+        hip.hipFree(p)
+
+
+def test_some_arrays_page_locked():
+    with lattice(300_000, precision=P.FP32) as lat:
+        lat.step(0, 3)
+        want = lat.read_macros()
+        out = [np.zeros(lat.N), P.host_array(lat.N), np.zeros(lat.N), P.host_array(lat.N)]
+        assert P.lib().plb_read_macros(lat._h, *[ctypes.c_void_p(o.ctypes.data) for o in out]) == 0
+        assert all(np.array_equal(o, w) for o, w in zip(out, want))
