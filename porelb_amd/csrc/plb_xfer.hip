@@ -55,11 +55,14 @@ static int contexts = 0;
 static void staging_free(Staging* s)
 {
     if (!s) return;
+    int current = s->device;   // the caller's, which stays
+    (void)hipGetDevice(&current);
     (void)hipSetDevice(s->device);
     if (s->host) (void)hipHostFree(s->host);
     dev_free(s->dev);
     for (hipEvent_t e : s->copied)
         if (e) (void)hipEventDestroy(e);
+    (void)hipSetDevice(current);
     delete s;
 }
 

@@ -1,0 +1,96 @@
+// The transfer slots and the kept device blocks (plb_xfer.hip, plb_mem.hip) on a
+// HIP runtime made of malloc: two devices, immediate copies.  Built and run by
+// tests/test_host_memory.py under the address sanitizer; argv[1] names the check.
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <map>
+#include <vector>
+
+#include "plb_xfer.hpp"
+
+static int current = 0, fails = 0;
+static size_t on_device = 0, locked_bytes = 0;
+static std::map<void*, size_t>* sizes = new std::map<void*, size_t>();   // outlives every static object
+
+#define CHECK(c)                                                               \
+    do {                                                                       \
+        if (!(c)) {                                                            \
+            fprintf(stderr, "check failed: %s (line %d)\n", #c, __LINE__);     \
+            fails++;                                                           \
+        }                                                                      \
+    } while (0)
+
+extern "C" {
+hipError_t hipGetDevice(int* d) { *d = current; return hipSuccess; }
+hipError_t hipSetDevice(int d) { current = d; return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipMalloc(void** p, size_t n)
+{
+    *p = malloc(n);
+    (*sizes)[*p] = n;
+    on_device += n;
+    return hipSuccess;
+}
+hipError_t hipFree(void* p)
+{
+    on_device -= (*sizes)[p];
+    sizes->erase(p);
+    free(p);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { locked_bytes += n; (*sizes)[*p = malloc(n)] = n; return hipSuccess; }
+hipError_t hipHostFree(void* p) { locked_bytes -= (*sizes)[p]; sizes->erase(p); free(p); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = (hipEvent_t)malloc(1); return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { free(e); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t*, const void*) { return hipErrorInvalidValue; }
+const char* hipGetErrorString(hipError_t) { return ""; }
+}
+void plb_set_hip_error(hipError_t, const char*, const char*, int) {}
+
+using namespace plb;
+
+constexpr size_t MB = (size_t)1 << 20;
+
+static void transfer(int device)
+{
+    std::vector<char> array(8 * MB);
+    hipSetDevice(device);
+    CHECK(download(device, nullptr, (int64_t)array.size(), 1, {array.data()}, [](int64_t, int64_t m, void* d) {
+              memset(d, 7, m);
+              return PLB_OK;
+          }) == PLB_OK);
+    CHECK(array.front() == 7 && array.back() == 7);
+}
+
+// The slots of another device go without a change of the caller's current one.
+static void device()
+{
+    xfer_context(1);
+    xfer_context(1);
+    transfer(0);
+    transfer(1);
+    CHECK(locked_bytes == 32 * MB);
+    for (int left : {1, 0}) {
+        hipSetDevice(0);
+        xfer_context(-1);
+        CHECK(current == 0);
+        CHECK(locked_bytes == (left ? 32 * MB : 0));
+    }
+    // a set that lasts for one call
+    transfer(0);
+    CHECK(current == 0 && locked_bytes == 0);
+}
+
+int main(int argc, char** argv)
+{
+    const char* what = argc > 1 ? argv[1] : "";
+    if (!strcmp(what, "device")) device();
+    else return 2;
+    return fails ? 1 : 0;
+}
