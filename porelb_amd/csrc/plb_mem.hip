@@ -25,18 +25,27 @@ struct Block {
     size_t size;
     int device;
 };
-static std::mutex mutex;
-static std::vector<Block> kept;                       // oldest first
-static std::unordered_map<void*, Block>* live = nullptr;  // never destroyed: owners may outlive static objects
-static size_t kept_bytes = 0;
+// Never destroyed: owners may outlive static objects.
+struct Pool {
+    std::mutex mutex;
+    std::vector<Block> kept;                   // oldest first
+    std::unordered_map<void*, Block> live;
+    size_t kept_bytes = 0;
+};
+static Pool& pool()
+{
+    static Pool* const p = new Pool();
+    return *p;
+}
 
 static void give_back_all()
 {
+    Pool& o = pool();
     std::vector<Block> gone;
     {
-        std::lock_guard<std::mutex> lock(mutex);
-        gone.swap(kept);
-        kept_bytes = 0;
+        std::lock_guard<std::mutex> lock(o.mutex);
+        gone.swap(o.kept);
+        o.kept_bytes = 0;
     }
     for (const Block& b : gone) (void)hipFree(b.p);
 }
@@ -56,8 +65,10 @@ hipError_t dev_alloc(void** p, size_t bytes)
     Block b = {nullptr, (bytes + MB - 1) / MB * MB, 0};
     hipError_t e = hipGetDevice(&b.device);
     if (e != hipSuccess) return e;
+    Pool& o = pool();
     {
-        std::lock_guard<std::mutex> lock(mutex);
+        std::lock_guard<std::mutex> lock(o.mutex);
+        std::vector<Block>& kept = o.kept;
         size_t best = kept.size();
         for (size_t k = 0; k < kept.size(); k++)
             if (kept[k].device == b.device && kept[k].size >= b.size && kept[k].size <= b.size + b.size / 2 &&
@@ -66,16 +77,15 @@ hipError_t dev_alloc(void** p, size_t bytes)
         if (best < kept.size()) {
             b = kept[best];
             kept.erase(kept.begin() + best);
-            kept_bytes -= b.size;
+            o.kept_bytes -= b.size;
         }
     }
     if (!b.p) {
         e = allocate(&b.p, b.size);
         if (e != hipSuccess) return e;
     }
-    std::lock_guard<std::mutex> lock(mutex);
-    if (!live) live = new std::unordered_map<void*, Block>();
-    (*live)[b.p] = b;
+    std::lock_guard<std::mutex> lock(o.mutex);
+    o.live[b.p] = b;
     *p = b.p;
     return hipSuccess;
 }
@@ -83,20 +93,21 @@ hipError_t dev_alloc(void** p, size_t bytes)
 void dev_free(void* p)
 {
     if (!p) return;
+    Pool& o = pool();
     std::vector<Block> gone;
     {
-        std::lock_guard<std::mutex> lock(mutex);
-        const auto it = live ? live->find(p) : std::unordered_map<void*, Block>::iterator();
-        if (!live || it == live->end()) {
+        std::lock_guard<std::mutex> lock(o.mutex);
+        const auto it = o.live.find(p);
+        if (it == o.live.end()) {
             gone.push_back({p, 0, 0});
         } else {
-            kept.push_back(it->second);
-            kept_bytes += it->second.size;
-            live->erase(it);
-            while (kept_bytes > KEEP_MOST) {
-                kept_bytes -= kept.front().size;
-                gone.push_back(kept.front());
-                kept.erase(kept.begin());
+            o.kept.push_back(it->second);
+            o.kept_bytes += it->second.size;
+            o.live.erase(it);
+            while (o.kept_bytes > KEEP_MOST) {
+                o.kept_bytes -= o.kept.front().size;
+                gone.push_back(o.kept.front());
+                o.kept.erase(o.kept.begin());
             }
         }
     }

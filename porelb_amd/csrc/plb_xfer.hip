@@ -48,9 +48,17 @@ struct Staging {
     bool busy = true;
 };
 
-static std::mutex pool_mutex;
-static std::vector<Staging*> pool;
-static int contexts = 0;
+// Never destroyed: a context may outlive static objects.
+struct Kept {
+    std::mutex mutex;
+    std::vector<Staging*> pool;
+    int contexts = 0;
+};
+static Kept& kept()
+{
+    static Kept* const k = new Kept();
+    return *k;
+}
 
 static void staging_free(Staging* s)
 {
@@ -68,15 +76,16 @@ static void staging_free(Staging* s)
 
 void xfer_context(int add)
 {
+    Kept& o = kept();
     std::vector<Staging*> gone;
     {
-        std::lock_guard<std::mutex> lock(pool_mutex);
-        contexts += add;
-        if (contexts > 0) return;
-        for (size_t k = 0; k < pool.size();)
-            if (!pool[k]->busy) {
-                gone.push_back(pool[k]);
-                pool.erase(pool.begin() + k);
+        std::lock_guard<std::mutex> lock(o.mutex);
+        o.contexts += add;
+        if (o.contexts > 0) return;
+        for (size_t k = 0; k < o.pool.size();)
+            if (!o.pool[k]->busy) {
+                gone.push_back(o.pool[k]);
+                o.pool.erase(o.pool.begin() + k);
             } else {
                 k++;
             }
@@ -86,8 +95,8 @@ void xfer_context(int add)
 
 static bool slots_are_kept()
 {
-    std::lock_guard<std::mutex> lock(pool_mutex);
-    return contexts > 0;
+    std::lock_guard<std::mutex> lock(kept().mutex);
+    return kept().contexts > 0;
 }
 
 static hipError_t staging_new(int device, Staging** out)
@@ -111,9 +120,10 @@ struct Lease {
     Staging* s = nullptr;
     hipError_t take(int device)
     {
+        Kept& o = kept();
         {
-            std::lock_guard<std::mutex> lock(pool_mutex);
-            for (Staging* p : pool)
+            std::lock_guard<std::mutex> lock(o.mutex);
+            for (Staging* p : o.pool)
                 if (!p->busy && p->device == device) {
                     p->busy = true;
                     s = p;
@@ -122,21 +132,22 @@ struct Lease {
         }
         const hipError_t e = staging_new(device, &s);
         if (e != hipSuccess) return e;
-        std::lock_guard<std::mutex> lock(pool_mutex);
-        if ((int)pool.size() < MAX_KEPT) pool.push_back(s);
+        std::lock_guard<std::mutex> lock(o.mutex);
+        if ((int)o.pool.size() < MAX_KEPT) o.pool.push_back(s);
         return hipSuccess;
     }
     ~Lease()
     {
         if (!s) return;
+        Kept& o = kept();
         Staging* gone = s;
         {
-            std::lock_guard<std::mutex> lock(pool_mutex);
+            std::lock_guard<std::mutex> lock(o.mutex);
             s->busy = false;
-            const auto it = std::find(pool.begin(), pool.end(), s);
-            if (it != pool.end()) {
-                if (contexts > 0) gone = nullptr;
-                else pool.erase(it);
+            const auto it = std::find(o.pool.begin(), o.pool.end(), s);
+            if (it != o.pool.end()) {
+                if (o.contexts > 0) gone = nullptr;
+                else o.pool.erase(it);
             }
         }
         staging_free(gone);

@@ -87,10 +87,39 @@ static void device()
     CHECK(current == 0 && locked_bytes == 0);
 }
 
+// An object of the caller's with static storage may go after the library's own static objects.
+struct Late {
+    std::vector<void*> blocks;
+    bool counted = false;
+    ~Late()
+    {
+        if (!counted) return;
+        for (void* p : blocks) dev_free(p);
+        void* p = nullptr;
+        if (dev_alloc(&p, 3 * MB) == hipSuccess) dev_free(p);
+        transfer(0);
+        xfer_context(-1);
+        if (fails) _Exit(1);
+    }
+};
+static Late late;   // made before the library's static objects: its source comes first on the command line
+
+static void at_exit()
+{
+    xfer_context(1);
+    transfer(0);
+    late.counted = true;
+    late.blocks.resize(5);
+    for (void*& p : late.blocks) CHECK(dev_alloc(&p, 2 * MB) == hipSuccess);
+    dev_free(late.blocks.back());
+    late.blocks.pop_back();
+}
+
 int main(int argc, char** argv)
 {
     const char* what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "device")) device();
+    else if (!strcmp(what, "at_exit")) at_exit();
     else return 2;
     return fails ? 1 : 0;
 }
