@@ -281,6 +281,13 @@ const char *plb_strerror(int code);
 void *plb_host_alloc(size_t bytes);
 void plb_host_free(void *p);
 
+/* What is kept from one call or context to the next and not in use goes back to
+ * the system: device blocks of 1 to 128 MB, 256 MB in all, which stay after the
+ * last context for the next one, and up to four sets of transfer slots (16 MB
+ * of page-locked and of device memory each), which otherwise go with it.  For
+ * programs that need the memory elsewhere; any thread, any time. */
+void plb_release_memory(void);
+
 /* plb_read_macros for the V-order nodes [first, first + n) without any
  * device allocation.  No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under HIP graph capture, serving loops,

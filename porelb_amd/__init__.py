@@ -119,6 +119,7 @@ def _lib():
             "plb_strerror": ([i32], C.c_char_p),
             "plb_host_alloc": ([C.c_size_t], C.c_void_p),
             "plb_host_free": ([C.c_void_p], None),
+            "plb_release_memory": ([], None),
             "plb_preprocess": ([p, i32, i32, i32, i32, i32, p, p, p], i32),
             "plb_batch_create": ([p, p, p, i32], i32),
             "plb_batch_run": ([p, i64, i64, d, p, p, p], i32),
@@ -226,6 +227,11 @@ def host_array(shape, dtype=np.float64):
     raw = (C.c_char * max(nbytes, 1)).from_address(p)
     weakref.finalize(raw, _lib().plb_host_free, p)
     return np.frombuffer(raw, dtype=dtype, count=int(np.prod(shape))).reshape(shape)
+
+
+def release_memory():
+    """Device blocks and transfer slots that are kept for later calls go back to the system."""
+    _lib().plb_release_memory()
 
 
 # ------------------------------------------------------------------ lattice

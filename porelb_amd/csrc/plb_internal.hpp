@@ -109,6 +109,7 @@ namespace plb {
 // dev_free: the work that uses the block has been waited for.
 hipError_t dev_alloc(void** p, size_t bytes);
 void dev_free(void* p);
+void dev_give_back();   // all kept blocks
 
 // Device memory with one owner.  reserve() takes one block that take() cuts
 // pieces from; what does not fit, or comes without a reserve, gets an

@@ -74,14 +74,13 @@ static void staging_free(Staging* s)
     delete s;
 }
 
-void xfer_context(int add)
+// Frees the sets that no call uses.
+static void free_idle()
 {
     Kept& o = kept();
     std::vector<Staging*> gone;
     {
         std::lock_guard<std::mutex> lock(o.mutex);
-        o.contexts += add;
-        if (o.contexts > 0) return;
         for (size_t k = 0; k < o.pool.size();)
             if (!o.pool[k]->busy) {
                 gone.push_back(o.pool[k]);
@@ -91,6 +90,16 @@ void xfer_context(int add)
             }
     }
     for (Staging* s : gone) staging_free(s);
+}
+
+void xfer_context(int add)
+{
+    {
+        std::lock_guard<std::mutex> lock(kept().mutex);
+        kept().contexts += add;
+        if (kept().contexts > 0) return;
+    }
+    free_idle();
 }
 
 static bool slots_are_kept()
@@ -332,6 +341,12 @@ static int move(int device, hipStream_t s, int64_t n, size_t item, const std::ve
     const hipError_t e = hipStreamSynchronize(s);  // the slots are free again, also after an error
     if (!rc) check(e);
     return rc;
+}
+
+extern "C" void plb_release_memory(void)
+{
+    free_idle();
+    dev_give_back();
 }
 
 int download(int device, hipStream_t s, int64_t n, size_t item, const std::vector<char*>& arrays,

@@ -11,7 +11,7 @@
 #include "plb_xfer.hpp"
 
 static int current = 0, fails = 0;
-static size_t on_device = 0, locked_bytes = 0;
+static size_t on_device = 0, locked_bytes = 0, capacity = ~(size_t)0;
 static std::map<void*, size_t>* sizes = new std::map<void*, size_t>();   // outlives every static object
 
 #define CHECK(c)                                                               \
@@ -28,6 +28,7 @@ hipError_t hipSetDevice(int d) { current = d; return hipSuccess; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipMalloc(void** p, size_t n)
 {
+    if (n > capacity || on_device > capacity - n) return hipErrorOutOfMemory;
     *p = malloc(n);
     (*sizes)[*p] = n;
     on_device += n;
@@ -87,6 +88,39 @@ static void device()
     CHECK(current == 0 && locked_bytes == 0);
 }
 
+// Kept blocks: 256 MB at most, for the next owner, and back to the system on request or when there is no more.
+static void release()
+{
+    std::vector<void*> p(10);
+    for (void*& q : p) CHECK(dev_alloc(&q, 64 * MB) == hipSuccess);
+    CHECK(on_device == 640 * MB);
+    for (void* q : p) dev_free(q);
+    CHECK(on_device == 256 * MB);
+    CHECK(dev_alloc(&p[0], 50 * MB) == hipSuccess && on_device == 256 * MB);
+    plb_release_memory();
+    CHECK(on_device == 64 * MB);   // the one in use
+    dev_free(p[0]);
+    CHECK(on_device == 64 * MB);
+    capacity = 100 * MB;
+    CHECK(dev_alloc(&p[0], 80 * MB) == hipSuccess && on_device == 80 * MB);
+    CHECK(dev_alloc(&p[1], 80 * MB) == hipErrorOutOfMemory);
+    dev_free(p[0]);
+    plb_release_memory();
+    CHECK(on_device == 0);
+    capacity = ~(size_t)0;
+    xfer_context(1);
+    transfer(1);
+    CHECK(locked_bytes == 16 * MB);
+    plb_release_memory();
+    CHECK(locked_bytes == 0 && on_device == 0);
+    transfer(1);
+    CHECK(locked_bytes == 16 * MB);
+    xfer_context(-1);
+    CHECK(locked_bytes == 0);
+    plb_release_memory();
+    CHECK(on_device == 0);
+}
+
 // An object of the caller's with static storage may go after the library's own static objects.
 struct Late {
     std::vector<void*> blocks;
@@ -119,6 +153,7 @@ int main(int argc, char** argv)
 {
     const char* what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "device")) device();
+    else if (!strcmp(what, "release")) release();
     else if (!strcmp(what, "at_exit")) at_exit();
     else return 2;
     return fails ? 1 : 0;

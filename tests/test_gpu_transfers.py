@@ -166,3 +166,27 @@ def test_some_arrays_page_locked():
         out = [np.zeros(lat.N), P.host_array(lat.N), np.zeros(lat.N), P.host_array(lat.N)]
         assert P.lib().plb_read_macros(lat._h, *[ctypes.c_void_p(o.ctypes.data) for o in out]) == 0
         assert all(np.array_equal(o, w) for o, w in zip(out, want))
+
+
+def test_release_memory():
+    """Device blocks that stay after the last lattice go back to the system on request."""
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    def use():
+        with lattice(200_000, precision=P.FP32) as lat:
+            lat.step(0, 200)
+            return lat.read_state()
+
+    want = use()
+    P.release_memory()
+    before = free()
+    assert np.array_equal(use(), want)
+    assert free() < before - 16 * MB      # kept for the next one
+    P.release_memory()
+    assert free() >= before - 4 * MB
+    assert np.array_equal(use(), want)
