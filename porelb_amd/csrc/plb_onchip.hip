@@ -867,27 +867,43 @@ static size_t lds_bytes(const plb_ctx* c, int NS, bool twice)
 // only some waves busy (1 037 nodes: 576 threads took 6.0 to 7.8 us a step, 1024 take 5.0 to 5.5).
 static int slots_for(int nodes) { return nodes > 1024 ? 2048 : (nodes + 63) / 64 * 64; }
 static bool fits_twice(const plb_ctx* c, int NS) { return lds_bytes(c, NS, true) + 64 <= (size_t)c->lds_per_cu; }
-static bool fits(const plb_ctx* c, int nodes)
+// Slots, nodes per thread, threads and copies of a block of up to `nodes` nodes.
+static void shape(const plb_ctx* c, OnchipPlan* p, int nodes)
 {
-    // FP16 blocks of more than 2048 slots (3 nodes per thread, one copy) spill:
-    // 22 us a step for 629 146 nodes, against 16.8 us with one launch per step.
-    const int most = c->cfg.precision == PLB_FP64 ? 1024 : 2048;
-    if (nodes > most) return false;
-    const int NS = slots_for(nodes);
-    if (c->cfg.precision == PLB_FP16 && !fits_twice(c, NS)) return false;
-    return lds_bytes(c, NS, false) + 64 <= (size_t)c->lds_per_cu;
+    p->NS = slots_for(nodes);
+    p->K = nodes > 1024 ? 2 : 1;
+    p->T = p->NS / p->K;
+    p->twice = fits_twice(c, p->NS);
 }
 
+// f(the kernel of a plan); false where there is none of its shape.
 template <typename F>
-static void with_kernel(const plb_ctx* c, const OnchipPlan* p, F f)
+static bool with_kernel(const plb_ctx* c, const OnchipPlan* p, F f)
 {
-    const bool small = p->T <= 512, twice = p->twice;
-    if (c->cfg.precision == PLB_FP64) twice ? f(k_onchip<double, 1, true, 512>) : f(k_onchip<double, 1, false, 1024>);
-    else if (c->cfg.precision == PLB_FP32)
+    const bool small = p->T <= 512, one = p->K == 1, twice = p->twice;
+    if (c->cfg.precision == PLB_FP64) {
+        if (!one || (twice && !small)) return false;
+        twice ? f(k_onchip<double, 1, true, 512>) : f(k_onchip<double, 1, false, 1024>);
+    } else if (c->cfg.precision == PLB_FP32) {
+        if (one != twice) return false;
         !twice ? f(k_onchip<float, 2, false, 1024>)
                : small ? f(k_onchip<float, 1, true, 512>) : f(k_onchip<float, 1, true, 1024>);
-    else if (p->K == 2) f(k_onchip<__half, 2, true, 1024>);
-    else small ? f(k_onchip<__half, 1, true, 512>) : f(k_onchip<__half, 1, true, 1024>);
+    } else {
+        // (Blocks of more than 2048 slots, with 3 nodes per thread and one copy, spill: 22 us a
+        // step for 629 146 nodes, against 16.8 us with one launch per step.)
+        if (!twice) return false;
+        !one ? f(k_onchip<__half, 2, true, 1024>)
+             : small ? f(k_onchip<__half, 1, true, 512>) : f(k_onchip<__half, 1, true, 1024>);
+    }
+    return true;
+}
+
+static bool fits(const plb_ctx* c, int nodes)
+{
+    if (nodes > (c->cfg.precision == PLB_FP64 ? 1024 : 2048)) return false;
+    OnchipPlan p;
+    shape(c, &p, nodes);
+    return with_kernel(c, &p, [](auto*) {}) && lds_bytes(c, p.NS, p.twice) + 64 <= (size_t)c->lds_per_cu;
 }
 
 // Slabs and rows of a sample, so that blocks are about as long as wide.
@@ -911,10 +927,8 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
     c->chip = p;
     hipStream_t s = c->stream;
     p->G = G;
-    p->K = NS > 1024 ? 2 : 1;
-    p->NS = NS = slots_for(NS);
-    p->T = NS / p->K;
-    p->twice = fits_twice(c, NS);
+    shape(c, p, NS);
+    NS = p->NS;
     const int ng = NS / 64;
     const int64_t Ntot = c->N;
     int64_t words = 0, rank = 0;
