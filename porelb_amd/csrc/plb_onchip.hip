@@ -61,7 +61,7 @@ namespace plb {
 // One lattice, or one sample of a batch: its nodes and its share of the blocks.
 struct OnchipSample {
     int64_t off, n;        // internal ids off .. off + n
-    int64_t rank0;         // first rank
+    int64_t rank0;         // its nodes' numbers within the plan, rank0 .. rank0 + n
     int64_t word0, words;  // its bitmask
     int32_t d[3];          // voxels along x, y, z
     int32_t block0, nblocks;
@@ -98,22 +98,25 @@ struct OnchipBox {
     int32_t lo[3], hi[3];
 };
 
+// The plan numbers the nodes of the samples that it holds, one after the other
+// ("number" below; for one lattice, its internal ids), so that its scratch, 230
+// bytes a node, is not taken for a batch's samples that do not fit the chip.
 struct OnchipBuild {
     const OnchipSample* samples;
     int nsamples;
-    int64_t Ntot;               // internal ids, pads between samples included
+    int64_t Ntot;               // numbers
     const uint64_t* xyz;
     const uint32_t* xyz_of;     // xyz is in V order: V id of an internal id (batches); null: by internal id
     const uint32_t* vid;        // V id of an internal id; null: identity
     const uint32_t* node_of_v;  // its inverse
     unsigned long long* bits;
     uint32_t* wpre;
-    uint16_t* group;            // slab, then row, of an internal id within its sample
+    uint16_t* group;            // slab, then row, of a number within its sample
     OnchipBox* box;             // [2][G] of the slabs and the rows
     uint32_t* base;             // [2][G] first bit of each
-    uint32_t* order;            // rank -> internal id
-    uint16_t* blk;              // internal id -> block
-    uint32_t* slot_of;          // internal id -> block * NS + slot
+    uint32_t* order;            // rank -> number
+    uint16_t* blk;              // number -> block
+    uint32_t* slot_of;          // number -> block * NS + slot
     int32_t* T;                 // [18][Ntot] pull sources
     uint32_t* M;                // [18][Ntot] node that pulls population re[j]
     uint32_t* at;               // [18][Ntot] the shared link's entry
@@ -129,10 +132,17 @@ __device__ __forceinline__ int sample_of(const OnchipBuild& b, int64_t k)
     int lo = 0, hi = b.nsamples - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (b.samples[mid].off <= k) lo = mid;
+        if (b.samples[mid].rank0 <= k) lo = mid;
         else hi = mid - 1;
     }
-    return k >= b.samples[lo].off && k < b.samples[lo].off + b.samples[lo].n && b.samples[lo].nblocks > 0 ? lo : -1;
+    return lo;   // the last that starts at k or before: those that the plan does not hold are empty
+}
+__device__ __forceinline__ int64_t id_of(const OnchipSample& s, int64_t k) { return s.off + (k - s.rank0); }
+__device__ __forceinline__ int64_t number_of(const OnchipSample& s, int64_t id) { return s.rank0 + (id - s.off); }
+__device__ __forceinline__ uint64_t coordinates(const OnchipBuild& b, const OnchipSample& s, int64_t k)
+{
+    const int64_t id = id_of(s, k);
+    return b.xyz[b.xyz_of ? (int64_t)b.xyz_of[id] : id];
 }
 
 // Partition.  The nodes are cut by rank, three times: along z into slabs, each
@@ -148,7 +158,7 @@ __device__ __forceinline__ int sample_of(const OnchipBuild& b, int64_t k)
 template <int LEVEL>
 __device__ __forceinline__ int64_t bit_of(const OnchipBuild& b, const OnchipSample& s, int64_t k)
 {
-    const uint64_t p = b.xyz[b.xyz_of ? (int64_t)b.xyz_of[k] : k];
+    const uint64_t p = coordinates(b, s, k);
     const int c[3] = {(int)(p & 0xffff), (int)((p >> 16) & 0xffff), (int)((p >> 32) & 0xffff)};
     if (c[0] >= s.d[0] || c[1] >= s.d[1] || c[2] >= s.d[2]) return -1;
     if constexpr (LEVEL == 0) return s.word0 * 64 + ((int64_t)c[2] * s.d[1] + c[1]) * s.d[0] + c[0];
@@ -168,9 +178,7 @@ __global__ void k_onchip_bits(const OnchipBuild b)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= b.Ntot) return;
-    const int s = sample_of(b, k);
-    if (s < 0) return;
-    const int64_t m = bit_of<LEVEL>(b, b.samples[s], k);
+    const int64_t m = bit_of<LEVEL>(b, b.samples[sample_of(b, k)], k);
     const unsigned long long bit = 1ull << (m & 63);
     // two records with the same coordinates, or some outside the box
     if (m < 0 || (atomicOr(b.bits + (m >> 6), bit) & bit)) *b.err = 1;
@@ -253,9 +261,7 @@ __global__ void k_onchip_rank(const OnchipBuild b)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= b.Ntot) return;
-    const int si = sample_of(b, k);
-    if (si < 0) return;
-    const OnchipSample s = b.samples[si];
+    const OnchipSample s = b.samples[sample_of(b, k)];
     const int64_t m = bit_of<LEVEL>(b, s, k);
     if (m < 0) return;
     const int64_t r = (int64_t)b.wpre[m >> 6] + __popcll(b.bits[m >> 6] & ((1ull << (m & 63)) - 1ull));
@@ -275,7 +281,7 @@ __global__ void k_onchip_rank(const OnchipBuild b)
         // Its box, from its first and its last node; the slab's along z, all of it along x.
         OnchipBox& o = b.box[(int64_t)LEVEL * b.G + s.block0 + g];
         const OnchipBox& slab = b.box[s.block0 + (LEVEL ? b.group[k] : 0)];
-        const uint64_t p = b.xyz[b.xyz_of ? (int64_t)b.xyz_of[k] : k];
+        const uint64_t p = coordinates(b, s, k);
         const int y = (int)((p >> 16) & 0xffff), z = (int)((p >> 32) & 0xffff);
         if (r == s.rank0 || group(r - 1) != g) {
             o.lo[0] = 0;
@@ -295,11 +301,14 @@ template <int LAYOUT, int IDX>
 __global__ void k_onchip_links(const StepArgs a, const OnchipBuild b)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= b.Ntot || sample_of(b, k) < 0) return;
+    if (k >= b.Ntot) return;
+    const OnchipSample& s = b.samples[sample_of(b, k)];
+    const int32_t shift = (int32_t)(s.rank0 - s.off);
     int32_t t[Q];
-    lane_sources<LAYOUT, IDX>(a, k, t);
+    lane_sources<LAYOUT, IDX>(a, id_of(s, k), t);
 #pragma unroll
     for (int j = 1; j < Q; j++) {
+        if (t[j] >= 0) t[j] += shift;
         b.T[(int64_t)(j - 1) * b.Ntot + k] = t[j];
         if (t[j] >= 0 && atomicExch(b.M + (int64_t)(RE[j] - 1) * b.Ntot + t[j], (uint32_t)k) != EMPTY) *b.err = 1;
     }
@@ -338,7 +347,8 @@ __global__ void __launch_bounds__(1024) k_onchip_slots(const OnchipBuild b, int 
                 bool shared = false;
                 int32_t t;
                 for (int j = 1; j < Q; j++) shared |= partner(b, k, j, (uint16_t)blk, t) != EMPTY;
-                v = (b.vid ? b.vid[k] : k) | (shared ? 0u : 0x80000000u);
+                const uint32_t id = (uint32_t)id_of(s, k);
+                v = (b.vid ? b.vid[id] : id) | (shared ? 0u : 0x80000000u);
             }
         }
         key[q] = v;
@@ -386,7 +396,7 @@ __global__ void __launch_bounds__(1024) k_onchip_slots(const OnchipBuild b, int 
             }
         }
         const uint32_t v = key[q] & 0x7fffffffu;
-        const uint32_t k = b.node_of_v ? b.node_of_v[v] : v;
+        const uint32_t k = (uint32_t)number_of(s, b.node_of_v ? b.node_of_v[v] : v);
         b.slot_of[k] = (uint32_t)blk * (uint32_t)b.NS + (uint32_t)slot;
         b.node[(int64_t)blk * b.NS + slot] = k;
     }
@@ -492,10 +502,12 @@ __global__ void __launch_bounds__(256) k_onchip_groups(const OnchipBuild b)
 }
 
 // The partner's entry is the other end of the same link: direction re[j] at
-// the partner node, and re[j] is the direction of the entry's LDS cell.
-__global__ void k_onchip_dst(const OnchipBuild b, int64_t E)
+// the partner node, and re[j] is the direction of the entry's LDS cell.  The
+// slots get their nodes' internal ids in place of the numbers.
+__global__ void k_onchip_dst(const OnchipBuild b, int64_t E, int64_t slots)
 {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < slots && b.node[e] != EMPTY) b.node[e] = (uint32_t)id_of(b.samples[b.block_sample[e / b.NS]], b.node[e]);
     if (e >= E) return;
     const uint32_t cell = b.ent_lds[e] & 0xffffu;
     if (cell < (uint32_t)b.NS * Q) b.ent_dst[e] = b.at[(int64_t)(cell % Q - 1) * b.Ntot + b.ent_dst[e]];
@@ -930,7 +942,6 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
     shape(c, p, NS);
     NS = p->NS;
     const int ng = NS / 64;
-    const int64_t Ntot = c->N;
     int64_t words = 0, rank = 0;
     std::vector<int32_t> block_sample(G);
     for (size_t k = 0; k < samples.size(); k++) {
@@ -944,6 +955,7 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
         for (int q = 0; q < smp.nblocks; q++) block_sample[smp.block0 + q] = (int32_t)k;
     }
     p->samples = samples;
+    const int64_t Ntot = rank;
     // arrays of the plan
     const int64_t slots = (int64_t)G * NS, groups = (int64_t)G * ng;
     PLB_HIP(dev_alloc(&p->fixed, sizeof(uint32_t) * (slots * 10 + groups + 1 + G)));
@@ -1055,7 +1067,7 @@ static int build_onchip(plb_ctx* c, std::vector<OnchipSample> samples, int G, in
         PLB_HIP(hipMemsetAsync(p->recv, 0, p->recv_bytes, s));
     }
     hipLaunchKernelGGL(k_onchip_groups<1>, dim3(nblk(groups, 4)), t256, 0, s, b);
-    if (E) hipLaunchKernelGGL(k_onchip_dst, dim3(nblk(E, 256)), t256, 0, s, b, (int64_t)E);
+    hipLaunchKernelGGL(k_onchip_dst, dim3(nblk(std::max<int64_t>(E, slots), 256)), t256, 0, s, b, (int64_t)E, slots);
     PLB_HIP(hipGetLastError());
     if (!batch) {
         PLB_HIP(dev_alloc((void**)&p->macros_own, sizeof(double) * 4 * c->Npad));

@@ -6,7 +6,14 @@ namespace plb {
 
 // Named by the host code, never called here.
 StepArgs make_args(plb_ctx*, int64_t, bool) { return StepArgs(); }
-hipError_t dev_alloc(void**, size_t) { return hipErrorOutOfMemory; }
+static std::vector<size_t> asked;
+hipError_t dev_alloc(void** p, size_t n)
+{
+    asked.push_back(n);
+    if (asked.size() > 1) return hipErrorOutOfMemory;   // the plan's own arrays, then its scratch
+    *p = malloc(64);
+    return hipSuccess;
+}
 void dev_free(void*) {}
 
 struct Kernel {
@@ -48,6 +55,31 @@ static int run()
                     fprintf(stderr, "precision %d, %d KB, %d nodes: K %d, T %d, NS %d, twice %d\n", precision, kb, nodes, p.K, p.T, p.NS, (int)p.twice);
             }
         }
+    // A plan's scratch does not grow with samples that do not fit the chip.
+    size_t scratch[2];
+    for (int with = 0; with < 2; with++) {
+        plb_ctx b;
+        b.cfg.precision = PLB_FP32;
+        b.elem = 4;
+        b.lds_per_cu = 160 * 1024;
+        std::vector<OnchipSample> samples(1 + with);
+        samples[0].n = 20000;
+        samples[0].nblocks = 20;
+        for (OnchipSample& s : samples) s.d[0] = s.d[1] = s.d[2] = 30;
+        if (with) {
+            samples[1].off = 20032;
+            samples[1].n = 100000000;
+            samples[1].block0 = 20;
+        }
+        b.N = samples.back().off + samples.back().n;
+        asked.clear();
+        build_onchip(&b, samples, 20, 1024);
+        scratch[with] = asked.size() == 2 ? asked[1] : 0;
+    }
+    if (!scratch[0] || scratch[1] > scratch[0] + 4096) {
+        fprintf(stderr, "scratch: %zu bytes, with a large sample beside it %zu\n", scratch[0], scratch[1]);
+        fails++;
+    }
     printf("%d plans, %d failed\n", plans, fails);
     return fails || !plans;
 }

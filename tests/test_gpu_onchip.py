@@ -165,3 +165,20 @@ def test_batch_stops_and_trips(plb):
     assert a.last_fault() == b.last_fault() and a.last_fault()[0] == 2
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("large", [0, 1, 3])
+def test_batch_with_a_sample_off_chip(plb, large):
+    """Samples on chip before, between and behind one that is too large for it:
+    the plan numbers its own samples' nodes only."""
+    flags = [mask_of(n, d, k) for k, (n, d) in enumerate([(3000, (20, 21, 22)), (40001, (41, 42, 43)), (700, (9, 70, 8))])]
+    flags.insert(large, mask_of(560_003, (100, 101, 102), 7))
+    taus, gxs = [0.6 + 0.1 * k for k in range(4)], [10.0 ** -(5 + 0.2 * k) for k in range(4)]
+    kw = dict(precision=1, bb_mode=large % 2, block_size=128, brick=(1, 16, 1), **SHAPE)
+    a, b = plb.Batch(flags, taus, gxs, **kw), plb.Batch(flags, taus, gxs, **kw)
+    ra, rb = a.run(140, 70, 0.0), b.run(140, 14, 0.0)
+    assert np.array_equal(ra[0], rb[0]) and ra[1] == rb[1]
+    assert all(np.array_equal(a.read_macros(s), b.read_macros(s)) for s in range(4))
+    assert a.reduce() == b.reduce()
+    a.close()
+    b.close()
