@@ -401,10 +401,10 @@ __global__ void k_brick_bits(const uint64_t* __restrict__ xyz, int64_t N, BrickA
 
 // The same bits where the mask is at hand: every word gathers its 64 voxels, so
 // there is no atomic per node (265 421 nodes: 19 us with atomics).
-__global__ void k_brick_words(const uint64_t* __restrict__ flag_bits, BrickArgs b, int64_t nvb, uint64_t* __restrict__ bits,
-                              uint64_t* __restrict__ cnt)
+__global__ void k_brick_words(const uint64_t* __restrict__ flag_bits, BrickArgs b, int64_t nvb, int64_t first,
+                              uint64_t* __restrict__ bits, uint64_t* __restrict__ cnt)
 {
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t v = first + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     bool pore = false;
     if (v < nvb) {
         const int64_t vol = (int64_t)b.bx * b.by * b.bz;
@@ -511,7 +511,11 @@ int compute_order(const plb_config& cfg, int nx, int ny, int nz, int64_t N, cons
     PLB_HIP(cnt.alloc(nw, scratch));
     PLB_HIP(wpre.alloc(nw, scratch));
     if (flag_bits) {
-        hipLaunchKernelGGL(k_brick_words, dim3(nblk(nw * 64, 256)), dim3(256), 0, s, flag_bits, b, nvb, bits.p, cnt.p);
+        // A launch has less than 2^32 threads, and bricks that stand out past the mask may make more voxels than that.
+        constexpr int64_t MOST = (int64_t)1 << 31;
+        for (int64_t first = 0; first < nw * 64; first += MOST)
+            hipLaunchKernelGGL(k_brick_words, dim3(nblk(std::min(MOST, nw * 64 - first), 256)), dim3(256), 0, s, flag_bits, b,
+                               nvb, first, bits.p, cnt.p);
     } else {
         PLB_HIP(hipMemsetAsync(bits, 0, sizeof(uint64_t) * nw, s));
         hipLaunchKernelGGL(k_brick_bits, dim3(nblk(N, 256)), dim3(256), 0, s, xyz_ref, N, b,

@@ -190,3 +190,19 @@ def test_release_memory():
     P.release_memory()
     assert free() >= before - 4 * MB
     assert np.array_equal(use(), want)
+
+
+def test_bricks_past_the_mask_make_more_than_2_32_voxels():
+    """1620^3 voxels are less than 2^32, rows of 64 rounded up (1664) make more."""
+    edge = 1620
+    flag = np.zeros((edge, edge, edge), np.uint8)
+    rng = np.random.default_rng(8)
+    for z, y, x in [(0, 0, 0), (edge - 20, edge - 20, edge - 40), (800, 1590, 700), (edge - 20, 0, 0)]:
+        flag[z:z + 20, y:y + 20, x:x + 40] = rng.random((20, 20, 40)) < 0.8
+    out = []
+    for kw in (dict(ordering=P.ORDER_REFERENCE), dict(ordering=P.ORDER_PENCIL, brick=(edge, 64, 1))):
+        with P.Lattice.from_flag(flag, 1, tau=0.8, gx=1e-5, precision=P.FP64, bb_mode=P.BB_HALFWAY, **kw) as lat:
+            table = lat.read_table()
+            lat.step(0, 9)
+            out.append((table, lat.read_state()))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
