@@ -392,14 +392,16 @@ def batch_samples(P, n_samples=64, seed=100):
 def study_batch(P, n_samples, max_steps, check, tol, seed=100, waves=0, tune_steps=20):
     """Config 5: n samples, edge L ~ U{64..192}, porosity ~ U[0.15, 0.45], half
     sphere packs (r U[6,12]) and half smoothed noise (sigma 2), FP32 storage,
-    half-way bounce-back, tau 1.0, g_x 1e-6.  One batched launch per step over
-    all active samples (per-sample convergence stop) vs the same samples run
-    one after another (one sample per launch, same kernels and convergence
-    rule); at most `waves` step-kernel waves per SIMD in both (TILE8, pencils
-    of 32 rows, 256 threads).  Then the same per-step batch in the shape
-    plb_batch_autotune picks for the whole batch, the persistent launch in the
-    shape tuned for it, and the per-step batch as one batch per size class
-    (L <= 128, L > 128), each in the shape tuned on that class."""
+    half-way bounce-back, tau 1.0, g_x 1e-6.  plb_batch_run and
+    plb_batch_run_persistent over all samples (per-sample convergence stop) vs
+    the same samples run one after another (batches of one); at most `waves`
+    step-kernel waves per SIMD (TILE8, pencils of 32 rows, 256 threads).  Then
+    both drivers in the shapes plb_batch_autotune picks for them, and
+    plb_batch_run on one batch per size class (L <= 128, L > 128), each in the
+    shape tuned on that class.  With checks 16 steps apart or more the samples
+    that fit the CUs' LDS run on chip with either driver; the shapes are those
+    of the others' launches per step, and plb_batch_run_persistent runs the
+    persistent kernel only where no sample fits."""
     flags = batch_samples(P, n_samples, seed)
     taus, gxs = [1.0] * n_samples, [1e-6] * n_samples
     kw = dict(precision=1, bb_mode=1, index_kind=1, layout=1, ordering=2, brick=(192, 32, 1), block_size=256,
@@ -420,8 +422,8 @@ def study_batch(P, n_samples, max_steps, check, tol, seed=100, waves=0, tune_ste
     for persistent in (False, True):
         m = run_batch(everyone, P.default_config(**kw), persistent)
         nodes = m.pop("nodes")
-        modes["persistent" if persistent else "per_step"] = m
-        log(f"batch {'persistent' if persistent else 'per-step'}: {m['ms']:.1f} ms, "
+        modes["run_persistent" if persistent else "run"] = m
+        log(f"batch {'plb_batch_run_persistent' if persistent else 'plb_batch_run'}: {m['ms']:.1f} ms, "
             f"{m['upd'] / (m['ms'] * 1e-3) / 1e6:.0f} MLUPS")
 
     def shape(cfg):
@@ -441,7 +443,7 @@ def study_batch(P, n_samples, max_steps, check, tol, seed=100, waves=0, tune_ste
     ptune_s = time.perf_counter() - t0
     ptuned = run_batch(everyone, ptuned_cfg, persistent=True)
     ptuned.pop("nodes")
-    log(f"batch persistent tuned {shape(ptuned_cfg)}: {ptuned['ms']:.1f} ms ({ptune_s:.1f} s of tuning)")
+    log(f"batch plb_batch_run_persistent tuned {shape(ptuned_cfg)}: {ptuned['ms']:.1f} ms ({ptune_s:.1f} s of tuning)")
     classes = {"L<=128": [k for k in everyone if max(flags[k].shape) <= 128],
                "L>128": [k for k in everyone if max(flags[k].shape) > 128]}
     per_class = {"updates": 0, "ms": 0.0, "classes": {}}
@@ -472,17 +474,18 @@ def study_batch(P, n_samples, max_steps, check, tol, seed=100, waves=0, tune_ste
     def rate(u, m):
         return {"updates": int(u), "ms": round(m, 1), "mlups": round(u / (m * 1e-3) / 1e6, 1)}
 
-    pst, per = modes["persistent"], modes["per_step"]
+    pst, per = modes["run_persistent"], modes["run"]
     out = {"study": "batch", "samples": n_samples, "pore_nodes_total": int(sum(nodes)), "waves_per_simd": waves,
            "tol": tol, "check_every": check, "max_steps": max_steps,
-           "per_step": rate(per["upd"], per["ms"]), "persistent": rate(pst["upd"], pst["ms"]),
+           "run": rate(per["upd"], per["ms"]), "run_persistent": rate(pst["upd"], pst["ms"]),
+           "on_chip": "samples that fit the CUs' LDS, with either driver, where check_every >= 16",
            "sequential": rate(seq_upd, seq_ms),
            "steps_min": int(min(per["steps"])), "steps_max": int(max(per["steps"])),
            "same_steps_all_three": per["steps"] == pst["steps"] == seq_steps,
-           "same_K_persistent_per_step": per["K"] == pst["K"],
+           "same_K_both_drivers": per["K"] == pst["K"],
            "K_range": [float(min(per["K"])), float(max(per["K"]))]}
-    out["speedup_per_step_vs_sequential"] = round(out["per_step"]["mlups"] / out["sequential"]["mlups"], 3)
-    out["speedup_persistent_vs_sequential"] = round(out["persistent"]["mlups"] / out["sequential"]["mlups"], 3)
+    out["speedup_run_vs_sequential"] = round(out["run"]["mlups"] / out["sequential"]["mlups"], 3)
+    out["speedup_run_persistent_vs_sequential"] = round(out["run_persistent"]["mlups"] / out["sequential"]["mlups"], 3)
     # Node values are shape-independent; the FP64 sums behind K and the stop
     # test follow the node order, so K may differ in its last bits.
     def kdiff(K):
@@ -490,9 +493,9 @@ def study_batch(P, n_samples, max_steps, check, tol, seed=100, waves=0, tune_ste
 
     out["tuned"] = dict(rate(tuned["upd"], tuned["ms"]), shape=shape(tuned_cfg), tuning_s=round(tune_s, 1),
                         same_steps=tuned["steps"] == per["steps"], K_max_rel_diff=kdiff(tuned["K"]))
-    out["persistent_tuned"] = dict(rate(ptuned["upd"], ptuned["ms"]), shape=shape(ptuned_cfg),
-                                   tuning_s=round(ptune_s, 1), same_steps=ptuned["steps"] == per["steps"],
-                                   K_max_rel_diff=kdiff(ptuned["K"]))
+    out["run_persistent_tuned"] = dict(rate(ptuned["upd"], ptuned["ms"]), shape=shape(ptuned_cfg),
+                                       tuning_s=round(ptune_s, 1), same_steps=ptuned["steps"] == per["steps"],
+                                       K_max_rel_diff=kdiff(ptuned["K"]))
     out["tuned_per_class"] = dict(rate(per_class["updates"], per_class["ms"]), classes=per_class["classes"],
                                   same_steps=class_steps == per["steps"], K_max_rel_diff=kdiff(class_K))
     print(json.dumps(out), flush=True)
@@ -502,7 +505,9 @@ def study_batch_steps(P, steps, waves=4, seed=100):
     """The 64-sample batch for a fixed number of steps (tol 0: no sample
     stops), once per step and as one persistent launch, in one shape (FP32,
     TILE8, AoSoA, pencils of 32 rows, 256 threads, at most `waves` waves per
-    SIMD): a short run for counter passes that compare the two drivers."""
+    SIMD): a short run for counter passes that compare the two drivers.  At
+    most 127 steps: from 128 on both run on chip."""
+    steps = min(steps, 127)
     flags = batch_samples(P, 64, seed)
     cfg = P.default_config(precision=1, bb_mode=1, index_kind=1, layout=1, ordering=2, brick=(192, 32, 1),
                            block_size=256, waves_per_simd=waves)
@@ -630,7 +635,7 @@ def main():
         study_aa(P)
         return
     if args.study == "batch-steps":
-        study_batch_steps(P, args.max_steps if args.max_steps != 100000 else 200)
+        study_batch_steps(P, args.max_steps if args.max_steps != 100000 else 120)
         return
     if args.study == "placement":
         study_placement(P, args.reserve_gib)

@@ -320,7 +320,9 @@ typedef struct {
 typedef struct plb_batch plb_batch;
 int plb_batch_create(plb_batch **out, const plb_config *cfg, const plb_sample *samples,
                      int n_samples);
-/* Runs until every sample has converged (|d<u_x>| <= tol * max(|<u_x>|,
+/* Samples that fit the CUs' LDS run on chip where checks are 16 steps apart or
+ * more and the run has 128 or more; the others take one launch per step.
+ * Runs until every sample has converged (|d<u_x>| <= tol * max(|<u_x>|,
  * 1e-3 |g_x|) between checks check_every steps apart; the floor stops samples
  * without a percolating path) or max_steps.  steps_done[s] = steps the
  * sample ran; updates[0] = total node updates performed; ms = device time. */

@@ -39,6 +39,10 @@ typedef struct {
  * is not NULL, a result stored there for the same mask (64-bit hash of the
  * voxels and dimensions), precision and bounce-back mode is returned without
  * timing, and new results are appended (one text line per result).
+ * What is timed is one launch per step, on lattices of every size: where
+ * plb_step runs on chip (calls of 16 steps or more of up to 262 144 nodes in
+ * FP64, 524 288 in FP32 and FP16) the shape is not used, and such lattices
+ * need no search unless they are stepped in shorter calls.
  * results (may be NULL) receives up to max_results timed candidates. */
 int plb_autotune(const plb_config *base, const uint8_t *flag, int nx, int ny, int nz, int num_p,
                  int steps, const char *cache_path, plb_config *best, plb_tune_result *results,
@@ -54,7 +58,9 @@ int plb_autotune(const plb_config *base, const uint8_t *flag, int nx, int ny, in
  * the winner.  Stage 3: waves per SIMD (no cap, 6, 5, 4), timed on one
  * batch.  Every candidate gives the same per-sample results.  Samples of one
  * size class make a representative input: a batch's best shape follows its
- * sample sizes.  results (may be NULL) receives up to max_results timed
+ * sample sizes.  The candidates are timed without on-chip runs, so the result
+ * is for the samples, check intervals and run lengths that do not go on chip
+ * (plb_batch_run_persistent, plb.h).  results (may be NULL) receives up to max_results timed
  * candidates. */
 int plb_batch_autotune(const plb_config *base, const plb_sample *samples, int n_samples, int steps,
                        int persistent, plb_config *best, plb_tune_result *results, int max_results,

@@ -380,7 +380,8 @@ def copy_bandwidth(nbytes=8 << 30, iters=5, device=0):
 def autotune(flag, num_p=1, steps=20, cache_path=None, cfg=None, **kw):
     """Fastest (index encoding, layout, node order, block size, nodes per
     thread, waves per SIMD) for this mask, by plb_autotune's two-stage search;
-    returns (Config, results)."""
+    returns (Config, results).  It times launches per step; calls of 16 steps
+    or more of a lattice that fits the CUs' LDS do not use the shape."""
     cfg = cfg or default_config(**kw)
     flag = np.ascontiguousarray(flag, dtype=np.uint8)
     nz, ny, nx = flag.shape
@@ -415,8 +416,9 @@ def _sample_array(flags, taus, gxs):
 def batch_autotune(flags, taus, gxs, steps=20, cfg=None, persistent=False, **kw):
     """Fastest (index encoding, layout, node order, block size, waves per
     SIMD) for a batch of these samples, by plb_batch_autotune's three-stage
-    search, timed with the per-step driver or (persistent=True) the
-    persistent launch; returns (Config, results)."""
+    search, timed with one launch per step or (persistent=True) the
+    persistent launch; returns (Config, results).  The samples of a run that
+    go on chip do not use the shape."""
     cfg = cfg or default_config(**kw)
     keep, arr = _sample_array(flags, taus, gxs)
     best = Config()
@@ -442,8 +444,10 @@ class Batch:
         self.nodes = [int(_lib().plb_batch_num_nodes(h, s)) for s in range(self.n)]
 
     def run(self, max_steps, check_every, tol, persistent=False):
-        """(steps per sample, node updates, device ms); persistent=True runs
-        plb_batch_run_persistent (one launch) instead of one launch per step."""
+        """(steps per sample, node updates, device ms).  Samples that fit the
+        CUs' LDS run on chip from 128 steps on, if checks are 16 or more apart;
+        the others take one launch per step or, with persistent=True
+        (plb_batch_run_persistent) where no sample runs on chip, one launch in all."""
         steps = np.zeros(self.n, dtype=np.int64)
         upd = C.c_int64(0)
         ms = C.c_double(0.0)
