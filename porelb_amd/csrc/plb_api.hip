@@ -394,9 +394,11 @@ extern "C" int plb_step_async(plb_ctx* c, int64_t it0, int64_t nsteps)
         (void)hipThreadExchangeStreamCaptureMode(&mode);
         if (rc) return rc;
     }
+    const bool chip = !c->fault_held && onchip_ready(c, nsteps);
+    if (c->timed) PLB_HIP(hipEventRecord(c->ev0, c->stream));  // behind the plan
     if (c->fault_held) return PLB_OK;  // the state stays that of a fault until plb_sync has reported it
     Segment seg{it0, nsteps, c->cur, 0, c->macros};
-    if (onchip_ready(c, nsteps)) {
+    if (chip) {
         int rc = launch_onchip(c, it0, nsteps, &seg.serial);
         if (rc) return rc;
         if (seg.serial) {
@@ -447,7 +449,6 @@ extern "C" int plb_step_timed(plb_ctx* c, int64_t it0, int64_t nsteps, double* m
     if (!c || !ms) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
     // Steps that are repeated, since an on-chip run of them did not complete, are timed where they are repeated.
-    PLB_HIP(hipEventRecord(c->ev0, c->stream));
     c->timed = true;
     int rc = plb_step_async(c, it0, nsteps);
     hipError_t e = rc ? hipSuccess : hipEventRecord(c->ev1, c->stream);
