@@ -144,7 +144,7 @@ int plb::ctx_begin(plb_ctx* c, const plb_config* cfg, int nx, int ny, int nz, in
     if (rc) return rc;
     PLB_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     if (cfg->placement_reserve_gib > 0)  // before every buffer of the context
-        PLB_HIP(hipMalloc(&c->reserve, (size_t)cfg->placement_reserve_gib << 30));
+        PLB_HIP(dev_malloc(&c->reserve, (size_t)cfg->placement_reserve_gib << 30));
     PLB_HIP(hipEventCreate(&c->ev0));
     PLB_HIP(hipEventCreate(&c->ev1));
     return PLB_OK;

@@ -110,7 +110,7 @@ static int batch_build(plb_batch* b, const plb_config* cfg, const plb_sample* sm
             int32_t* t2 = nullptr;
             rc = compute_order(scfg, smp[s].nx, smp[s].ny, smp[s].nz, ns, xyzs[s], c->stream, &invs[s],
                                nullptr, nullptr, nullptr, nullptr, nullptr);
-            if (!rc && hipMalloc(&t2, sizeof(int32_t) * (Q - 1) * ns) != hipSuccess) rc = PLB_ERR_NOMEM;
+            if (!rc && dev_malloc(&t2, sizeof(int32_t) * (Q - 1) * ns) != hipSuccess) rc = PLB_ERR_NOMEM;
             if (!rc) rc = permute_ref_table(tabs[s], ns, invs[s], t2, c->stream);
             if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = PLB_ERR_HIP;
             if (!rc) {
@@ -214,17 +214,17 @@ extern "C" int plb_batch_create(plb_batch** out, const plb_config* cfg, const pl
             b->tau.push_back(samples[s].tau);
             b->gx.push_back(samples[s].gx);
         }
-        hipError_t e = hipMalloc(&b->d_block_sample, sizeof(int32_t) * nblocks);
-        if (e == hipSuccess) e = hipMalloc(&b->d_active, sizeof(int32_t) * nblocks);
-        if (e == hipSuccess) e = hipMalloc(&b->d_stepped, sizeof(int32_t) * nblocks);
-        if (e == hipSuccess) e = hipMalloc(&b->d_chip, sizeof(int32_t) * (b->c->Npad / ONCHIP_MIN_SLOTS + n_samples));
-        if (e == hipSuccess) e = hipMalloc(&b->d_end, sizeof(int64_t) * n_samples);
-        if (e == hipSuccess) e = hipMalloc(&b->d_off, sizeof(int64_t) * n_samples);
-        if (e == hipSuccess) e = hipMalloc(&b->d_n, sizeof(int64_t) * n_samples);
-        if (e == hipSuccess) e = hipMalloc(&b->d_omega, sizeof(double) * n_samples);
-        if (e == hipSuccess) e = hipMalloc(&b->d_gx, sizeof(double) * n_samples);
-        if (e == hipSuccess) e = hipMalloc(&b->d_sums, sizeof(double) * n_samples);
-        if (e == hipSuccess) e = hipMalloc(&b->d_partial, sizeof(double) * nblocks);
+        hipError_t e = dev_malloc(&b->d_block_sample, sizeof(int32_t) * nblocks);
+        if (e == hipSuccess) e = dev_malloc(&b->d_active, sizeof(int32_t) * nblocks);
+        if (e == hipSuccess) e = dev_malloc(&b->d_stepped, sizeof(int32_t) * nblocks);
+        if (e == hipSuccess) e = dev_malloc(&b->d_chip, sizeof(int32_t) * (b->c->Npad / ONCHIP_MIN_SLOTS + n_samples));
+        if (e == hipSuccess) e = dev_malloc(&b->d_end, sizeof(int64_t) * n_samples);
+        if (e == hipSuccess) e = dev_malloc(&b->d_off, sizeof(int64_t) * n_samples);
+        if (e == hipSuccess) e = dev_malloc(&b->d_n, sizeof(int64_t) * n_samples);
+        if (e == hipSuccess) e = dev_malloc(&b->d_omega, sizeof(double) * n_samples);
+        if (e == hipSuccess) e = dev_malloc(&b->d_gx, sizeof(double) * n_samples);
+        if (e == hipSuccess) e = dev_malloc(&b->d_sums, sizeof(double) * n_samples);
+        if (e == hipSuccess) e = dev_malloc(&b->d_partial, sizeof(double) * nblocks);
         if (e == hipSuccess) e = hipMemset(b->d_partial, 0, sizeof(double) * nblocks);
         if (e == hipSuccess)
             e = hipMemcpy(b->d_block_sample, b->block_sample.data(), sizeof(int32_t) * nblocks,

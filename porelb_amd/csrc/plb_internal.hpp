@@ -108,6 +108,13 @@ namespace plb {
 // Device memory that may come from, and go to, the kept blocks (plb_mem.hip).
 // dev_free: the work that uses the block has been waited for.
 hipError_t dev_alloc(void** p, size_t bytes);
+// Plain device memory, freed with hipFree; kept blocks make room for it.
+hipError_t dev_malloc(void** p, size_t bytes);
+template <typename T>
+hipError_t dev_malloc(T** p, size_t bytes)
+{
+    return dev_malloc((void**)p, bytes);
+}
 void dev_free(void* p);
 void dev_give_back();   // all kept blocks
 
@@ -195,7 +202,7 @@ struct DevBuf {
     {
         from = arena;
         if (arena) return arena->take(&p, n);
-        return hipMalloc((void**)&p, sizeof(T) * (size_t)(n > 0 ? n : 1));
+        return dev_malloc(&p, sizeof(T) * (size_t)(n > 0 ? n : 1));
     }
     T* release()
     {

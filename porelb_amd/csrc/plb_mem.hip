@@ -5,7 +5,7 @@
 // 265 421 nodes was 3.6 ms of a 16 ms study.  Blocks of 1 to 128 MB that are
 // released are therefore kept, up to KEEP_MOST in the process, the oldest
 // leaving first, and go to the next owner of about that size on that device.
-// They are given back when an allocation does not succeed, as soon as newer ones
+// They are given back when an allocation of the library does not succeed, as soon as newer ones
 // take their room, and by plb_release_memory.  (Not with the last context: programs
 // that make one lattice after another would lose most of the gain, 9.5 -> 12.8 ms
 // for a study of that sample, 45.1 -> 48.1 for one of 1.4 M FP64 nodes.)  Whoever releases a block has waited for the work that
@@ -52,7 +52,7 @@ void dev_give_back()
     for (const Block& b : gone) (void)hipFree(b.p);
 }
 
-static hipError_t allocate(void** p, size_t bytes)
+hipError_t dev_malloc(void** p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipErrorOutOfMemory) return e;
@@ -63,7 +63,7 @@ static hipError_t allocate(void** p, size_t bytes)
 
 hipError_t dev_alloc(void** p, size_t bytes)
 {
-    if (bytes < KEEP_FROM || bytes > KEEP_TO) return allocate(p, bytes);
+    if (bytes < KEEP_FROM || bytes > KEEP_TO) return dev_malloc(p, bytes);
     Block b = {nullptr, (bytes + MB - 1) / MB * MB, 0};
     hipError_t e = hipGetDevice(&b.device);
     if (e != hipSuccess) return e;
@@ -83,7 +83,7 @@ hipError_t dev_alloc(void** p, size_t bytes)
         }
     }
     if (!b.p) {
-        e = allocate(&b.p, b.size);
+        e = dev_malloc(&b.p, b.size);
         if (e != hipSuccess) return e;
     }
     std::lock_guard<std::mutex> lock(o.mutex);

@@ -31,8 +31,8 @@ extern "C" int plb_copy_bandwidth(int device, int64_t bytes, int iters, double* 
     PLB_HIP(hipSetDevice(device));
     const int64_t n = bytes / 16;
     u32x4 *a = nullptr, *b = nullptr;
-    PLB_HIP(hipMalloc(&a, n * 16));
-    PLB_HIP(hipMalloc(&b, n * 16));
+    PLB_HIP(dev_malloc(&a, n * 16));
+    PLB_HIP(dev_malloc(&b, n * 16));
     PLB_HIP(hipMemset(a, 1, n * 16));
     hipEvent_t e0, e1;
     PLB_HIP(hipEventCreate(&e0));

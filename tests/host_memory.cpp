@@ -121,6 +121,26 @@ static void release()
     CHECK(on_device == 0);
 }
 
+// Kept blocks make room for every allocation of the library, also those that are not blocks of that kind.
+static void room()
+{
+    void* p = nullptr;
+    CHECK(dev_alloc(&p, 80 * MB) == hipSuccess);
+    dev_free(p);
+    CHECK(on_device == 80 * MB);
+    capacity = 100 * MB;
+    {
+        DevBuf<char> b;
+        CHECK(b.alloc(60 * MB) == hipSuccess && on_device == 60 * MB);
+    }
+    CHECK(dev_alloc(&p, 80 * MB) == hipSuccess);
+    dev_free(p);
+    Arena a;
+    CHECK(a.take(&p, (size_t)1000) == hipSuccess && on_device < 81 * MB);
+    DevBuf<char> b;
+    CHECK(b.alloc(99 * MB) == hipSuccess && on_device < 100 * MB);
+}
+
 // An object of the caller's with static storage may go after the library's own static objects.
 struct Late {
     std::vector<void*> blocks;
@@ -154,6 +174,7 @@ int main(int argc, char** argv)
     const char* what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "device")) device();
     else if (!strcmp(what, "release")) release();
+    else if (!strcmp(what, "room")) room();
     else if (!strcmp(what, "at_exit")) at_exit();
     else return 2;
     return fails ? 1 : 0;

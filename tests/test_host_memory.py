@@ -26,7 +26,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["device", "at_exit", "release"])
+@pytest.mark.parametrize("check", ["device", "at_exit", "release", "room"])
 def test_host_memory(exe, check):
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1:verify_asan_link_order=0")
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=120, env=env)
