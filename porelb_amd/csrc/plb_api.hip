@@ -501,13 +501,13 @@ extern "C" int plb_read_macros(plb_ctx* c, double* rho, double* ux, double* uy, 
 int plb::read_macros_range(plb_ctx* c, int64_t first, int64_t n, double* rho, double* ux, double* uy, double* uz)
 {
     double* const outs[4] = {rho, ux, uy, uz};
-    std::vector<char*> arrays;
+    Arrays arrays;
     MacroList list;
     for (int k = 0; k < 4; k++)
         if (outs[k]) {
             list.out[list.n] = outs[k];
             list.comp[list.n++] = k;
-            arrays.push_back((char*)outs[k]);
+            arrays.add(outs[k]);
         }
     // Page-locked arrays take the kernel's own stores: a row of 64 values of one
     // component is 512 bytes on the bus, 54 GB/s from the first call on.
@@ -530,7 +530,7 @@ extern "C" int plb_read_populations(plb_ctx* c, double* f_aos)
     if (!c || (!f_aos && c->N)) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
     if (const int rcs = settle_for_read(c)) return rcs;
-    return download(c->device, c->stream, c->N, sizeof(double) * Q, {(char*)f_aos},
+    return download(c->device, c->stream, c->N, sizeof(double) * Q, f_aos,
                     [&](int64_t b, int64_t m, void* d) { return launch_read_pop(c, b, m, (double*)d); });
 }
 
@@ -562,7 +562,7 @@ extern "C" int plb_read_state(plb_ctx* c, void* buf)
     if (!c || (!buf && c->N)) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
     if (const int rcs = settle_for_read(c)) return rcs;
-    return download(c->device, c->stream, c->N, Q * c->elem, {(char*)buf},
+    return download(c->device, c->stream, c->N, Q * c->elem, buf,
                     [&](int64_t b, int64_t m, void* d) { return launch_copy_state(c, b, m, d, false); });
 }
 
@@ -580,8 +580,8 @@ extern "C" int plb_read_table(plb_ctx* c, int32_t* tab)
 {
     if (!c || (!tab && c->N)) return PLB_ERR_INVALID;
     PLB_HIP(hipSetDevice(c->device));
-    std::vector<char*> rows;
-    for (int j = 0; j < Q - 1; j++) rows.push_back((char*)(tab + (int64_t)j * c->N));
+    Arrays rows;
+    for (int j = 0; j < Q - 1; j++) rows.add(tab + (int64_t)j * c->N);
     return download(c->device, c->stream, c->N, sizeof(int32_t), rows,
                     [&](int64_t b, int64_t m, void* d) { return launch_read_table(c, b, m, (int32_t*)d); });
 }

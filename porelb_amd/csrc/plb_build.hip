@@ -1134,7 +1134,7 @@ static int preprocess_on(int device, hipStream_t s, const uint8_t* flag, int nx,
     if (V_sub_start_out)
         PLB_HIP(hipMemcpyAsync(V_sub_start_out, dstart, sizeof(int32_t) * num_p, hipMemcpyDeviceToHost, s));
     if (V_out && fi.N) {
-        rc = download(device, s, fi.N, sizeof(plb_node_info), {(char*)V_out}, [&](int64_t first, int64_t m, void* d) {
+        rc = download(device, s, fi.N, sizeof(plb_node_info), V_out, [&](int64_t first, int64_t m, void* d) {
             GridArgs ac = a;
             ac.xyz = fi.xyz.p + first;
             ac.N = m;

@@ -118,6 +118,17 @@ hipError_t dev_malloc(T** p, size_t bytes)
 void dev_free(void* p);
 void dev_give_back();   // all kept blocks
 
+// Host memory that runs out does not leave a C entry as an exception.
+template <typename F>
+int guarded(F f)
+{
+    try {
+        return f();
+    } catch (...) {
+        return PLB_ERR_NOMEM;
+    }
+}
+
 // Device memory with one owner.  reserve() takes one block that take() cuts
 // pieces from; what does not fit, or comes without a reserve, gets an
 // allocation of its own, and give() frees only that.  An allocation costs 25 to
@@ -140,9 +151,8 @@ public:
     hipError_t reserve(size_t bytes)
     {
         void* p = nullptr;
-        const hipError_t e = dev_alloc(&p, bytes);
+        const hipError_t e = own(&p, bytes);
         if (e != hipSuccess) return e;
-        own_.push_back(p);
         base_ = (char*)p;
         size_ = bytes;
         used_ = 0;
@@ -156,9 +166,8 @@ public:
             used_ += need;
             return hipSuccess;
         }
-        const hipError_t e = dev_alloc(p, need);
-        if (e == hipSuccess) own_.push_back(*p);
-        else *p = nullptr;
+        const hipError_t e = own(p, need);
+        if (e != hipSuccess) *p = nullptr;
         return e;
     }
     template <typename T>
@@ -178,6 +187,18 @@ public:
     }
 
 private:
+    hipError_t own(void** p, size_t bytes)
+    {
+        try {
+            own_.push_back(nullptr);
+        } catch (...) {
+            return hipErrorOutOfMemory;
+        }
+        const hipError_t e = dev_alloc(p, bytes);
+        if (e == hipSuccess) own_.back() = *p;
+        else own_.pop_back();
+        return e;
+    }
     std::vector<void*> own_;
     hipStream_t stream_ = nullptr;
     char* base_ = nullptr;

@@ -12,8 +12,8 @@
 // uses it: a block may serve another stream or thread the moment it is released.
 #include <algorithm>
 #include <mutex>
+#include <new>
 #include <unordered_map>
-#include <vector>
 
 #include "plb_internal.hpp"
 
@@ -21,36 +21,53 @@ namespace plb {
 
 constexpr size_t MB = (size_t)1 << 20;
 constexpr size_t KEEP_FROM = MB, KEEP_TO = 128 * MB, KEEP_MOST = 256 * MB;
+constexpr int BLOCKS_MOST = KEEP_MOST / KEEP_FROM + 1;   // with the one that takes the others' room
 
 struct Block {
     void* p;
     size_t size;
     int device;
 };
-// Never destroyed: owners may outlive static objects.
 struct Pool {
     std::mutex mutex;
-    std::vector<Block> kept;                   // oldest first
-    std::unordered_map<void*, Block> live;
+    Block kept[BLOCKS_MOST];                   // oldest first
+    int n = 0;
     size_t kept_bytes = 0;
+    std::unordered_map<void*, Block> live;
+
+    Block take(int k)
+    {
+        const Block b = kept[k];
+        std::move(kept + k + 1, kept + n, kept + k);
+        n--;
+        kept_bytes -= b.size;
+        return b;
+    }
 };
+// Never destroyed: owners may outlive static objects.
 static Pool& pool()
 {
-    static Pool* const p = new Pool();
+    alignas(Pool) static char place[sizeof(Pool)];
+    static Pool* const p = new (place) Pool();
     return *p;
 }
 
-void dev_give_back()
+// Frees the oldest blocks until no more than `most` bytes are kept.
+static void give_back(size_t most)
 {
     Pool& o = pool();
-    std::vector<Block> gone;
-    {
-        std::lock_guard<std::mutex> lock(o.mutex);
-        gone.swap(o.kept);
-        o.kept_bytes = 0;
+    for (;;) {
+        Block b;
+        {
+            std::lock_guard<std::mutex> lock(o.mutex);
+            if (o.kept_bytes <= most) return;
+            b = o.take(0);
+        }
+        (void)hipFree(b.p);
     }
-    for (const Block& b : gone) (void)hipFree(b.p);
 }
+
+void dev_give_back() { give_back(0); }
 
 hipError_t dev_malloc(void** p, size_t bytes)
 {
@@ -70,24 +87,24 @@ hipError_t dev_alloc(void** p, size_t bytes)
     Pool& o = pool();
     {
         std::lock_guard<std::mutex> lock(o.mutex);
-        std::vector<Block>& kept = o.kept;
-        size_t best = kept.size();
-        for (size_t k = 0; k < kept.size(); k++)
-            if (kept[k].device == b.device && kept[k].size >= b.size && kept[k].size <= b.size + b.size / 2 &&
-                (best == kept.size() || kept[k].size < kept[best].size))
+        int best = -1;
+        for (int k = 0; k < o.n; k++)
+            if (o.kept[k].device == b.device && o.kept[k].size >= b.size && o.kept[k].size <= b.size + b.size / 2 &&
+                (best < 0 || o.kept[k].size < o.kept[best].size))
                 best = k;
-        if (best < kept.size()) {
-            b = kept[best];
-            kept.erase(kept.begin() + best);
-            o.kept_bytes -= b.size;
-        }
+        if (best >= 0) b = o.take(best);
     }
     if (!b.p) {
         e = dev_malloc(&b.p, b.size);
         if (e != hipSuccess) return e;
     }
-    std::lock_guard<std::mutex> lock(o.mutex);
-    o.live[b.p] = b;
+    try {
+        std::lock_guard<std::mutex> lock(o.mutex);
+        o.live[b.p] = b;
+    } catch (const std::bad_alloc&) {
+        (void)hipFree(b.p);
+        return hipErrorOutOfMemory;
+    }
     *p = b.p;
     return hipSuccess;
 }
@@ -96,24 +113,19 @@ void dev_free(void* p)
 {
     if (!p) return;
     Pool& o = pool();
-    std::vector<Block> gone;
+    bool known;
     {
         std::lock_guard<std::mutex> lock(o.mutex);
         const auto it = o.live.find(p);
-        if (it == o.live.end()) {
-            gone.push_back({p, 0, 0});
-        } else {
-            o.kept.push_back(it->second);
+        known = it != o.live.end() && o.n < BLOCKS_MOST;
+        if (known) {
+            o.kept[o.n++] = it->second;
             o.kept_bytes += it->second.size;
-            o.live.erase(it);
-            while (o.kept_bytes > KEEP_MOST) {
-                o.kept_bytes -= o.kept.front().size;
-                gone.push_back(o.kept.front());
-                o.kept.erase(o.kept.begin());
-            }
         }
+        if (it != o.live.end()) o.live.erase(it);
     }
-    for (const Block& b : gone) (void)hipFree(b.p);
+    if (known) give_back(KEEP_MOST);
+    else (void)hipFree(p);
 }
 
 }  // namespace plb

@@ -1135,7 +1135,7 @@ bool onchip_ready(plb_ctx* c, int64_t nsteps)
         // a capture of the caller's elsewhere in this thread is none of the plan's business
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
         (void)hipThreadExchangeStreamCaptureMode(&mode);
-        const int rc = plan_single(c);
+        const int rc = guarded([&] { return plan_single(c); });
         (void)hipThreadExchangeStreamCaptureMode(&mode);
         if (rc) {  // too large, or no memory for the plan: one launch per step
             (void)hipGetLastError();
@@ -1310,7 +1310,7 @@ bool onchip_batch_ready(plb_ctx* c, const std::vector<int64_t>& off, const std::
     if (G == 0 || G > 65535) return false;
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     (void)hipThreadExchangeStreamCaptureMode(&mode);
-    const int rc = build_onchip(c, samples, G, NS);
+    const int rc = guarded([&] { return build_onchip(c, samples, G, NS); });
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (rc) {
         (void)hipGetLastError();

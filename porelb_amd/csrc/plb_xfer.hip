@@ -24,6 +24,7 @@
 #include <functional>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -48,15 +49,17 @@ struct Staging {
     bool busy = true;
 };
 
-// Never destroyed: a context may outlive static objects.
 struct Kept {
     std::mutex mutex;
-    std::vector<Staging*> pool;
+    Staging* pool[MAX_KEPT];
+    int n = 0;
     int contexts = 0;
 };
+// Never destroyed: a context may outlive static objects.
 static Kept& kept()
 {
-    static Kept* const k = new Kept();
+    alignas(Kept) static char place[sizeof(Kept)];
+    static Kept* const k = new (place) Kept();
     return *k;
 }
 
@@ -78,18 +81,17 @@ static void staging_free(Staging* s)
 static void free_idle()
 {
     Kept& o = kept();
-    std::vector<Staging*> gone;
-    {
-        std::lock_guard<std::mutex> lock(o.mutex);
-        for (size_t k = 0; k < o.pool.size();)
-            if (!o.pool[k]->busy) {
-                gone.push_back(o.pool[k]);
-                o.pool.erase(o.pool.begin() + k);
-            } else {
-                k++;
-            }
+    for (;;) {
+        Staging* gone;
+        {
+            std::lock_guard<std::mutex> lock(o.mutex);
+            Staging** const idle = std::find_if(o.pool, o.pool + o.n, [](Staging* s) { return !s->busy; });
+            if (idle == o.pool + o.n) return;
+            gone = *idle;
+            *idle = o.pool[--o.n];
+        }
+        staging_free(gone);
     }
-    for (Staging* s : gone) staging_free(s);
 }
 
 void xfer_context(int add)
@@ -110,7 +112,8 @@ static bool slots_are_kept()
 
 static hipError_t staging_new(int device, Staging** out)
 {
-    Staging* s = new Staging();
+    Staging* s = new (std::nothrow) Staging();
+    if (!s) return hipErrorOutOfMemory;
     s->device = device;
     hipError_t e = hipHostMalloc((void**)&s->host, SLOT * SLOTS, hipHostMallocCoherent);
     if (e == hipSuccess) e = dev_alloc((void**)&s->dev, SLOT * SLOTS);
@@ -132,17 +135,17 @@ struct Lease {
         Kept& o = kept();
         {
             std::lock_guard<std::mutex> lock(o.mutex);
-            for (Staging* p : o.pool)
-                if (!p->busy && p->device == device) {
-                    p->busy = true;
-                    s = p;
+            for (int k = 0; k < o.n; k++)
+                if (!o.pool[k]->busy && o.pool[k]->device == device) {
+                    s = o.pool[k];
+                    s->busy = true;
                     return hipSuccess;
                 }
         }
         const hipError_t e = staging_new(device, &s);
         if (e != hipSuccess) return e;
         std::lock_guard<std::mutex> lock(o.mutex);
-        if ((int)o.pool.size() < MAX_KEPT) o.pool.push_back(s);
+        if (o.n < MAX_KEPT) o.pool[o.n++] = s;
         return hipSuccess;
     }
     ~Lease()
@@ -153,10 +156,10 @@ struct Lease {
         {
             std::lock_guard<std::mutex> lock(o.mutex);
             s->busy = false;
-            const auto it = std::find(o.pool.begin(), o.pool.end(), s);
-            if (it != o.pool.end()) {
+            Staging** const it = std::find(o.pool, o.pool + o.n, s);
+            if (it != o.pool + o.n) {
                 if (o.contexts > 0) gone = nullptr;
-                else o.pool.erase(it);
+                else *it = o.pool[--o.n];
             }
         }
         staging_free(gone);
@@ -234,15 +237,15 @@ static int threads_for(size_t bytes)
 // [part][m] in a slot and [part][n] at the caller (arrays[part]).  Kernels and
 // copies share the caller's stream: a copy stream of its own gained nothing
 // over its events (9.2 -> 12.2 ms for 382 MB of FP32 state).
-static int move(int device, hipStream_t s, int64_t n, size_t item, const std::vector<char*>& arrays, bool to_device,
+static int move(int device, hipStream_t s, int64_t n, size_t item, const Arrays& arrays, bool to_device,
                 const ChunkKernel& kernel)
 {
-    const size_t row = item * arrays.size(), bytes = row * (size_t)n;
+    const size_t row = item * arrays.n, bytes = row * (size_t)n;
     if (bytes == 0) return PLB_OK;
     // Threads move host memory, if any of it is pageable; device and managed memory is left to the runtime's copies.
     bool host = true, locked = true;
-    for (const char* a : arrays) {
-        const hipMemoryType type = attributes(a).type;
+    for (size_t p = 0; p < arrays.n; p++) {
+        const hipMemoryType type = attributes(arrays.at[p]).type;
         locked = locked && type == hipMemoryTypeHost;
         host = host && (type == hipMemoryTypeHost || type == hipMemoryTypeUnregistered);
     }
@@ -260,8 +263,8 @@ static int move(int device, hipStream_t s, int64_t n, size_t item, const std::ve
     // the kernel and the copies of m nodes from `first` on, in stream order
     auto transfer = [&](int64_t first, int64_t m, char* dev) {
         if (!to_device && (rc = kernel(first, m, dev))) return false;
-        for (size_t p = 0; p < arrays.size(); p++) {
-            char* const mine = arrays[p] + (size_t)first * item;
+        for (size_t p = 0; p < arrays.n; p++) {
+            char* const mine = arrays.at[p] + (size_t)first * item;
             char* const part = dev + (size_t)m * p * item;
             if (!check(to_device ? hipMemcpyAsync(part, mine, m * item, hipMemcpyHostToDevice, s)
                                  : hipMemcpyAsync(mine, part, m * item, hipMemcpyDeviceToHost, s)))
@@ -278,8 +281,8 @@ static int move(int device, hipStream_t s, int64_t n, size_t item, const std::ve
         team.reset(new Team(threads_for(bytes), chunks, [&](int64_t k, int t, int T) {
             const int64_t first = k * per, m = std::min(per, n - first);
             const int64_t a = m * t / T, b = m * (t + 1) / T;
-            for (size_t p = 0; p < arrays.size(); p++) {
-                char* const mine = arrays[p] + (size_t)(first + a) * item;
+            for (size_t p = 0; p < arrays.n; p++) {
+                char* const mine = arrays.at[p] + (size_t)(first + a) * item;
                 char* const staged = lease.s->host + SLOT * (k % SLOTS) + ((size_t)m * p + a) * item;
                 if (to_device) memcpy(staged, mine, (size_t)(b - a) * item);
                 else memcpy(mine, staged, (size_t)(b - a) * item);
@@ -349,23 +352,14 @@ extern "C" void plb_release_memory(void)
     dev_give_back();
 }
 
-int download(int device, hipStream_t s, int64_t n, size_t item, const std::vector<char*>& arrays,
-             const ChunkKernel& kernel)
+int download(int device, hipStream_t s, int64_t n, size_t item, const Arrays& arrays, const ChunkKernel& kernel)
 {
-    try {
-        return move(device, s, n, item, arrays, false, kernel);
-    } catch (...) {
-        return PLB_ERR_NOMEM;
-    }
+    return guarded([&] { return move(device, s, n, item, arrays, false, kernel); });
 }
 
 int upload(int device, hipStream_t s, int64_t n, size_t item, const void* array, const ChunkKernel& kernel)
 {
-    try {
-        return move(device, s, n, item, {(char*)array}, true, kernel);
-    } catch (...) {
-        return PLB_ERR_NOMEM;
-    }
+    return guarded([&] { return move(device, s, n, item, Arrays((void*)array), true, kernel); });
 }
 
 }  // namespace plb

@@ -62,7 +62,7 @@ static void transfer(int device)
 {
     std::vector<char> array(8 * MB);
     hipSetDevice(device);
-    CHECK(download(device, nullptr, (int64_t)array.size(), 1, {array.data()}, [](int64_t, int64_t m, void* d) {
+    CHECK(download(device, nullptr, (int64_t)array.size(), 1, Arrays(array.data()), [](int64_t, int64_t m, void* d) {
               memset(d, 7, m);
               return PLB_OK;
           }) == PLB_OK);
